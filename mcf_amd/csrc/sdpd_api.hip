@@ -227,8 +227,14 @@ int derive_params(const sdpd_params& p, DevParams& P, const char*& err) {
                             : 105.0 / (16.0 * kPi * P.h * P.h * P.h);
   }
   P.coef_grad = -P.coef / P.h;
-  P.inv_h = 1.0 / P.h;
   P.w0 = p.kernel_type == 1 ? P.coef * (243.0 + -192.0 + 15.0) : P.coef;
+  const double h4 = P.h * P.h * P.h * P.h;
+  P.h1 = P.h;
+  P.h2 = 2.0 * P.h;
+  P.h3 = 3.0 * P.h;
+  P.cw = p.kernel_type == 1 ? P.coef / (h4 * P.h) : P.coef / h4;
+  P.cg = p.kernel_type == 1 ? 5.0 * P.coef_grad / h4 : 12.0 * P.coef_grad / (h4 / P.h);
+  P.w0q = p.kernel_type == 1 ? 66.0 * (h4 * P.h) : h4;
   P.c2 = p.c * p.c;
   P.rho0 = p.rho;
   P.rho_ref = p.rho_ref;
@@ -243,6 +249,7 @@ int derive_params(const sdpd_params& p, DevParams& P, const char*& err) {
   P.sqrt_dt = std::sqrt(p.dt);
   P.inv_sqrt_dt = 1.0 / P.sqrt_dt;
   P.sqrt_2kt_eta = std::sqrt(2.0 * P.kt * P.eta);
+  P.knoise = 2.0 * P.kt / (P.dt * -P.cg);
   P.tau = p.tau;
   P.G = p.n_p * p.kt_p;  // particles_compute_pressure_tensor.F90:94
   for (int d = 0; d < 3; ++d) P.bf[d] = p.body_force[d];

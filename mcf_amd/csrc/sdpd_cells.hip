@@ -262,6 +262,8 @@ __global__ void k_copy_back(DevParams P, DeviceState S, const int32_t* __restric
     if (S.x_ref) S.x_ref[(int64_t)d * n + i] = xv;
     S.v[(int64_t)d * n + i] = S.v_alt[(int64_t)d * n + i];
   }
+  if (!P.mixed)
+    reinterpret_cast<double2*>(S.rec64)[i] = make_double2(S.x_alt[i], S.x_alt[(int64_t)n + i]);
   S.m[i] = S.m_alt[i];
   S.pid[i] = S.pid_alt[i];
   S.perm[i] = S.perm_alt[i];

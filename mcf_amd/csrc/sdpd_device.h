@@ -33,7 +33,11 @@ struct DevParams {
   double rd_ref[3];       // nm_ref / length (PPM's rdx)
   double cs[3];           // cell edge length / nm
   double cut_off, cut2;
-  double h, inv_h, coef, coef_grad, w0;
+  double h, coef, coef_grad, w0;
+  // FP64 pair bodies: multiples of h, the factors left out of kernel_w and
+  // kernel_g, the self term without its factor, and the thermal amplitude
+  // 2 kT / (dt |cg|) of kernel_g's unit
+  double h1, h2, h3, cw, cg, w0q, knoise;
   double c2, rho_ref, gamma, p0;
   double eta, eta_coef, kt, dt, sqrt_dt, inv_sqrt_dt, sqrt_2kt_eta;
   double tau, G;
@@ -198,26 +202,36 @@ __device__ __forceinline__ int32_t cell_key_geo(const RepGeom& g, int dim, doubl
 // smoothing kernel (kernel_kernel_quintic_spline.F90:160-215,
 // kernel_kernel_Lucy.F90), same operation order as the reference
 // ---------------------------------------------------------------------
-// W and dW/dr at s = r/h without branches: with t_k = max(k - s, 0) the
-// piecewise quintic spline is coef (t3^5 - 6 t2^5 + 15 t1^5) and its
-// derivative coef_grad (5 t3^4 - 30 t2^4 + 75 t1^4), coef_grad = -coef/h
-// (kernel_kernel_quintic_spline.F90:1-221); Lucy: coef (1 + 3s) t1^3 and
-// coef_grad 12 s t1^2 (kernel_kernel_Lucy.F90:1-174).  Zero from s = 3
-// (quintic) or s = 1 (Lucy) on.
-__device__ __forceinline__ void kernel_eval(const DevParams& P, double s, double& w,
-                                            double& gw) {
+// W and dW/dr without branches: with t_k = max(k h - r, 0) the piecewise
+// quintic spline is cw (t3^5 - 6 t2^5 + 15 t1^5), cw = coef / h^5, and its
+// derivative cg (t3^4 - 6 t2^4 + 15 t1^4), cg = 5 coef_grad / h^4 with
+// coef_grad = -coef / h (kernel_kernel_quintic_spline.F90:1-221); Lucy:
+// cw (h + 3 r) t1^3, cw = coef / h^4, and cg r t1^2, cg = 12 coef_grad / h^3
+// (kernel_kernel_Lucy.F90:1-174).  Zero from r = 3 h (quintic) or r = h
+// (Lucy) on.  The constant factors cw and cg are the caller's, who applies
+// them once per particle where the sum is linear in them.
+__device__ __forceinline__ double kernel_w(const DevParams& P, double r) {
+  const double t1 = fmax(P.h1 - r, 0.0);
   if (P.kernel_type == 1) {
-    const double t1 = fmax(1.0 - s, 0.0), t2 = fmax(2.0 - s, 0.0), t3 = fmax(3.0 - s, 0.0);
+    const double t2 = fmax(P.h2 - r, 0.0), t3 = fmax(P.h3 - r, 0.0);
     const double q1 = (t1 * t1) * (t1 * t1);
     const double q2 = (t2 * t2) * (t2 * t2);
     const double q3 = (t3 * t3) * (t3 * t3);
-    w = P.coef * (q3 * t3 - 6.0 * (q2 * t2) + 15.0 * (q1 * t1));
-    gw = P.coef_grad * (5.0 * q3 - 30.0 * q2 + 75.0 * q1);
-  } else {
-    const double t = fmax(1.0 - s, 0.0);
-    w = P.coef * (1.0 + 3.0 * s) * (t * t * t);
-    gw = P.coef_grad * 12.0 * s * (t * t);
+    return q3 * t3 - 6.0 * (q2 * t2) + 15.0 * (q1 * t1);
   }
+  return (P.h1 + 3.0 * r) * (t1 * t1 * t1);
+}
+// (never negative: next to r = 0 the quintic's three terms cancel to rounding)
+__device__ __forceinline__ double kernel_g(const DevParams& P, double r) {
+  const double t1 = fmax(P.h1 - r, 0.0);
+  if (P.kernel_type == 1) {
+    const double t2 = fmax(P.h2 - r, 0.0), t3 = fmax(P.h3 - r, 0.0);
+    const double q1 = (t1 * t1) * (t1 * t1);
+    const double q2 = (t2 * t2) * (t2 * t2);
+    const double q3 = (t3 * t3) * (t3 * t3);
+    return fmax(q3 - 6.0 * q2 + 15.0 * q1, 0.0);
+  }
+  return r * (t1 * t1);
 }
 
 __device__ __forceinline__ void kernel_w_gradw_f32(int kernel_type, float s, float coef,
@@ -244,6 +258,10 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   const double e = fma(-(0.5 * x) * y, y, 0.5);
   return fma(y, e, y);
 }
+
+// sqrt(x) for x >= 0 with a clamp in place of sqrt_nr's selects (x below
+// 1e-300 gives less than 1e-150, and 0 for 0).
+__device__ __forceinline__ double sqrt_pos(double x) { return x * rsqrt_nr(fmax(x, 1e-300)); }
 
 // sqrt(x) for x >= 0 through rsqrt_nr (0 for x = 0).
 __device__ __forceinline__ double sqrt_nr(double x) { return x > 0.0 ? x * rsqrt_nr(x) : 0.0; }

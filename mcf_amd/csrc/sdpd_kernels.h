@@ -28,8 +28,9 @@ struct DeviceState {
   // work map of the pair kernels (chunks of <= 64 particles of one row)
   int32_t *row_nchunk, *row_chunk_off, *chunk_row;
   int32_t *scan_tmp;     // tile sums of the exclusive scans
-  // FP64 records of the force pass: x, y, z, p/n^2, vx, vy, vz, 1/n^2;
-  // Oldroyd-B also Pi / n^2 as (xx, yy, zz, xy, xz, yz) (2D: xx, yy, 0, xy)
+  // FP64 records of the force pass, planes of n 16-byte entries: (x, y),
+  // (z, p/n^2), (vx, vy), (vz, 1/n^2); Oldroyd-B also Pi / n^2 as (xx, yy),
+  // (zz, xy), (xz, yz) (2D: zz and the last plane 0)
   double *rec64;
   double *pt64;
   float4 *vr;            // velocity, w = 1 / n^2; Oldroyd-B: w = pid bits

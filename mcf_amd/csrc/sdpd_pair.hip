@@ -32,6 +32,8 @@
 // up, and stores the lists of a chunk as one block of groups of 8 entries
 // per lane: every store fills whole 32-byte sectors and the force pass of
 // the same step (positions unchanged) reads 2 KB contiguous per group.
+#include <type_traits>
+
 #include "sdpd_kernels.h"
 
 namespace sdpd {
@@ -99,6 +101,7 @@ struct Geo {
   int cell_base, row_base;
   double L0, L1, L2;    // edge lengths
   double csd0;          // FP64 cell edge along x
+  double half2;         // squared half of the shortest edge, a rounding margin less
   float cs0, cs1, cs2;  // FP32 cell edges
 };
 
@@ -196,7 +199,7 @@ __device__ __forceinline__ double exact_d2_pos(const DevParams& P, const Home& h
 // one (returned in sg; -1 when no sheared face lies between them), with the
 // formula and roundings of exact_d2_le.
 template <int DIM>
-__device__ __forceinline__ double exact_d2_verlet(const DevParams& P, const Home& h, double xj0,
+__device__ __forceinline__ double exact_d2_image(const DevParams& P, const Home& h, double xj0,
                                                   double xj1, double xj2, double& d0,
                                                   double& d1, double& d2, int& sg) {
   sg = -1;
@@ -228,6 +231,31 @@ __device__ __forceinline__ double exact_d2_verlet(const DevParams& P, const Home
     d2 = image_diff(h.x2, xj2, h.G.L2, mg);
   }
   return DIM == 3 ? dist2_exact(d0, d1, d2) : dist2_exact2(d0, d1);
+}
+
+// The plain coordinate differences of a pair and their squared distance as
+// the reference rounds it.  When that distance is at most half the shortest
+// edge (G.half2), no coordinate differs by more than half its edge and no
+// face lies between the two: exact_d2_image would return the same bits.
+// Only the few pairs across a face then take its selects, about 36 of the
+// 172 vector instructions an FP64 force pair took with them.
+template <int DIM>
+__device__ __forceinline__ double plain_d2(const Home& h, double xj0, double xj1, double xj2,
+                                           double& d0, double& d1, double& d2) {
+  d0 = h.x0 - xj0;
+  d1 = h.x1 - xj1;
+  d2 = DIM == 3 ? h.x2 - xj2 : 0.0;
+  return DIM == 3 ? dist2_exact(d0, d1, d2) : dist2_exact2(d0, d1);
+}
+
+template <int DIM>
+__device__ __forceinline__ double exact_d2_verlet(const DevParams& P, const Home& h, double xj0,
+                                                  double xj1, double xj2, double& d0,
+                                                  double& d1, double& d2, int& sg) {
+  sg = -1;
+  double r2 = plain_d2<DIM>(h, xj0, xj1, xj2, d0, d1, d2);
+  if (!(r2 <= h.G.half2)) r2 = exact_d2_image<DIM>(P, h, xj0, xj1, xj2, d0, d1, d2, sg);
+  return r2;
 }
 
 // FP32 squared distance, rounded as the candidate scan rounds it, so the
@@ -298,6 +326,8 @@ __device__ __forceinline__ bool load_chunk(const DevParams& P, const DeviceState
   ch.G.L1 = g.L[1];
   ch.G.L2 = g.L[2];
   ch.G.csd0 = g.cs[0];
+  const double lmin = fmin(fmin(g.L[0], g.L[1]), P.dim == 3 ? g.L[2] : g.L[1]);
+  ch.G.half2 = 0.25 * lmin * lmin * (1.0 - 1e-13);
   ch.G.cs0 = g.csf[0];
   ch.G.cs1 = g.csf[1];
   ch.G.cs2 = g.csf[2];
@@ -312,7 +342,10 @@ __device__ __forceinline__ bool load_chunk(const DevParams& P, const DeviceState
 }
 
 // Neighbour list block of a chunk: list_cap / 8 groups, each 64 lanes x 8
-// entries; a lane's group g holds its entries 8g .. 8g+7.
+// entries; a lane's group g holds its entries 8g .. 8g+7.  Verlet lists
+// store them as (0, 4), (1, 5), (2, 6), (3, 7): four lanes walk a particle's
+// list, lane s takes the entries s and s + 4 of a group in one 8-byte load,
+// and a wave's 64 loads are contiguous.
 __device__ __forceinline__ uint32_t* list_block(const DevParams& P, uint32_t* list, const Chunk& ch) {
   return list + (int64_t)ch.c * P.list_cap * kWave;
 }
@@ -531,14 +564,15 @@ __device__ __forceinline__ int staged_scan(const DevParams& P, const DeviceState
     if (blk) {
       for (int q = 0; __ballot(q < w) != 0ull; q += 8) {
         if (q < w && stored + q + 8 <= P.list_cap) {
+          // (SKIN: Verlet lists, entries paired for the four-lane walk)
           uint4 lo, hi;
           lo.x = buf[(q + 0) * kWave + lane];
-          lo.y = buf[(q + 1) * kWave + lane];
-          lo.z = buf[(q + 2) * kWave + lane];
-          lo.w = buf[(q + 3) * kWave + lane];
-          hi.x = buf[(q + 4) * kWave + lane];
-          hi.y = buf[(q + 5) * kWave + lane];
-          hi.z = buf[(q + 6) * kWave + lane];
+          lo.y = buf[(q + (SKIN ? 4 : 1)) * kWave + lane];
+          lo.z = buf[(q + (SKIN ? 1 : 2)) * kWave + lane];
+          lo.w = buf[(q + (SKIN ? 5 : 3)) * kWave + lane];
+          hi.x = buf[(q + (SKIN ? 2 : 4)) * kWave + lane];
+          hi.y = buf[(q + (SKIN ? 6 : 5)) * kWave + lane];
+          hi.z = buf[(q + (SKIN ? 3 : 6)) * kWave + lane];
           hi.w = buf[(q + 7) * kWave + lane];
           uint4* dst = reinterpret_cast<uint4*>(blk + group_offset(stored + q, lane));
           dst[0] = lo;
@@ -720,16 +754,19 @@ __device__ __forceinline__ double pair_d2(const DevParams& P, const Home& h, con
   return DIM == 3 ? fma(d2, d2, fma(d1, d1, d0 * d0)) : fma(d1, d1, d0 * d0);
 }
 
+// Element j of a device array, addressed as base + 32-bit byte offset (at
+// most 2^25 elements of 16 bytes).
+template <class T>
+__device__ __forceinline__ T load_at(const T* base, uint32_t j) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
+                                     (size_t)(j * (uint32_t)sizeof(T)));
+}
+
 // DECIDE (Verlet lists): the entries are candidates within rc + skin; the
 // body takes the exact in / out decision on the current positions and
-// counts the in-cut-off neighbours (nin) and the FP64 re-decisions.
-// Verlet lists evaluate in batches of eight: the positions of the batch's
-// neighbours are gathered before the first pair is evaluated (three 8-byte
-// gathers each, whose latency a one-at-a-time walk exposes); the sums keep
-// the entries' order.  On the 128^3 box the walk takes 0.89 ms in batches
-// of four, 0.72 in eight, 0.74 in sixteen.  The per-step lists go one at a
-// time (the batch's registers cost the candidate scan occupancy every
-// step).
+// counts the in-cut-off neighbours (nin) and the FP64 re-decisions.  The
+// positions come as (x, y) from the record's first plane and z: two gathers
+// per entry.
 template <int DIM, bool DECIDE = false>
 struct DensityF64 {
   const DevParams& P;
@@ -740,48 +777,100 @@ struct DensityF64 {
   static constexpr bool kImages = true;
   static constexpr bool kBatched = DECIDE;
   static constexpr int kBatch = 8;
+  static constexpr int kTerms = 1;
+  static constexpr int kWalk = 4;
   __device__ __forceinline__ void body(uint32_t ent) {
     const int j = (int)(ent & kIndexMask);
     const int64_t n = P.n;
     double d0, d1, d2;
     const double r2 = pair_d2<DIM>(P, h, decode_images(ent), S.x[j], S.x[n + j],
                                    DIM == 3 ? S.x[2 * n + j] : 0.0, d0, d1, d2);
-    double w, gw;
-    kernel_eval(P, sqrt_nr(r2) * P.inv_h, w, gw);
+    const double w = kernel_w(P, sqrt_pos(r2));
     acc = acc + (P.density_type == 1 ? S.m[j] * w : w);
+  }
+  // what a batch gathers, and the terms of its NB entries (0 outside the
+  // cut-off and in empty slots)
+  struct Rec {
+    double2 a;
+    double z;
+  };
+  __device__ __forceinline__ Rec gather(uint32_t ent) const {
+    const uint32_t j = ent & kIndexMask;
+    return {load_at(reinterpret_cast<const double2*>(S.rec64), j),
+            DIM == 3 ? load_at(S.x + 2 * (int64_t)P.n, j) : 0.0};
+  }
+  template <int NB>
+  __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                        Rec (&r)[NB], double (&t)[NB][kTerms]) {
+    // the reference's decision (pp_interaction.inc:37-46) on the current
+    // positions; one branch of the wave for the batches with a pair across a
+    // face
+    double r2[NB];
+    uint64_t far = 0;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      double d0, d1, d2;
+      r2[k] = plain_d2<DIM>(h, r[k].a.x, r[k].a.y, r[k].z, d0, d1, d2);
+      far |= __ballot(!(r2[k] <= h.G.half2));
+    }
+    if (__builtin_expect(far != 0, 0)) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        double d0, d1, d2;
+        int sg;
+        r2[k] = exact_d2_image<DIM>(P, h, r[k].a.x, r[k].a.y, r[k].z, d0, d1, d2, sg);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const bool use = ok[k] && r2[k] < P.cut2;
+      nin += use ? 1 : 0;
+      double w = kernel_w(P, sqrt_pos(r2[k]));
+      if (P.density_type == 1) w = S.m[(int)(e[k] & kIndexMask)] * w;
+      t[k][0] = use ? w : 0.0;
+    }
   }
   template <int NB>
   __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
-    const int64_t n = P.n;
-    double x0[NB], x1[NB], x2[NB];
+    double t[NB][kTerms];
+    Rec r[NB];
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const int j = (int)(e[k] & kIndexMask);
-      x0[k] = S.x[j];
-      x1[k] = S.x[n + j];
-      x2[k] = DIM == 3 ? S.x[2 * n + j] : 0.0;
-    }
+    for (int k = 0; k < NB; ++k) r[k] = gather(e[k]);
+    terms(e, ok, r, t);
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      double d0, d1, d2, r2;
-      bool use = ok[k];
-      if (DECIDE) {
-        // the reference's decision (pp_interaction.inc:37-46) on the
-        // current positions
-        int sg;
-        r2 = exact_d2_verlet<DIM>(P, h, x0[k], x1[k], x2[k], d0, d1, d2, sg);
-        use = use && r2 < P.cut2;
-        nin += use ? 1 : 0;
-      } else {
-        r2 = pair_d2<DIM>(P, h, decode_images(e[k]), x0[k], x1[k], x2[k], d0, d1, d2);
-      }
-      // beyond the cut-off the kernel is 0: no branch on the decision
-      double w, gw;
-      kernel_eval(P, sqrt_nr(r2) * P.inv_h, w, gw);
-      if (use) acc = acc + (P.density_type == 1 ? S.m[(int)(e[k] & kIndexMask)] * w : w);
-    }
+    for (int k = 0; k < NB; ++k) acc = acc + t[k][0];
   }
 };
+
+// Plain coordinate differences taken to the nearest image (one rounding, as
+// pair_d2's; across a sheared face j's copy is moved by the shear length and
+// jump is its extra x velocity).  False for a NaN separation, which an in /
+// out decision leaves out: it goes outside the cut-off.
+template <int DIM>
+__device__ __forceinline__ bool nearest_image(const DevParams& P, const Home& h, double& d0,
+                                              double& d1, double& d2, double& jump) {
+  auto fold = [](double d, double L) {
+    return d > 0.5 * L ? d - L : (d < -0.5 * L ? d + L : d);
+  };
+  if (P.le_g >= 0) {
+    const double raw = P.le_g == 1 ? d1 : d2;
+    const double Lg = P.le_g == 1 ? h.G.L1 : h.G.L2;
+    const int sg = raw > 0.5 * Lg ? 0 : (raw < -0.5 * Lg ? 1 : -1);
+    if (sg >= 0) {
+      const double t = d0 - h.le.sp(sg);
+      d0 = t - h.G.L0 * rint(t / h.G.L0);
+      jump = sg == 0 ? P.le_u : -P.le_u;
+    }
+  }
+  d0 = fold(d0, h.G.L0);
+  d1 = fold(d1, h.G.L1);
+  if (DIM == 3) d2 = fold(d2, h.G.L2);
+  const double r2 = DIM == 3 ? dist2_exact(d0, d1, d2) : dist2_exact2(d0, d1);
+  if (r2 <= h.G.half2) return true;
+  d0 = 2.0 * P.cut_off;
+  d1 = d2 = 0.0;
+  return false;
+}
 
 // The in / out decision of a candidate from its FP32 squared distance: in
 // below the band, out above it, inside it the reference's FP64 formula.
@@ -797,34 +886,38 @@ __device__ __forceinline__ bool mixed_inside(const DevParams& P, const DeviceSta
                            e2) < P.cut2;
 }
 
+// Per-step lists sum compensated in FP32, Verlet lists in FP64.
 template <int DIM, bool DECIDE = false>
 struct DensityMixed {
   const DevParams& P;
   const DeviceState& S;
   const Home& h;
-  KahanF acc;
+  std::conditional_t<DECIDE, WideF, KahanF> acc;
   int nin = 0, rechecks = 0;
   static constexpr bool kImages = false;
   // in batches of eight (the 128^3 Tait box in mixed precision: 0.59 ms in
   // fours, 0.51 in eights, 0.55 in sixteens)
   static constexpr bool kBatched = true;
   static constexpr int kBatch = 8;
+  static constexpr int kTerms = 1;
+  static constexpr int kWalk = 4;
+  struct Rec {
+    float4 q;
+    float mj;
+  };
+  __device__ __forceinline__ Rec gather(uint32_t ent) const {
+    const int j = (int)(ent & kIndexMask);
+    return {load_xyz(S.xa + j), P.density_type == 1 ? (float)S.m[j] : 1.f};
+  }
   template <int NB>
-  __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
-    float4 q[NB];
-    float mj[NB];
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const int j = (int)(e[k] & kIndexMask);
-      q[k] = load_xyz(S.xa + j);
-      mj[k] = P.density_type == 1 ? (float)S.m[j] : 1.f;
-    }
+  __device__ __forceinline__ void terms_f(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                          Rec (&rec)[NB], float (&t)[NB]) {
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
       // the lane's own particle in a padding slot: code 62 is offset 0
       const Offsets o = decode_code(ok[k] ? e[k] >> kCodeShift : 62u);
       float d0, d1, d2;
-      rel_diff<DIM>(P, h, q[k], o, d0, d1, d2);
+      rel_diff<DIM>(P, h, rec[k].q, o, d0, d1, d2);
       const float s2 = mixed_s2(d0, d1, d2);
       bool use = ok[k];
       if (DECIDE && use) {
@@ -834,13 +927,37 @@ struct DensityMixed {
       const float r = __builtin_amdgcn_sqrtf(s2);
       float w, gw;
       kernel_w_gradw_f32(P.kernel_type, r * P.inv_hf, P.coeff, P.coef_gradf, w, gw);
-      if (use) acc.add(P.density_type == 1 ? mj[k] * w : w);
+      t[k] = use ? (P.density_type == 1 ? rec[k].mj * w : w) : 0.f;
     }
+  }
+  template <int NB>
+  __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                        Rec (&rec)[NB], double (&t)[NB][kTerms]) {
+    float f[NB];
+    terms_f(e, ok, rec, f);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) t[k][0] = (double)f[k];
+  }
+  template <int NB>
+  __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
+    float t[NB];
+    Rec rec[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) rec[k] = gather(e[k]);
+    terms_f(e, ok, rec, t);
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+      if (DECIDE || ok[k]) acc.add(t[k]);
   }
 };
 
 // Records of the force pass, written once the density is known.
-//   FP64: (x, y, z, p/n^2, vx, vy, vz, 1/n^2).
+//   FP64: four planes of n 16-byte entries, (x, y), (z, p/n^2), (vx, vy) and
+//   (vz, 1/n^2).  Neighbours in a list are near each other in memory, so the
+//   lanes of a 16-byte gather share lines: gathers alone at the 128^3 box's
+//   lists take 151 CU cycles per wave-entry this way and 221 from 64-byte
+//   records (four lanes per particle).  With Verlet lists the (x, y) plane
+//   follows the positions (boundary, sort, track) and is not written here.
 //   FP32 Newtonian: (cell-relative x, y, z, p/n^2 for Hu-Adams or p for the
 //   angular form) and (vx, vy, vz, 1/n^2); the pair body gathers these two
 //   and the particle id.
@@ -872,9 +989,11 @@ __device__ __forceinline__ void write_force_records(const DevParams& P, const De
       }
     }
   } else {
-    double4* r = reinterpret_cast<double4*>(S.rec64 + 8 * (int64_t)i);
-    r[0] = make_double4(S.x[i], S.x[n + i], DIM == 3 ? S.x[2 * n + i] : 0.0, an);
-    r[1] = make_double4(S.v[i], S.v[n + i], DIM == 3 ? S.v[2 * n + i] : 0.0, bn);
+    double2* pl = reinterpret_cast<double2*>(S.rec64);
+    if (!P.verlet) pl[i] = make_double2(S.x[i], S.x[n + i]);
+    pl[n + i] = make_double2(DIM == 3 ? S.x[2 * n + i] : 0.0, an);
+    pl[2 * n + i] = make_double2(S.v[i], S.v[n + i]);
+    pl[3 * n + i] = make_double2(DIM == 3 ? S.v[2 * n + i] : 0.0, bn);
     if (!P.newtonian) {
       // Oldroyd-B: Pi / n^2 as (xx, yy, zz, xy, xz, yz), Pi = (p + G) I - G c
       // (particles_compute_pressure_tensor.F90:114-133; c is symmetric)
@@ -882,15 +1001,15 @@ __device__ __forceinline__ void write_force_records(const DevParams& P, const De
         const double c = S.ct[(int64_t)(a + DIM * b) * n + i];
         return ((a == b ? press + P.G : 0.0) - P.G * c) * bn;
       };
-      double2* q = reinterpret_cast<double2*>(S.pt64 + 6 * (int64_t)i);
+      double2* q = reinterpret_cast<double2*>(S.pt64) + i;
       if (DIM == 3) {
         q[0] = make_double2(pib(0, 0), pib(1, 1));
-        q[1] = make_double2(pib(2, 2), pib(0, 1));
-        q[2] = make_double2(pib(0, 2), pib(1, 2));
+        q[n] = make_double2(pib(2, 2), pib(0, 1));
+        q[2 * n] = make_double2(pib(0, 2), pib(1, 2));
       } else {
         q[0] = make_double2(pib(0, 0), pib(1, 1));
-        q[1] = make_double2(0.0, pib(0, 1));
-        q[2] = make_double2(0.0, 0.0);
+        q[n] = make_double2(0.0, pib(0, 1));
+        q[2 * n] = make_double2(0.0, 0.0);
       }
     }
   }
@@ -905,11 +1024,8 @@ __device__ __forceinline__ bool list_overflow(const DevParams& P, const DeviceSt
   return __ballot(cnt > P.list_cap) != 0ull;
 }
 
-// Walk the neighbours stored in a chunk's lists (waves without list
-// overflow): the in-cut-off pairs of the step's density pass, or the Verlet
-// lists' candidates.  Policies that evaluate in batches get Pol::kBatch
-// entries at a time from every lane (slots past a lane's count carry its
-// own particle and are flagged off).
+// Walk the in-cut-off pairs stored in a chunk's lists by the step's density
+// pass (lists rebuilt every step; waves without list overflow).
 template <int DIM, class Pol>
 __device__ __forceinline__ void for_each_listed(const DevParams& P, const DeviceState& S,
                                                 const Chunk& ch, const Home& h, Pol& pol,
@@ -917,71 +1033,166 @@ __device__ __forceinline__ void for_each_listed(const DevParams& P, const Device
   const int cnt = h.active ? S.nbr_count[h.i] : 0;
   const uint32_t* __restrict__ blk = list_block(P, S.nlist, ch);
   const int lane = threadIdx.x;
-  if constexpr (Pol::kBatched) {
-    (void)buf;
-    // G groups of eight entries per iteration (the batch may span two);
-    // a group past the lane's count is not read
-    constexpr int NB = Pol::kBatch;
-    constexpr int G = (NB + 7) / 8;
-    for (int q = 0; __ballot(q < cnt) != 0ull; q += 8 * G) {
-      uint32_t ee[8 * G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        uint4 lo = make_uint4(0u, 0u, 0u, 0u), hi = lo;
-        if (q + 8 * g < cnt) {
-          const uint4* src = reinterpret_cast<const uint4*>(blk + group_offset(q + 8 * g, lane));
-          lo = src[0];
-          hi = src[1];
-        }
-        ee[8 * g + 0] = lo.x;
-        ee[8 * g + 1] = lo.y;
-        ee[8 * g + 2] = lo.z;
-        ee[8 * g + 3] = lo.w;
-        ee[8 * g + 4] = hi.x;
-        ee[8 * g + 5] = hi.y;
-        ee[8 * g + 6] = hi.z;
-        ee[8 * g + 7] = hi.w;
-      }
-#pragma unroll
-      for (int b0 = 0; b0 < 8 * G; b0 += NB) {
-        uint32_t e[NB];
-        bool ok[NB];
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          ok[k] = q + b0 + k < cnt;
-          e[k] = ok[k] ? ee[b0 + k] : (uint32_t)h.ii;
-        }
-        pol.body_batch(e, ok);
-      }
-    }
-  } else {
-    for (int q = 0; __ballot(q < cnt) != 0ull; q += 8) {
-      if (q < cnt) {
-        // eight entries per pair of 16-byte loads; entries past cnt are
-        // padding inside the row and are not evaluated.  The group goes to
-        // LDS (entry u of a lane at buf[u * 64 + lane], conflict-free), and
-        // the loop reads one entry per pair, the next one ahead of the body.
-        const uint4* src = reinterpret_cast<const uint4*>(blk + group_offset(q, lane));
-        const uint4 lo = src[0], hi = src[1];
-        buf[0 * kWave + lane] = lo.x;
-        buf[1 * kWave + lane] = lo.y;
-        buf[2 * kWave + lane] = lo.z;
-        buf[3 * kWave + lane] = lo.w;
-        buf[4 * kWave + lane] = hi.x;
-        buf[5 * kWave + lane] = hi.y;
-        buf[6 * kWave + lane] = hi.z;
-        buf[7 * kWave + lane] = hi.w;
-        const int m = min(8, cnt - q);
-        uint32_t ent = buf[lane];
+  for (int q = 0; __ballot(q < cnt) != 0ull; q += 8) {
+    if (q < cnt) {
+      // eight entries per pair of 16-byte loads; entries past cnt are
+      // padding inside the row and are not evaluated.  The group goes to
+      // LDS (entry u of a lane at buf[u * 64 + lane], conflict-free), and
+      // the loop reads one entry per pair, the next one ahead of the body.
+      const uint4* src = reinterpret_cast<const uint4*>(blk + group_offset(q, lane));
+      const uint4 lo = src[0], hi = src[1];
+      buf[0 * kWave + lane] = lo.x;
+      buf[1 * kWave + lane] = lo.y;
+      buf[2 * kWave + lane] = lo.z;
+      buf[3 * kWave + lane] = lo.w;
+      buf[4 * kWave + lane] = hi.x;
+      buf[5 * kWave + lane] = hi.y;
+      buf[6 * kWave + lane] = hi.z;
+      buf[7 * kWave + lane] = hi.w;
+      const int m = min(8, cnt - q);
+      uint32_t ent = buf[lane];
 #pragma unroll 1
-        for (int u = 0; u < m; ++u) {
-          const uint32_t cur = ent;
-          ent = buf[((u + 1) & 7) * kWave + lane];
-          pol.body(cur);
-        }
+      for (int u = 0; u < m; ++u) {
+        const uint32_t cur = ent;
+        ent = buf[((u + 1) & 7) * kWave + lane];
+        pol.body(cur);
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------
+// the walk of Verlet lists: four lanes per particle
+// ---------------------------------------------------------------------
+// A wave takes 16 consecutive particles of a chunk (a "quarter"), lane
+// 4 p + s every fourth entry of particle p.  Against one particle per lane,
+// neighbouring lanes gather neighbouring list entries (fewer lines per
+// gather), a wave runs as long as the longest of 16 lists instead of 64,
+// and a small box has four times the waves, each a quarter as long.
+//
+// The terms are still added in list order: a group's four lanes put their
+// terms into LDS, and lane s adds component s (4 + s, 8 + s) of its particle's
+// four entries one after another.  So a particle's sum does not depend on
+// where its in-cut-off pairs stand among the candidates, and equals the
+// one-particle-per-lane sums of the candidate scans bit for bit.  Four FP64
+// adds per four components and group; the matrix cores' v_mfma_f64_4x4x4
+// (an fma chain over k, the same order) takes 4 CU cycles per component, and
+// on the 128^3 box the force walk took 1.54 ms with it.
+constexpr int kQuarter = 16;
+// a component's row of 64 lanes' terms: 66 doubles, so that the 16-byte reads
+// of the four lanes' rows fall on different banks
+constexpr int kTermRow = 66;
+template <int TERMS>
+constexpr int kTermWords = (TERMS + 3) / 4 * 4 * kTermRow;
+
+// the sums of the 16 particles after the walk: component c of particle p
+__device__ __forceinline__ double& quarter_sum(double* lds, int p, int c) {
+  return lds[c * kTermRow + p];
+}
+
+// start: what the sum of component 0 starts from (lane 4 p).  Leaves the sums
+// in lds (quarter_sum).
+template <int DIM, class Pol>
+__device__ __forceinline__ void walk_quarter(const DevParams& P, const DeviceState& S,
+                                             const Chunk& ch, int quarter, const Home& h, Pol& pol,
+                                             double start, double* __restrict__ lds) {
+  constexpr int NB = Pol::kWalk;  // entries per lane and batch (even)
+  constexpr int T = Pol::kTerms, M = (T + 3) / 4;
+  const int lane = threadIdx.x;
+  const int s = lane & 3, p = lane >> 2;
+  const int cnt = h.active ? S.nbr_count[h.i] : 0;
+  const uint32_t* __restrict__ src =
+      list_block(P, S.nlist, ch) + (kQuarter * quarter + p) * 8 + 2 * s;
+  double* __restrict__ put = lds + lane;
+  const double2* __restrict__ get = reinterpret_cast<const double2*>(lds + s * kTermRow + 4 * p);
+  double sum[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) sum[m] = 0.0;
+  if (s == 0) sum[0] = start;
+  // the next batch's entries are loaded behind the current batch's gathers,
+  // without a branch (a group past the list's capacity reads its last one)
+  const int last = (P.list_cap >> 3) - 1;
+  uint2 nx[NB / 2];
+  auto fetch = [&](int q) {
+#pragma unroll
+    for (int g = 0; g < NB / 2; ++g)
+      nx[g] = *reinterpret_cast<const uint2*>(src + (int64_t)min((q >> 3) + g, last) * (8 * kWave));
+  };
+  fetch(0);
+  for (int q = 0; __ballot(q < cnt) != 0ull; q += 4 * NB) {
+    uint32_t e[NB];
+    bool ok[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      ok[k] = q + 4 * k + s < cnt;
+      e[k] = ok[k] ? ((k & 1) ? nx[k / 2].y : nx[k / 2].x) : (uint32_t)h.ii;
+    }
+    typename Pol::Rec r[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) r[k] = pol.gather(e[k]);
+    fetch(q + 4 * NB);
+    // (the density bodies are short: the scheduler would sink some of these
+    // loads to their first use, one wait each -- the FP64 walk of the 128^3
+    // box takes 0.78 instead of 0.58 ms then)
+    if constexpr (T == 1) __builtin_amdgcn_sched_barrier(0);
+    double t[NB][T];
+    pol.terms(e, ok, r, t);
+    // (one wave per workgroup: its LDS operations complete in order)
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int c = 0; c < T; ++c) put[c * kTermRow] = t[k][c];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const double2 a = get[2 * m * kTermRow], b = get[2 * m * kTermRow + 1];
+        sum[m] = sum[m] + a.x;
+        sum[m] = sum[m] + a.y;
+        sum[m] = sum[m] + b.x;
+        sum[m] = sum[m] + b.y;
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int m = 0; m < M; ++m) quarter_sum(lds, p, 4 * m + s) = sum[m];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// The home particle of a lane in the walk of a quarter.
+template <int DIM>
+__device__ __forceinline__ Home load_quarter_home(const DevParams& P, const DeviceState& S,
+                                                  const Chunk& ch, int quarter) {
+  Home h;
+  h.i = ch.p0 + kQuarter * quarter + ((int)threadIdx.x >> 2);
+  h.active = h.i < ch.p1;
+  h.ii = h.active ? h.i : ch.p0;
+  const int64_t n = P.n;
+  h.G = ch.G;
+  h.cx = (S.key_sorted[h.ii] - ch.G.cell_base) % ch.G.nm0;
+  const int lr = ch.row - ch.G.row_base;
+  h.cy = lr % ch.G.nm1;
+  h.cz = lr / ch.G.nm1;
+  h.a = S.xa[h.ii];
+  h.x0 = S.x[h.ii];
+  h.x1 = S.x[n + h.ii];
+  h.x2 = DIM == 3 ? S.x[2 * n + h.ii] : 0.0;
+  if (P.le_g >= 0) {
+    h.le.t = S.time_dev[1];
+    h.le.sp0 = f_modulo((P.le_vhi - P.le_vlo) * h.le.t, ch.G.L0);
+    h.le.sp1 = f_modulo((P.le_vlo - P.le_vhi) * h.le.t, ch.G.L0);
+  }
+  return h;
+}
+
+// Chunk slot and first quarter of a workgroup that takes NQ quarters: the
+// workgroups of a chunk are 8 apart, so they share an XCD.
+template <int NQ>
+__device__ __forceinline__ int quarter_slot(int b, int& quarter) {
+  constexpr int G = 4 / NQ;
+  quarter = (b / 8) % G * NQ;
+  return b / (8 * G) * 8 + b % 8;
 }
 
 // Whether a chunk's row of cells lies within `cells` cells of a face of
@@ -1008,49 +1219,12 @@ __device__ __forceinline__ bool chunk_meets_le_face(int le_g, const Chunk& ch, i
 // without storing, for the chunks with an overflowed list; kScanAll does
 // that for every chunk whatever the gate (the autotuner).  The walk and the
 // scans visit the candidates in the same order, so they give the same sums.
-enum DensityMode { kStore = 0, kBuild = 1, kWalk = 2, kRescan = 3, kScanAll = 4 };
+enum DensityMode { kStore = 0, kBuild = 1, kRescan = 3, kScanAll = 4 };
 
-// One chunk slot of the density pass.
-template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
-__device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceState& S, int slot,
-                                              int le_box, float4* __restrict__ tile,
-                                              uint32_t* __restrict__ buf) {
-  constexpr bool kDecide = MODE != kStore;
-  constexpr bool kScan = MODE != kWalk;
-  Chunk ch;
-  if (!load_chunk(P, S, ch, slot)) return;
-  if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
-  if ((MODE == kWalk || MODE == kRescan) && list_overflow(P, S, ch) != (MODE == kRescan)) return;
-  const Home h = load_home<DIM>(P, S, ch);
-  const double mi = S.m[h.ii];
-  uint32_t* list = (MODE == kStore || MODE == kBuild) ? S.nlist : nullptr;
-  double rho;
-  int rechecks = 0, cnt = 0, nin;
-  if (MIXED) {
-    using Pol = DensityMixed<DIM, kDecide>;
-    Pol pol{P, S, h, KahanF{}};
-    pol.acc.add(P.density_type == 1 ? (float)(P.w0 * mi) : (float)P.w0);
-    if constexpr (kScan)
-      cnt = staged_scan<DIM, Pol, TILE, BUF, kDecide>(P, S, ch, h, pol, tile, buf, rechecks, list);
-    else
-      for_each_listed<DIM>(P, S, ch, h, pol, buf);
-    rho = pol.acc.value();
-    nin = kDecide ? pol.nin : cnt;
-    rechecks += pol.rechecks;
-  } else {
-    // self term first (particles_compute_density.F90:369-558)
-    using Pol = DensityF64<DIM, kDecide>;
-    Pol pol{P, S, h, P.density_type == 1 ? P.w0 * mi : P.w0};
-    if constexpr (kScan)
-      cnt = staged_scan<DIM, Pol, TILE, BUF, kDecide>(P, S, ch, h, pol, tile, buf, rechecks, list);
-    else
-      for_each_listed<DIM>(P, S, ch, h, pol, buf);
-    rho = pol.acc;
-    nin = kDecide ? pol.nin : cnt;
-    rechecks += pol.rechecks;
-  }
-  if (!h.active) return;
-  const int i = h.i;
+// Density epilogue of particle i with number (or mass) density sum rho.
+template <int DIM>
+__device__ __forceinline__ void finish_density(const DevParams& P, const DeviceState& S, int i,
+                                               double mi, double rho, int nin, int rechecks) {
   // colloid boundary particles of constant density take the initial
   // density rho (number density rho / m) instead of the sum
   // (particles_compute_density.F90:442-473, 526-556)
@@ -1065,14 +1239,109 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
   const double bn = (P.newtonian && P.force_type <= 2) ? 1.0 / rho : 1.0 / (rho * rho);
   S.an[i] = an;
   S.bn[i] = bn;
+  S.nbr_in[i] = nin;
+  S.recheck[i] = rechecks;
+  write_force_records<DIM>(P, S, i, an, bn, press);
+}
+
+// The self term that starts a particle's density sum
+// (particles_compute_density.F90:369-558).
+template <bool MIXED>
+__device__ __forceinline__ double self_density(const DevParams& P, double mi) {
+  if (MIXED) return (double)(float)(P.density_type == 1 ? P.w0 * mi : P.w0);
+  // (FP64 sums leave the kernel's factor cw to density_of)
+  return P.density_type == 1 ? P.w0q * mi : P.w0q;
+}
+template <bool MIXED>
+__device__ __forceinline__ double density_of(const DevParams& P, double sum) {
+  return MIXED ? sum : P.cw * sum;
+}
+
+// One chunk slot of a density pass that scans the stencil.
+template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
+__device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceState& S, int slot,
+                                              int le_box, float4* __restrict__ tile,
+                                              uint32_t* __restrict__ buf) {
+  constexpr bool kDecide = MODE != kStore;
+  Chunk ch;
+  if (!load_chunk(P, S, ch, slot)) return;
+  if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
+  if (MODE == kRescan && !list_overflow(P, S, ch)) return;
+  const Home h = load_home<DIM>(P, S, ch);
+  const double mi = S.m[h.ii];
+  uint32_t* list = (MODE == kStore || MODE == kBuild) ? S.nlist : nullptr;
+  using Pol = std::conditional_t<MIXED, DensityMixed<DIM, kDecide>, DensityF64<DIM, kDecide>>;
+  Pol pol{P, S, h, {}};
+  if constexpr (MIXED)
+    pol.acc.add((float)self_density<true>(P, mi));
+  else
+    pol.acc = self_density<false>(P, mi);
+  int rechecks = 0;
+  const int cnt =
+      staged_scan<DIM, Pol, TILE, BUF, kDecide>(P, S, ch, h, pol, tile, buf, rechecks, list);
+  double rho;
+  if constexpr (MIXED)
+    rho = pol.acc.value();
+  else
+    rho = density_of<false>(P, pol.acc);
+  if (!h.active) return;
+  const int i = h.i;
   if (MODE == kStore || MODE == kBuild) S.nbr_count[i] = cnt;
   if (MODE == kBuild && cnt > P.list_cap) S.gate[2] = 1;  // every writer stores 1
   // the shear time of the build (the copies across sheared faces drift
   // from their build positions as it advances)
   if (MODE == kBuild && i == 0) S.time_dev[3] = S.time_dev[1];
-  S.nbr_in[i] = nin;
-  S.recheck[i] = rechecks;
-  write_force_records<DIM>(P, S, i, an, bn, press);
+  finish_density<DIM>(P, S, i, mi, rho, kDecide ? pol.nin : cnt, rechecks + pol.rechecks);
+}
+
+// The walk of the step's Verlet lists: NQ quarters of a chunk per workgroup.
+// Quarters one after the other let the epilogue (equation of state, force
+// records) run once on 64 lanes; a small box takes one quarter per workgroup
+// to fill the GPU.  QUINTIC: the quintic spline and the number density as
+// constants, so the batch's terms carry no branches.
+template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ>
+__global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState S) {
+  if (S.gate[0] != 0) return;
+  __shared__ __align__(16) double lds[kTermWords<1>];
+  const int le_box = P.le_g;
+  if (!LE) P.le_g = -1;
+  if (QUINTIC) {
+    P.kernel_type = 1;
+    P.density_type = 2;
+  }
+  int q0;
+  Chunk ch;
+  if (!load_chunk(P, S, ch, quarter_slot<NQ>(blockIdx.x, q0))) return;
+  if (ch.p0 + kQuarter * q0 >= ch.p1) return;
+  if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
+  if (S.gate[2] != 0 && list_overflow(P, S, ch)) return;
+  const int lane = threadIdx.x;
+  double rho = 0.0;
+  int nin = 0, rechecks = 0;
+#pragma unroll 1
+  for (int q = 0; q < NQ && ch.p0 + kQuarter * (q0 + q) < ch.p1; ++q) {
+    const Home h = load_quarter_home<DIM>(P, S, ch, q0 + q);
+    using Pol = std::conditional_t<MIXED, DensityMixed<DIM, true>, DensityF64<DIM, true>>;
+    Pol pol{P, S, h, {}};
+    walk_quarter<DIM>(P, S, ch, q0 + q, h, pol,
+                      self_density<MIXED>(P, QUINTIC ? 1.0 : S.m[h.ii]), lds);
+    int in = pol.nin, re = pol.rechecks;
+    in += __shfl_xor(in, 1);
+    re += __shfl_xor(re, 1);
+    in += __shfl_xor(in, 2);
+    re += __shfl_xor(re, 2);
+    const double r = quarter_sum(lds, lane & 15, 0);
+    in = __shfl(in, 4 * (lane & 15));
+    re = __shfl(re, 4 * (lane & 15));
+    if ((lane >> 4) == q) {
+      rho = r;
+      nin = in;
+      rechecks = re;
+    }
+  }
+  const int i = ch.p0 + kQuarter * q0 + lane;
+  if (lane >= kQuarter * NQ || i >= ch.p1) return;
+  finish_density<DIM>(P, S, i, S.m[i], density_of<MIXED>(P, rho), nin, rechecks);
 }
 
 // The rescan (kRescan) has work only after a list overflowed at the build;
@@ -1081,13 +1350,12 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
 template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
 __global__ __launch_bounds__(kWave) void k_density(DevParams P, DeviceState S) {
   if (MODE == kBuild && S.gate[0] == 0) return;
-  if ((MODE == kWalk || MODE == kRescan) && S.gate[0] != 0) return;
+  if (MODE == kRescan && S.gate[0] != 0) return;
   // no list overflowed at the build: nothing to rescan
   if (MODE == kRescan && S.gate[2] == 0) return;
-  constexpr bool kScan = MODE != kWalk;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
-  __shared__ float4 tile[kScan ? TILE + 1 : 1];
+  __shared__ float4 tile[TILE + 1];
   // whole groups of 8 rows: the final flush stores the last group of a
   // lane's entries as 8 rows, of which those past its count are padding
   __shared__ uint32_t buf[(BUF + 7) / 8 * 8 * kWave];
@@ -1155,11 +1423,36 @@ __device__ __forceinline__ void noise_vector(const DevParams& P, int64_t step, u
   }
 }
 
+// One FP64 force record, gathered from its four planes.
+struct RecF64 {
+  double2 a, b, c, d;  // (x, y), (z, p/n^2), (vx, vy), (vz, 1/n^2)
+  uint32_t pid;        // with thermal noise
+  double2 q0, q1, q2;  // Oldroyd-B: Pi / n^2 as (xx, yy), (zz, xy), (xz, yz)
+};
+template <bool TENSOR>
+__device__ __forceinline__ RecF64 load_rec(const DevParams& P, const DeviceState& S, uint32_t j) {
+  const double2* __restrict__ pl = reinterpret_cast<const double2*>(S.rec64);
+  const int64_t n = P.n;
+  RecF64 r;
+  r.a = load_at(pl, j);
+  r.b = load_at(pl + n, j);
+  r.c = load_at(pl + 2 * n, j);
+  r.d = load_at(pl + 3 * n, j);
+  r.pid = P.noise ? (uint32_t)load_at(S.pid, j) : 0u;
+  if (TENSOR) {
+    const double2* __restrict__ pt = reinterpret_cast<const double2*>(S.pt64);
+    r.q0 = load_at(pt, j);
+    r.q1 = load_at(pt + n, j);
+    r.q2 = load_at(pt + 2 * n, j);
+  }
+  return r;
+}
+
 // force types: 3 Hu-Adams, 4 Hu-Adams angular, 5 Oldroyd-B (non-Newtonian
-// Hu-Adams).  The bodies sum m_i times the acceleration; finish_force
-// divides by m_i once.  DECIDE (Verlet lists): the entries are candidates
-// within rc + skin and the body skips those outside the cut-off, deciding
-// exactly as the density pass of the same step did.
+// Hu-Adams).  The bodies sum m_i times the acceleration (and the Oldroyd-B
+// velocity gradient); finish_force divides by m_i once.  DECIDE (Verlet
+// lists): the entries are candidates within rc + skin; those outside the
+// cut-off add 0.
 template <int DIM, int FT, bool COLL = false, bool DECIDE = false>
 struct ForceF64 {
   const DevParams& P;
@@ -1168,8 +1461,13 @@ struct ForceF64 {
   double vi0, vi1, vi2, ai, bi, pi, inv_ni;
   uint32_t pidi;
   int64_t step;            // noise step (the context's marching step)
-  double f0 = 0.0, f1 = 0.0, f2 = 0.0;
-  double L[9];
+  // the acceleration's components, then the velocity gradient's
+  static constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
+  double sum[kTerms];
+  // kUnit: the terms leave out the factor cg of the kernel gradient, and the
+  // velocity gradient's leave out 1 / n_i (not around colloids): finish_pairs
+  static constexpr bool kUnit = FT == 3 || FT == 5;
+  // Oldroyd-B: own Pi / n_i^2 (Pi for the angular form)
   double pti[9];
   // colloids: own species id; a boundary particle's position relative to
   // the nearest image of its colloid's centre and that image's velocity;
@@ -1178,79 +1476,125 @@ struct ForceF64 {
   double rxc_i[3] = {0.0, 0.0, 0.0}, vcoll_i[3] = {0.0, 0.0, 0.0};
   double le_t = 0.0;
   static constexpr bool kImages = true;
-  // Verlet lists: the walk takes eight entries at a time (two with the
-  // Oldroyd-B body's registers) and gathers their records and pids before
-  // it evaluates the first pair, so a wave keeps more loads in flight.
-  // Measured on the 128^3 box: forces 1.824 ms one entry at a time, 1.819
-  // two, 1.761 four, 1.65 eight (193 VGPRs, two waves per SIMD); the
-  // Oldroyd-B batch of 256 boxes 6.62 -> 6.23 ms with two.
-  // With colloids the Verlet walk takes twos (512 spheres of radius 5 in
-  // the sheared 128^3 box: forces 3.66 ms one at a time, 3.31 in twos, 3.69
-  // in fours; the substitution branch's registers leave no room for more).
   static constexpr bool kBatched = DECIDE;
-  static constexpr int kBatch = COLL ? 2 : (FT >= 5 ? 2 : 8);
+  static constexpr int kBatch = 2;
+  static constexpr int kWalk = 2;
+  // fluid pairs of Verlet lists need no in / out decision of their own:
+  // outside the cut-off the kernel gradient is 0
+  static constexpr bool kStraight = DECIDE && !COLL;
   __device__ __forceinline__ void body(uint32_t ent) {
-    const int j = (int)(ent & kIndexMask);
+    const uint32_t j = ent & kIndexMask;
     if (COLL) {
       // two boundary particles do not interact (pp_interaction.inc: same
       // colloid CYCLE, colloid-colloid pair forces off)
       if (sidi != 0 && (ent & kBoundaryBit) != 0u) return;
     }
-    // both halves of the record into registers up front (a reference into
-    // global memory would leave each field's load at its first use)
-    const double4* rj = reinterpret_cast<const double4*>(S.rec64 + 8 * (int64_t)j);
-    const double4 ra = rj[0], rb = rj[1];
-    eval<false>(ent, ra, rb, 0u);
+    const RecF64 r = load_rec<(FT >= 5)>(P, S, j);
+    const Images o = decode_images(ent);
+    double d0, d1, d2;
+    const double r2 = pair_d2<DIM>(P, h, o, r.a.x, r.a.y, r.b.x, d0, d1, d2);
+    double t[kTerms];
+    eval(ent, r, d0, d1, d2, r2, le_dv(P, o), t);
+#pragma unroll
+    for (int c = 0; c < kTerms; ++c) sum[c] = sum[c] + t[c];
   }
   template <int NB>
   __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
-    double4 ra[NB], rb[NB];
-    uint32_t pj[NB];
+    double t[NB][kTerms];
+    Rec r[NB];
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const int j = (int)(e[k] & kIndexMask);
-      const double4* rj = reinterpret_cast<const double4*>(S.rec64 + 8 * (int64_t)j);
-      ra[k] = rj[0];
-      rb[k] = rj[1];
-      pj[k] = P.noise ? (uint32_t)S.pid[j] : 0u;
-    }
+    for (int k = 0; k < NB; ++k) r[k] = gather(e[k]);
+    terms(e, ok, r, t);
 #pragma unroll
     for (int k = 0; k < NB; ++k)
-      if (ok[k]) eval<true>(e[k], ra[k], rb[k], pj[k]);
+#pragma unroll
+      for (int c = 0; c < kTerms; ++c) sum[c] = sum[c] + t[k][c];
   }
-  // One pair from j's record; PID: j's pid given (else gathered for the
-  // noise term).
-  template <bool PID>
-  __device__ __forceinline__ void eval(uint32_t ent, const double4& ra, const double4& rb,
-                                       uint32_t pid_in) {
-    const int j = (int)(ent & kIndexMask);
-    const Images o = decode_images(ent);
-    const bool jb = COLL && (ent & kBoundaryBit) != 0u;
-    // two boundary particles do not interact
-    if (COLL && sidi != 0 && jb) return;
-    double d0, d1, d2, r2;
-    double jump;  // x velocity of j's image minus j's own
-    if (DECIDE) {
-      // the image and the sheared face crossed come from the positions
-      int sg;
-      r2 = exact_d2_verlet<DIM>(P, h, ra.x, ra.y, ra.z, d0, d1, d2, sg);
-      if (!(r2 < P.cut2)) return;
-      jump = sg == 0 ? P.le_u : (sg == 1 ? -P.le_u : 0.0);
+  using Rec = RecF64;
+  __device__ __forceinline__ Rec gather(uint32_t ent) const {
+    return load_rec<(FT >= 5)>(P, S, ent & kIndexMask);
+  }
+  // The terms of NB candidates, whose records are gathered already.
+  template <int NB>
+  __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                        Rec (&r)[NB], double (&t)[NB][kTerms]) const {
+    if constexpr (kStraight) {
+      auto square = [](double a, double b, double c) {
+        return DIM == 3 ? fma(c, c, fma(b, b, a * a)) : fma(b, b, a * a);
+      };
+      // the plain differences, a branch of the wave for the batches with a
+      // pair across a face and one for those with an empty slot: the pairs
+      // are then evaluated without branches
+      double d[NB][3], r2[NB];
+      uint64_t far = 0, empty = 0;
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        d[k][0] = h.x0 - r[k].a.x;
+        d[k][1] = h.x1 - r[k].a.y;
+        d[k][2] = DIM == 3 ? h.x2 - r[k].b.x : 0.0;
+        r2[k] = square(d[k][0], d[k][1], d[k][2]);
+        far |= __ballot(!(r2[k] <= h.G.half2));
+        empty |= __ballot(!ok[k]);
+      }
+      if (__builtin_expect(far != 0, 0)) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          double jump = 0.0;
+          if (nearest_image<DIM>(P, h, d[k][0], d[k][1], d[k][2], jump)) {
+            if (P.le_g >= 0) r[k].c.x = r[k].c.x + jump;
+          } else {
+            // (no velocity difference either, should j's be NaN as well)
+            r[k].c = make_double2(vi0, vi1);
+            r[k].d.x = vi2;
+          }
+          r2[k] = square(d[k][0], d[k][1], d[k][2]);
+        }
+      }
+      // an empty slot holds the lane's own particle, no separation and no
+      // velocity difference: at a squared distance outside the cut-off it
+      // adds 0
+      if (__builtin_expect(empty != 0, 0)) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k) r2[k] = ok[k] ? r2[k] : 4.0 * P.cut2;
+      }
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        eval(e[k], r[k], d[k][0], d[k][1], d[k][2], r2[k], 0.0, t[k]);
     } else {
-      r2 = pair_d2<DIM>(P, h, o, ra.x, ra.y, ra.z, d0, d1, d2);
-      jump = le_dv(P, o);
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+#pragma unroll
+        for (int c = 0; c < kTerms; ++c) t[k][c] = 0.0;
+        // two boundary particles do not interact
+        if (!ok[k] || (COLL && sidi != 0 && (e[k] & kBoundaryBit) != 0u)) continue;
+        // the image and the sheared face crossed come from the positions
+        double d0, d1, d2;
+        int sg;
+        const double r2 =
+            exact_d2_verlet<DIM>(P, h, r[k].a.x, r[k].a.y, r[k].b.x, d0, d1, d2, sg);
+        if (!(r2 < P.cut2)) continue;
+        eval(e[k], r[k], d0, d1, d2, r2, sg == 0 ? P.le_u : (sg == 1 ? -P.le_u : 0.0), t[k]);
+      }
     }
+  }
+  // The terms of one pair: j's record, the separation d and its square, the
+  // x velocity of j's image minus j's own.
+  __device__ __forceinline__ void eval(uint32_t ent, const RecF64& rj, double d0, double d1,
+                                       double d2, double r2, double jump,
+                                       double (&t)[kTerms]) const {
+    const int j = (int)(ent & kIndexMask);
+    const uint32_t pidj = rj.pid;
+    const bool jb = COLL && (ent & kBoundaryBit) != 0u;
     const double ir = rsqrt_nr(r2);
     const double r = r2 * ir;
-    double w, gw;
-    kernel_eval(P, r * P.inv_h, w, gw);
+    const double gw = kUnit ? kernel_g(P, r) : P.cg * kernel_g(P, r);
     // (without sheared faces the jump is the constant 0 and no add is made)
-    double u0 = vi0 - (P.le_g >= 0 ? rb.x + jump : rb.x), u1 = vi1 - rb.y,
-           u2 = DIM == 3 ? vi2 - rb.z : 0.0;
-    const double bj = rb.w;
+    double u0 = vi0 - (P.le_g >= 0 && !kStraight ? rj.c.x + jump : rj.c.x), u1 = vi1 - rj.c.y,
+           u2 = DIM == 3 ? vi2 - rj.d.x : 0.0;
+    const double an = rj.b.y, bj = rj.d.y;
     // pressure terms: p_i / n_i^2 + p_j / n_j^2 (type 3), (p_i + p_j) / 2 (type 4)
     double psum = 0.0, pij = 0.0;
-    if (FT <= 3) psum = ai + ra.w;
+    if (FT <= 3) psum = ai + an;
     if (FT == 4) pij = (pi + S.p[j]) * 0.5;
     // with a colloid boundary particle in an Oldroyd-B flow both sides take
     // the fluid particle's 1/n^2 and Pi/n^2
@@ -1262,10 +1606,10 @@ struct ForceF64 {
       // particle's velocity changes, and its pressure (Newtonian) or its
       // number density and pressure tensor (Oldroyd-B)
       double pb;
-      colloid_substitute(j, jb ? S.sid[j] : 0, ra, rb, d0, d1, d2, jump, u0, u1, u2, pb);
-      if (FT == 3) psum = sidi == 0 ? ai + pb * bj : pb * bi + ra.w;
+      colloid_substitute(j, jb ? S.sid[j] : 0, rj, d0, d1, d2, jump, u0, u1, u2, pb);
+      if (FT == 3) psum = sidi == 0 ? ai + pb * bj : pb * bi + an;
       // Morris and Espanol: bi, bj = 1/rho
-      if (FT <= 2) psum = sidi == 0 ? ai + pb * (bj * bj) : pb * (bi * bi) + ra.w;
+      if (FT <= 2) psum = sidi == 0 ? ai + pb * (bj * bj) : pb * (bi * bi) + an;
       if (FT == 4) pij = pb;
       if (FT == 5) bsum = sidi == 0 ? bi + bi : bj + bj;
     }
@@ -1291,7 +1635,7 @@ struct ForceF64 {
       a0 = fd1 * u0 + se * d0;
       a1 = fd1 * u1 + se * d1;
       a2 = fd1 * u2 + se * d2;
-      if (P.noise) espanol_noise(PID ? pid_in : (uint32_t)S.pid[j], d0, d1, d2, ir, gnn, a0, a1, a2);
+      if (P.noise) espanol_noise(pidj, d0, d1, d2, ir, gnn, a0, a1, a2);
     } else if (FT == 4) {
       // rhs_force_ff_Newtonian_HuAdams_angular.F90:166-229: everything
       // along e = d / r
@@ -1299,9 +1643,8 @@ struct ForceF64 {
       const double aij = (bi + bj) * gw;
       double sc = P.eta_coef * P.eta * aij * du * (ir * ir) - aij * pij;
       if (P.noise) {
-        const uint32_t pj_ = PID ? pid_in : (uint32_t)S.pid[j];
         float g[4];
-        pair_normals(P.seed, pidi < pj_ ? pidi : pj_, pidi < pj_ ? pj_ : pidi, step, g);
+        pair_normals(P.seed, pidi < pidj ? pidi : pidj, pidi < pidj ? pidj : pidi, step, g);
         sc = sc + (double)g[0] * P.sqrt_2kt_eta * sqrt_nr(-P.eta_coef * aij * ir) * P.inv_sqrt_dt;
       }
       sc = sc * ir;
@@ -1310,7 +1653,7 @@ struct ForceF64 {
       a2 = sc * d2;
     } else {
       const double gir = gw * ir;
-      const double fd = P.eta * (FT >= 5 ? bsum : bi + bj) * gir;
+      const double fd = (COLL && FT >= 5 ? P.eta * bsum : fma(P.eta, bj, P.eta * bi)) * gir;
       if (FT == 3) {
         // rhs_force_ff_Newtonian_HuAdams.F90:140-237
         const double fcr = psum * gir;
@@ -1322,18 +1665,18 @@ struct ForceF64 {
         // FT 6, differs only in the noise; the angular form, FT 7, below) with
         // Pi = (p + G) I - G c (particles_compute_pressure_tensor.F90:114-133),
         // and the velocity gradient of pp_vgt_ip.inc:16-20
-        const double du[3] = {-u0, -u1, -u2};
         const double dx[3] = {d0, d1, d2};
         // a boundary particle's gradient divides by its fluid partner's n
-        const double gfac = gw * ((cpair && sidi != 0) ? 1.0 / S.rho[j] : inv_ni) * ir;
+        const double gfac =
+            COLL ? gir * ((cpair && sidi != 0) ? 1.0 / S.rho[j] : inv_ni) : gir;
+        const double ug[3] = {-u0 * gfac, -u1 * gfac, -u2 * gfac};
 #pragma unroll
         for (int b = 0; b < DIM; ++b)
 #pragma unroll
-          for (int a = 0; a < DIM; ++a) L[a + DIM * b] = fma(du[a] * dx[b], gfac, L[a + DIM * b]);
-        // j's Pi / n^2 from its 48-byte record (c is symmetric)
-        const double2* __restrict__ rp = reinterpret_cast<const double2*>(S.pt64 + 6 * (int64_t)j);
-        const double2 q0 = rp[0], q1 = rp[1], q2 = rp[2];
-        const double pjb[9] = {q0.x, q1.y, q2.x, q1.y, q0.y, q2.y, q2.x, q2.y, q1.x};
+          for (int a = 0; a < DIM; ++a) t[DIM + a + DIM * b] = ug[a] * dx[b];
+        // j's Pi / n^2 (c is symmetric)
+        const double pjb[9] = {rj.q0.x, rj.q1.y, rj.q2.x, rj.q1.y, rj.q0.y,
+                               rj.q2.y, rj.q2.x, rj.q2.y, rj.q1.x};
         double fc[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int jj = 0; jj < DIM; ++jj)
@@ -1341,12 +1684,12 @@ struct ForceF64 {
           for (int a = 0; a < DIM; ++a) {
             const double ptjb = DIM == 3 ? pjb[a + 3 * jj] : pjb[(a == jj ? (a == 0 ? 0 : 4) : 1)];
             // colloid pairs: the fluid particle's Pi / n^2 on both sides
-            double t = cpair ? (sidi == 0 ? 2.0 * (pti[a + DIM * jj] * bi) : ptjb + ptjb)
-                             : pti[a + DIM * jj] * bi + ptjb;
+            const double ptib = FT == 7 ? pti[a + DIM * jj] * bi : pti[a + DIM * jj];
+            double pij2 = cpair ? (sidi == 0 ? ptib + ptib : ptjb + ptjb) : ptib + ptjb;
             // rhs_force_ff_non_Newtonian_HuAdams_angular.F90: the diagonal
             // averaged, (Pi_i + Pi_j) / 2 (1/n_i^2 + 1/n_j^2)
-            if (FT == 7 && a == jj) t = 0.5 * (pti[a + DIM * jj] + ptjb / bj) * (bi + bj);
-            fc[jj] = fc[jj] + t * dx[a];
+            if (FT == 7 && a == jj) pij2 = 0.5 * (pti[a + DIM * jj] + ptjb / bj) * (bi + bj);
+            fc[jj] = fc[jj] + pij2 * dx[a];
           }
         if (FT == 7) {
           // its dissipative term acts along e: eta_coef eta (1/n_i^2 +
@@ -1363,35 +1706,35 @@ struct ForceF64 {
         }
       }
       if (FT == 6 && P.noise) {
-        espanol_noise(PID ? pid_in : (uint32_t)S.pid[j], d0, d1, d2, ir,
+        espanol_noise(pidj, d0, d1, d2, ir,
                       gw * ir * inv_ni / S.rho[j], a0, a1, a2);
       } else if (FT != 7 && P.noise) {
-        // f_r W e with W e = s (ca g + cb (g.e) e), e = d / r, s = +1 when
+        // f_r W e with W e = s ca (g + cb / ca (g.e) e), e = d / r, s = +1 when
         // pid_i < pid_j (noise_vector), written on d to save operations
-        const uint32_t pidj = PID ? pid_in : (uint32_t)S.pid[j];
         float g[4];
         pair_normals(P.seed, pidi < pidj ? pidi : pidj, pidi < pidj ? pidj : pidi, step, g);
-        // sqrt(-4 kT f_d) / sqrt(dt) as one root (the factor is uniform)
-        const double fr = sqrt_nr((-4.0 * P.kt / P.dt) * fd);
-        const double sfr = pidi < pidj ? fr : -fr;
-        const double ca = 0.70710678118654752440;
+        // sqrt(-4 kT f_d / dt) / sqrt(2) as one root, in units of cg < 0 (the
+        // unit turns the sign)
+        const double fr = sqrt_pos(P.knoise * fd);
+        const double sfr = pidi < pidj ? -fr : fr;
         const double g0 = (double)g[0], g1 = (double)g[1];
         if (DIM == 3) {
-          const double cb = 0.81649658092772603273 - 0.70710678118654752440;
+          // cb / ca
+          const double cba = 0.81649658092772603273 * 1.41421356237309504880 - 1.0;
           const double g2 = (double)g[2];
-          const double k = cb * fma(g2, d2, fma(g1, d1, g0 * d0)) * (ir * ir);
-          a0 = fma(sfr, fma(k, d0, ca * g0), a0);
-          a1 = fma(sfr, fma(k, d1, ca * g1), a1);
-          a2 = fma(sfr, fma(k, d2, ca * g2), a2);
+          const double k = cba * fma(g2, d2, fma(g1, d1, g0 * d0)) * (ir * ir);
+          a0 = fma(sfr, fma(k, d0, g0), a0);
+          a1 = fma(sfr, fma(k, d1, g1), a1);
+          a2 = fma(sfr, fma(k, d2, g2), a2);
         } else {
-          a0 = fma(sfr, ca * g0, a0);
-          a1 = fma(sfr, ca * g1, a1);
+          a0 = fma(sfr, g0, a0);
+          a1 = fma(sfr, g1, a1);
         }
       }
     }
-    f0 = f0 + a0;
-    f1 = f1 + a1;
-    if (DIM == 3) f2 = f2 + a2;
+    t[0] = a0;
+    t[1] = a1;
+    if (DIM == 3) t[2] = a2;
   }
 
   // Espanol's thermal force (rhs_force_ff_Newtonian_Espanol.F90:198-249,
@@ -1435,14 +1778,13 @@ struct ForceF64 {
   // fluid particle sits at r_xc + (x_f - x_c) and moves at its image
   // velocity, so both sides of the pair see the same relative velocity
   // u = v_i - v_j.
-  __device__ __forceinline__ void colloid_substitute(int j, int sj, const double4& ra,
-                                                     const double4& rb, double d0, double d1,
-                                                     double d2, double jump, double& u0,
-                                                     double& u1, double& u2, double& pb) {
+  __device__ __forceinline__ void colloid_substitute(int j, int sj, const RecF64& rj, double d0,
+                                                     double d1, double d2, double jump, double& u0,
+                                                     double& u1, double& u2, double& pb) const {
     double vc[3];
     if (sidi == 0) {
       const CollHot C = S.coll_hot[sj - 1];
-      const double xj[3] = {ra.x, ra.y, DIM == 3 ? ra.z : 0.0};
+      const double xj[3] = {rj.a.x, rj.a.y, DIM == 3 ? rj.b.x : 0.0};
       double rxc[3], vcoll[3];
       coll_nearest<DIM>(P, C, xj, le_t, rxc, vcoll);
       const double rxf[3] = {rxc[0] + d0, rxc[1] + d1, DIM == 3 ? rxc[2] + d2 : 0.0};
@@ -1455,7 +1797,7 @@ struct ForceF64 {
     } else {
       const CollHot C = S.coll_hot[sidi - 1];
       const double rxf[3] = {rxc_i[0] - d0, rxc_i[1] - d1, DIM == 3 ? rxc_i[2] - d2 : 0.0};
-      const double vf[3] = {P.le_g >= 0 ? rb.x + jump : rb.x, rb.y, DIM == 3 ? rb.z : 0.0};
+      const double vf[3] = {P.le_g >= 0 ? rj.c.x + jump : rj.c.x, rj.c.y, DIM == 3 ? rj.d.x : 0.0};
       coll_noslip<DIM>(P, C, rxc_i, vcoll_i, rxf, vf, vc);
       u0 = vc[0] - vf[0];
       u1 = vc[1] - vf[1];
@@ -1473,18 +1815,24 @@ struct ForceMixed {
   float vi0, vi1, vi2, ai, bi, pi;
   uint32_t pidi;
   int64_t step;            // noise step (the context's marching step)
-  KahanF f0, f1, f2;
-  // Oldroyd-B: own Pi / n^2 (xx, yy, zz, xy, xz, yz), 1 / n, velocity gradient
+  // Oldroyd-B: own Pi / n^2 (xx, yy, zz, xy, xz, yz), 1 / n
   float pb[6];
   float inv_ni;
-  WideF L[DIM * DIM];
+  // the acceleration's components, then the velocity gradient's: with
+  // Verlet lists FP64 sums of the FP32 terms; per-step lists sum the
+  // acceleration compensated in FP32
+  static constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
+  std::conditional_t<DECIDE, WideF, KahanF> facc[DIM];
+  WideF gacc[DIM * DIM];
   static constexpr bool kImages = false;
-  // Verlet lists: entries four at a time, the records of all four
-  // gathered before the first pair is evaluated (the 128^3 Tait box: forces
-  // 1.27 ms one at a time, 1.16 in fours, 1.19 in eights; 256 Oldroyd-B
-  // boxes of 2k-60k particles: 3.94 in twos, 3.87 in fours)
+  // Verlet lists: the records of a lane's kWalk entries are gathered before
+  // the first pair is evaluated
   static constexpr bool kBatched = DECIDE;
-  static constexpr int kBatch = 4;
+  static constexpr int kBatch = 2;
+  static constexpr int kWalk = FT >= 5 ? 2 : 4;
+  __device__ __forceinline__ double sum(int c) const {
+    return c < DIM ? facc[c < DIM ? c : 0].value() : gacc[c < DIM ? 0 : c - DIM].value();
+  }
   // j's records: FP32 position (w: p/n^2 or p, Newtonian), velocity (w:
   // 1/n^2, or the pid bits for Oldroyd-B), pid, and the Oldroyd-B
   // (1/n^2, Pxx, Pyy, Pzz) and (Pxy, Pxz, Pyz, 0)
@@ -1508,31 +1856,62 @@ struct ForceMixed {
     }
     return r;
   }
+  __device__ __forceinline__ Rec gather(uint32_t ent) const {
+    return load_rec((int)(ent & kIndexMask));
+  }
+  __device__ __forceinline__ void add(const float (&t)[kTerms]) {
+#pragma unroll
+    for (int c = 0; c < kTerms; ++c) {
+      if (c < DIM)
+        facc[c < DIM ? c : 0].add(t[c]);
+      else
+        gacc[c < DIM ? 0 : c - DIM].add(t[c]);
+    }
+  }
   __device__ __forceinline__ void body(uint32_t ent) {
     const int j = (int)(ent & kIndexMask);
     const Rec r = load_rec(j);
-    body_rec(j, r.x, r.v, r.pid, r.q, r.q2, decode_code(ent >> kCodeShift));
+    float t[kTerms];
+    eval(j, r.x, r.v, r.pid, r.q, r.q2, decode_code(ent >> kCodeShift), true, t);
+    add(t);
+  }
+  template <int NB>
+  __device__ __forceinline__ void terms_f(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                          Rec (&r)[NB], float (&t)[NB][kTerms]) const {
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+      eval((int)(e[k] & kIndexMask), r[k].x, r[k].v, r[k].pid, r[k].q, r[k].q2,
+           decode_code(ok[k] ? e[k] >> kCodeShift : 62u), ok[k], t[k]);
+  }
+  template <int NB>
+  __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
+                                        Rec (&r)[NB], double (&t)[NB][kTerms]) const {
+    float f[NB][kTerms];
+    terms_f(e, ok, r, f);
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int c = 0; c < kTerms; ++c) t[k][c] = (double)f[k][c];
   }
   template <int NB>
   __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
+    float t[NB][kTerms];
     Rec r[NB];
 #pragma unroll
-    for (int k = 0; k < NB; ++k) r[k] = load_rec((int)(e[k] & kIndexMask));
+    for (int k = 0; k < NB; ++k) r[k] = gather(e[k]);
+    terms_f(e, ok, r, t);
 #pragma unroll
-    for (int k = 0; k < NB; ++k)
-      if (ok[k])
-        body_rec((int)(e[k] & kIndexMask), r[k].x, r[k].v, r[k].pid, r[k].q, r[k].q2,
-                 decode_code(e[k] >> kCodeShift));
+    for (int k = 0; k < NB; ++k) add(t[k]);
   }
   // xj: cell-relative position (w: p/n^2 for Hu-Adams, p for the angular
   // form); vj: velocity (w: 1/n^2, Newtonian); Oldroyd-B qj: (1/n^2, Pxx,
   // Pyy, Pzz), q2: (Pxy, Pxz, Pyz, 0)
-  __device__ __forceinline__ void body_rec(int jidx, const float4& xj, const float4& vj,
-                                           uint32_t pidj, const float4& qj, const float4& q2,
-                                           const Offsets& o) {
+  __device__ __forceinline__ void eval(int jidx, const float4& xj, const float4& vj,
+                                       uint32_t pidj, const float4& qj, const float4& q2,
+                                       const Offsets& o, bool ok, float (&t)[kTerms]) const {
     float d0, d1, d2;
     rel_diff<DIM>(P, h, xj, o, d0, d1, d2);
-    const float r2 = mixed_s2(d0, d1, d2);
+    float r2 = mixed_s2(d0, d1, d2);
     // Verlet candidates: the pair is evaluated either way (outside the
     // cut-off the kernel gradient is 0) and only added when inside.  The
     // record's w is pinned to a register ahead of the decision (an empty
@@ -1543,7 +1922,8 @@ struct ForceMixed {
     if (DECIDE) {
       asm volatile("" : "+v"(xjw));
       int rechecks = 0;
-      use = mixed_inside<DIM>(P, S, h, jidx, r2, rechecks);
+      use = ok && mixed_inside<DIM>(P, S, h, jidx, r2, rechecks);
+      if (!ok) r2 = P.cut2_hi_f32;  // an empty slot (the lane's own particle)
     }
     const float ir = __builtin_amdgcn_rsqf(r2);
     const float r = r2 * ir;
@@ -1591,12 +1971,11 @@ struct ForceMixed {
       const float gfac = gir * inv_ni;
       const float du[3] = {-u0, -u1, -u2};
       const float dx[3] = {d0, d1, d2};
-      if (use) {
 #pragma unroll
-        for (int b = 0; b < DIM; ++b)
+      for (int b = 0; b < DIM; ++b)
 #pragma unroll
-          for (int a = 0; a < DIM; ++a) L[a + DIM * b].add(du[a] * dx[b] * gfac);
-      }
+        for (int a = 0; a < DIM; ++a)
+          t[DIM + a + DIM * b] = use ? du[a] * dx[b] * gfac : 0.f;
       if (FT == 6 && P.noise) {
         // Espanol's (A S e + B tr e) / sqrt(dt), Z = 4 kT W' / (r n_i n_j)
         float w0, w1, w2, g3;
@@ -1683,10 +2062,9 @@ struct ForceMixed {
       fi1 = sc * d1;
       fi2 = sc * d2;
     }
-    if (!use) return;
-    f0.add(fi0);
-    f1.add(fi1);
-    if (DIM == 3) f2.add(fi2);
+    t[0] = use ? fi0 : 0.f;
+    t[1] = use ? fi1 : 0.f;
+    if (DIM == 3) t[2] = use ? fi2 : 0.f;
   }
 };
 
@@ -1734,39 +2112,106 @@ __device__ __forceinline__ void conformation_rate(const DevParams& P, const Devi
     }
 }
 
-// The neighbours of a chunk: its stored lists, or (SCAN) the stencil
-// scanned again.
-template <int DIM, bool SCAN, bool SKIN, class Pol>
-__device__ __forceinline__ void visit_neighbours(const DevParams& P, const DeviceState& S,
-                                                 const Chunk& ch, const Home& h, Pol& pol,
-                                                 float4* __restrict__ tile,
-                                                 uint32_t* __restrict__ buf) {
-  if constexpr (SCAN) {
-    int rechecks = 0;
-    (void)staged_scan<DIM, Pol, kTile, kBuf, SKIN>(P, S, ch, h, pol, tile, buf, rechecks, nullptr);
-  } else {
-    (void)tile;
-    for_each_listed<DIM>(P, S, ch, h, pol, buf);
-  }
-}
-
 // The FP64 walk of per-step lists (without colloids) takes 8 KB of LDS per
 // workgroup, its entry buffer plus a reserve.  That holds it to five waves
 // per SIMD.  Its registers alone would allow six, but on the 128^3 box six
-// waves' gathers ran 6 % slower (1.99 against 1.88 ms per pass).  The
-// Verlet walk evaluates in batches from registers and takes no LDS.
+// waves' gathers ran 6 % slower (1.99 against 1.88 ms per pass).
 constexpr int kForceLdsWordsF64 = 2048;
 
-// Two launches over the same grid: SCAN = false takes the chunks whose
-// lists hold every neighbour and walks them, SCAN = true takes the others
-// and scans their stencil again.  Every chunk is done by exactly one of
-// them, and the list walk carries none of the scan's state (it needs 40 %
-// fewer registers, so more waves share a SIMD).  With colloids a box with
-// sheared faces splits the chunks once more: the Lees-Edwards
-// instantiation takes the rows within coll_le_cells of a face, the plain
-// one (a quarter fewer registers) the interior.  VERLET: the lists hold
-// the Verlet candidates and the bodies decide in / out of the cut-off.
-// One chunk slot of the force pass.
+// What the pair bodies need of the home particle ii.
+template <int DIM, int FT, bool DECIDE>
+__device__ __forceinline__ ForceMixed<DIM, FT, DECIDE> mixed_policy(const DevParams& P,
+                                                                    const DeviceState& S,
+                                                                    const Home& h) {
+  const int ii = h.ii;
+  const float4 vi = S.vr[ii];
+  const float4 qi = S.qr[ii];
+  // Newtonian records: qi.w = p/n^2 (Hu-Adams) or p (angular), vi.w = 1/n^2
+  ForceMixed<DIM, FT, DECIDE> pol{P, S, h, vi.x, vi.y, vi.z, FT <= 3 ? qi.w : 0.f, vi.w,
+                                  FT == 4 ? qi.w : 0.f,
+                                  FT >= 5 ? __float_as_uint(vi.w) : (uint32_t)S.pid[ii],
+                                  S.step_dev[0]};
+  if (FT >= 5) {
+    const float4 q2 = S.qr2[ii];
+    pol.bi = qi.x;
+    pol.pb[0] = qi.y;
+    pol.pb[1] = qi.z;
+    pol.pb[2] = qi.w;
+    pol.pb[3] = q2.x;
+    pol.pb[4] = q2.y;
+    pol.pb[5] = q2.z;
+    pol.inv_ni = (float)(1.0 / S.rho[ii]);
+  }
+  return pol;
+}
+
+template <int DIM, int FT, bool COLL, bool DECIDE>
+__device__ __forceinline__ ForceF64<DIM, FT, COLL, DECIDE> f64_policy(const DevParams& P,
+                                                                      const DeviceState& S,
+                                                                      const Home& h) {
+  const int ii = h.ii;
+  const int64_t n = P.n;
+  ForceF64<DIM, FT, COLL, DECIDE> pol{P, S, h};
+  if (COLL) {
+    pol.sidi = S.sid[ii];
+    pol.le_t = S.time_dev[1];
+    if (pol.sidi != 0) {
+      const double xi[3] = {h.x0, h.x1, DIM == 3 ? h.x2 : 0.0};
+      coll_nearest<DIM>(P, S.coll_hot[pol.sidi - 1], xi, pol.le_t, pol.rxc_i, pol.vcoll_i);
+    }
+  }
+  pol.vi0 = S.v[ii];
+  pol.vi1 = S.v[n + ii];
+  pol.vi2 = DIM == 3 ? S.v[2 * n + ii] : 0.0;
+  pol.ai = S.an[ii];
+  pol.bi = S.bn[ii];
+  pol.pi = S.p[ii];
+  pol.inv_ni = 1.0 / S.rho[ii];
+  pol.pidi = (uint32_t)S.pid[ii];
+  pol.step = S.step_dev[0];
+#pragma unroll
+  for (int q = 0; q < pol.kTerms; ++q) pol.sum[q] = 0.0;
+  if (FT >= 5) {
+    // particles_compute_pressure_tensor.F90:114-133
+#pragma unroll
+    for (int b = 0; b < DIM; ++b)
+#pragma unroll
+      for (int a = 0; a < DIM; ++a) {
+        double val = -P.G * S.ct[(int64_t)(a + DIM * b) * n + ii];
+        if (a == b) val = val + pol.pi + P.G;
+        pol.pti[a + DIM * b] = FT == 7 ? val : val * pol.bi;
+      }
+  }
+  return pol;
+}
+
+// Acceleration (and conformation rate) of particle i from its pair sums;
+// F64: with the factors the FP64 bodies leave out.
+template <int DIM, int FT, bool F64, bool COLL>
+__device__ __forceinline__ void finish_pairs(const DevParams& P, const DeviceState& S, int i,
+                                             const double* sum, bool fluid) {
+  constexpr bool kUnit = F64 && (FT == 3 || FT == 5);
+  // the Morris body sums accelerations already
+  const double inv_mi = (kUnit ? P.cg : 1.0) * (FT == 1 ? 1.0 : 1.0 / S.m[i]);
+  finish_force<DIM>(P, S, i, sum[0] * inv_mi, sum[1] * inv_mi, DIM == 3 ? sum[DIM - 1] * inv_mi : 0.0,
+                    fluid);
+  if (FT >= 5) {
+    const double fac = (kUnit ? P.cg : 1.0) * (F64 && !COLL ? 1.0 / S.rho[i] : 1.0);
+    double L[DIM * DIM];
+#pragma unroll
+    for (int q = 0; q < DIM * DIM; ++q) L[q] = sum[DIM + q] * fac;
+    conformation_rate<DIM>(P, S, i, L);
+  }
+}
+
+// One chunk slot of a force pass with one particle per lane.  Two launches
+// over the same grid: SCAN = false takes the chunks whose lists hold every
+// neighbour and walks them (per-step lists), SCAN = true takes the others
+// and scans their stencil again; every chunk is done by exactly one launch.
+// With colloids a box with sheared faces splits the chunks once more: the
+// Lees-Edwards instantiation takes the rows within coll_le_cells of a face,
+// the plain one (a quarter fewer registers) the interior.  VERLET: the scan
+// takes the Verlet candidates.
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, bool SCAN, bool VERLET>
 __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceState& S, int slot,
                                              int le_box, float4* __restrict__ tile,
@@ -1776,78 +2221,31 @@ __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceSta
   if (list_overflow(P, S, ch) != SCAN) return;
   if (COLL && le_box >= 0 && chunk_meets_le_face(le_box, ch, P.coll_le_cells) != LE) return;
   const Home h = load_home<DIM>(P, S, ch);
-  const int64_t n = P.n;
-  const int ii = h.ii;
-  // the Morris body sums accelerations already
-  const double inv_mi = FT == 1 ? 1.0 : 1.0 / S.m[ii];
-  if (MIXED) {
-    const float4 vi = S.vr[ii];
-    const float4 qi = S.qr[ii];
-    // Newtonian records: qi.w = p/n^2 (Hu-Adams) or p (angular), vi.w = 1/n^2
-    ForceMixed<DIM, FT, VERLET> pol{P, S, h, vi.x, vi.y, vi.z, FT <= 3 ? qi.w : 0.f, vi.w,
-                            FT == 4 ? qi.w : 0.f,
-                            FT >= 5 ? __float_as_uint(vi.w) : (uint32_t)S.pid[ii],
-                            S.step_dev[0]};
-    if (FT >= 5) {
-      const float4 q2 = S.qr2[ii];
-      pol.bi = qi.x;
-      pol.pb[0] = qi.y;
-      pol.pb[1] = qi.z;
-      pol.pb[2] = qi.w;
-      pol.pb[3] = q2.x;
-      pol.pb[4] = q2.y;
-      pol.pb[5] = q2.z;
-      pol.inv_ni = (float)(1.0 / S.rho[ii]);
+  double sum[DIM + DIM * DIM];
+  bool fluid = true;
+  auto visit = [&](auto& pol) {
+    if constexpr (SCAN) {
+      int rechecks = 0;
+      (void)staged_scan<DIM, std::remove_reference_t<decltype(pol)>, kTile, kBuf, VERLET>(
+          P, S, ch, h, pol, tile, buf, rechecks, nullptr);
+    } else {
+      (void)tile;
+      for_each_listed<DIM>(P, S, ch, h, pol, buf);
     }
-    visit_neighbours<DIM, SCAN, VERLET>(P, S, ch, h, pol, tile, buf);
-    if (!h.active) return;
-    finish_force<DIM>(P, S, h.i, pol.f0.value() * inv_mi, pol.f1.value() * inv_mi,
-                      DIM == 3 ? pol.f2.value() * inv_mi : 0.0);
-    if (FT >= 5) {
-      double Ld[DIM * DIM];
+  };
+  if constexpr (MIXED) {
+    auto pol = mixed_policy<DIM, FT, VERLET>(P, S, h);
+    visit(pol);
 #pragma unroll
-      for (int q = 0; q < DIM * DIM; ++q) Ld[q] = pol.L[q].value();
-      conformation_rate<DIM>(P, S, h.i, Ld);
-    }
+    for (int c = 0; c < pol.kTerms; ++c) sum[c] = pol.sum(c);
   } else {
-    ForceF64<DIM, FT, COLL, VERLET> pol{P, S, h};
-    if (COLL) {
-      pol.sidi = S.sid[ii];
-      pol.le_t = S.time_dev[1];
-      if (pol.sidi != 0) {
-        const double xi[3] = {h.x0, h.x1, DIM == 3 ? h.x2 : 0.0};
-        coll_nearest<DIM>(P, S.coll_hot[pol.sidi - 1], xi, pol.le_t, pol.rxc_i, pol.vcoll_i);
-      }
-    }
-    pol.vi0 = S.v[ii];
-    pol.vi1 = S.v[n + ii];
-    pol.vi2 = DIM == 3 ? S.v[2 * n + ii] : 0.0;
-    pol.ai = S.an[ii];
-    pol.bi = S.bn[ii];
-    pol.pi = S.p[ii];
-    pol.inv_ni = 1.0 / S.rho[ii];
-    pol.pidi = (uint32_t)S.pid[ii];
-    pol.step = S.step_dev[0];
+    auto pol = f64_policy<DIM, FT, COLL, VERLET>(P, S, h);
+    visit(pol);
 #pragma unroll
-    for (int q = 0; q < 9; ++q) pol.L[q] = 0.0;
-    if (FT >= 5) {
-      // particles_compute_pressure_tensor.F90:114-133
-#pragma unroll
-      for (int b = 0; b < DIM; ++b)
-#pragma unroll
-        for (int a = 0; a < DIM; ++a) {
-          double val = -P.G * S.ct[(int64_t)(a + DIM * b) * n + ii];
-          if (a == b) val = val + pol.pi + P.G;
-          pol.pti[a + DIM * b] = val;
-        }
-    }
-    visit_neighbours<DIM, SCAN, VERLET>(P, S, ch, h, pol, tile, buf);
-    if (!h.active) return;
-    const int i = h.i;
-    finish_force<DIM>(P, S, i, pol.f0 * inv_mi, pol.f1 * inv_mi, pol.f2 * inv_mi,
-                      !COLL || pol.sidi == 0);
-    if (FT >= 5) conformation_rate<DIM>(P, S, i, pol.L);
+    for (int c = 0; c < pol.kTerms; ++c) sum[c] = pol.sum[c];
+    fluid = !COLL || pol.sidi == 0;
   }
+  if (h.active) finish_pairs<DIM, FT, !MIXED, COLL>(P, S, h.i, sum, fluid);
 }
 
 // With Verlet lists the rescan (SCAN) has work only if a list overflowed at
@@ -1870,6 +2268,49 @@ __global__ __launch_bounds__(kWave) void k_forces(DevParams P, DeviceState S) {
   } else {
     forces_chunk<DIM, FT, MIXED, COLL, LE, SCAN, VERLET>(P, S, blockIdx.x, le_box, tile, buf);
   }
+}
+
+// The force walk of Verlet lists: one quarter of a chunk per workgroup.
+// SPEC: the quintic spline as a constant, with (kNoisy) or without (kQuiet)
+// thermal noise, so that a batch's pairs form one block without run-time
+// branches; kAny leaves both to the parameters.
+enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
+//
+// The FP64 Hu-Adams body is held to 128 registers, four waves per SIMD; left
+// alone the compiler interleaves more of the two pairs' noise and takes 191.
+// Two entries per lane and batch: the 128^3 box takes 1.33 ms with two, 1.47
+// with four (191 registers); it took 1.66 with one particle per lane.
+template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC>
+__global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : 1) void k_force_walk(DevParams P, DeviceState S) {
+  const int le_box = P.le_g;
+  if (!LE) P.le_g = -1;
+  if (SPEC != kAny) {
+    P.kernel_type = 1;
+    P.noise = SPEC == kNoisy ? 1 : 0;
+  }
+  int quarter;
+  Chunk ch;
+  if (!load_chunk(P, S, ch, quarter_slot<1>(blockIdx.x, quarter))) return;
+  if (ch.p0 + kQuarter * quarter >= ch.p1) return;
+  if (COLL && le_box >= 0 && chunk_meets_le_face(le_box, ch, P.coll_le_cells) != LE) return;
+  if (S.gate[2] != 0 && list_overflow(P, S, ch)) return;
+  const Home h = load_quarter_home<DIM>(P, S, ch, quarter);
+  constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
+  __shared__ __align__(16) double lds[kTermWords<kTerms>];
+  auto walk = [&](auto& pol) { walk_quarter<DIM>(P, S, ch, quarter, h, pol, 0.0, lds); };
+  if constexpr (MIXED) {
+    auto pol = mixed_policy<DIM, FT, true>(P, S, h);
+    walk(pol);
+  } else {
+    auto pol = f64_policy<DIM, FT, COLL, true>(P, S, h);
+    walk(pol);
+  }
+  const int i = ch.p0 + kQuarter * quarter + (int)threadIdx.x;
+  if (threadIdx.x >= kQuarter || i >= ch.p1) return;
+  double sum[kTerms];
+#pragma unroll
+  for (int c = 0; c < kTerms; ++c) sum[c] = quarter_sum(lds, threadIdx.x, c);
+  finish_pairs<DIM, FT, !MIXED, COLL>(P, S, i, sum, !COLL || S.sid[i] == 0);
 }
 
 // ---------------------------------------------------------------------
@@ -1936,6 +2377,28 @@ __global__ __launch_bounds__(kWave) void k_signature(DevParams P, DeviceState S)
 // ---------------------------------------------------------------------
 static inline int nchunks_max(const DevParams& P) { return chunk_slots(P); }
 
+// Chunk slots from which a density walk takes a whole chunk per workgroup.
+constexpr int kWholeChunkSlots = 4096;
+
+template <int DIM, bool MIXED, bool LE>
+static void launch_density_walk(hipStream_t s, const DevParams& P, const DeviceState& S) {
+  const int slots = chunk_slots(P);
+  const dim3 b(kWave);
+  const bool quintic = P.kernel_type == 1 && P.density_type == 2;
+  if (slots >= kWholeChunkSlots) {
+    if (quintic)
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 4>), dim3(slots), b, 0, s, P, S);
+    else
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 4>), dim3(slots), b, 0, s, P, S);
+  } else {
+    if (quintic)
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 1>), dim3(4 * slots), b, 0, s, P, S);
+    else
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 1>), dim3(4 * slots), b, 0, s, P,
+                         S);
+  }
+}
+
 // Workgroups of a rescan launch (a multiple of 8, at most the slots): few
 // enough that the launch is cheap on the steps without an overflowed list
 // (on the 128^3 box, whose 33k slots each took a workgroup before, the two
@@ -1977,17 +2440,17 @@ static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceSt
   // selects it (build, or walk + rescan of overflowed chunks); a box with
   // sheared faces splits the chunks between the Lees-Edwards and the plain
   // instantiations, as its per-step lists do
-  dim3 g(nchunks_max(P)), b(kWave);
+  const dim3 b(kWave);
   if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
     if (P.le_g >= 0) {
       launch_density_shape<DIM, MIXED, true, kBuild>(s, P, S);
-      hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, true, kWalk>), g, b, 0, s, P, S);
+      launch_density_walk<DIM, MIXED, true>(s, P, S);
       hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, true, kRescan>), rescan_grid(P), b,
                          0, s, P, S);
     }
   }
   launch_density_shape<DIM, MIXED, false, kBuild>(s, P, S);
-  hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, false, kWalk>), g, b, 0, s, P, S);
+  launch_density_walk<DIM, MIXED, false>(s, P, S);
   hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, false, kRescan>), rescan_grid(P), b, 0,
                      s, P, S);
   launch_lists_current(s, S);
@@ -2023,15 +2486,25 @@ static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceStat
     // as the lists rebuilt every step: with colloids the chunks near a
     // sheared face take the Lees-Edwards instantiation and the others the
     // plain one; without, a sheared box runs the Lees-Edwards one alone
+    const dim3 gq(4 * chunk_slots(P));
     if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
       if (P.le_g >= 0) {
-        hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, true, false, true>), g, b, 0, s, P, S);
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, true, kAny>), gq, b, 0, s, P, S);
         hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, true, true, true>), rescan_grid(P), b,
                            0, s, P, S);
       }
     }
     if (P.le_g < 0 || COLL) {
-      hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, false, false, true>), g, b, 0, s, P, S);
+      constexpr int kWithNoise = !COLL && FT != 1 && FT != 7 ? kNoisy : kAny;
+      constexpr int kNoNoise = !COLL ? kQuiet : kAny;
+      if (P.kernel_type != 1)
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kAny>), gq, b, 0, s, P, S);
+      else if (P.noise)
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kWithNoise>), gq, b, 0, s, P,
+                           S);
+      else
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kNoNoise>), gq, b, 0, s, P,
+                           S);
       hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, false, true, true>), rescan_grid(P), b,
                          0, s, P, S);
     }

@@ -151,6 +151,8 @@ __device__ __forceinline__ double track_particle(const DevParams& P, const Devic
     const double dd = raw + w[d];
     d2 = d2 + dd * dd;
   }
+  // the (x, y) plane of the FP64 records follows the positions
+  if (!P.mixed) reinterpret_cast<double2*>(S.rec64)[i] = make_double2(xv[0], xv[1]);
   if (P.mixed || P.le_g >= 0) {
     const int kl = S.key_sorted[i] - g.cell_base;
     const int cc[3] = {kl % g.nm[0], (kl / g.nm[0]) % g.nm[1], kl / (g.nm[0] * g.nm[1])};
