@@ -267,6 +267,14 @@ int derive_params(const sdpd_params& p, DevParams& P, const char*& err) {
   P.ktf = (float)P.kt;
   P.inv_sqrt_dtf = (float)P.inv_sqrt_dt;
   P.sqrt_2kt_etaf = (float)std::sqrt(2.0 * P.kt * P.eta);
+  {
+    // Hu-Adams (also Oldroyd-B): the kernel gradient's factor split into a
+    // power of two, kept in the FP32 records, and the rest
+    const double cgn = (p.kernel_type == 1 ? 5.0 : 12.0) * P.coef_grad;
+    P.rec_scale = p.rhs_force_type == 3 ? std::exp2(std::round(std::log2(-cgn))) : 1.0;
+    P.sum_scale = p.rhs_force_type == 3 ? cgn / P.rec_scale : 1.0;
+    P.knoisef = (float)(2.0 * P.kt / P.dt * (P.rec_scale / -cgn));
+  }
   return SDPD_OK;
 }
 
@@ -371,6 +379,7 @@ int build_geometry(sdpd_ctx* c) {
       }
       g.csf[d] = (float)g.cs[d];
     }
+    sdpd::set_fixed_point(g, dim, c->prm.cut_off);
     g.cell_base = (int32_t)cells;
     g.row_base = (int32_t)rows;
     const int nr = g.nm[1] * g.nm[2];
@@ -416,7 +425,7 @@ void free_state(DeviceState& S) {
                   S.rstart,   S.runsorted, S.rlpdx,  S.nlist,   S.nbr_sig_count,
                   S.row_nchunk, S.row_chunk_off, S.chunk_row, S.scan_tmp, S.rec64,
                   (void*)S.geo, S.rep,      S.rep_alt,  S.row_cell, S.row_len,  S.row_rep,
-                  S.rep_stats, S.qr2,     S.step_dev, S.time_dev, S.sid,
+                  S.rep_stats, S.qr2,     S.xq,       S.an32,     S.step_dev, S.time_dev, S.sid,
                   S.sid_alt,  S.slot_of,  (void*)S.coll_hot, (void*)S.coll, S.coll_start,
                   S.coll_members, S.x_ref, S.gate, (void*)S.disp, S.nbr_in};
   for (void* q : ptrs)
@@ -463,6 +472,8 @@ int alloc_state(sdpd_ctx* c, int n) {
     ALLOC(vr, N);
     ALLOC(qr, N);
     if (!P.newtonian) ALLOC(qr2, N);
+    ALLOC(xq, N);
+    ALLOC(an32, N);
   } else {
     ALLOC(rec64, 8 * N);
     if (!P.newtonian) ALLOC(pt64, 6 * N);

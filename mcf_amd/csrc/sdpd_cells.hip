@@ -262,7 +262,13 @@ __global__ void k_copy_back(DevParams P, DeviceState S, const int32_t* __restric
     if (S.x_ref) S.x_ref[(int64_t)d * n + i] = xv;
     S.v[(int64_t)d * n + i] = S.v_alt[(int64_t)d * n + i];
   }
-  if (!P.mixed)
+  if (P.mixed) {
+    const RepGeom& g = S.geo[S.rep_alt[i]];
+    S.xq[i] = make_uint4(fixed_position(g, 0, S.x_alt[i]),
+                         fixed_position(g, 1, S.x_alt[(int64_t)n + i]),
+                         P.dim == 3 ? fixed_position(g, 2, S.x_alt[2 * (int64_t)n + i]) : 0u,
+                         (uint32_t)S.pid_alt[i]);
+  } else
     reinterpret_cast<double2*>(S.rec64)[i] = make_double2(S.x_alt[i], S.x_alt[(int64_t)n + i]);
   S.m[i] = S.m_alt[i];
   S.pid[i] = S.pid_alt[i];

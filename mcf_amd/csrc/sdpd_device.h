@@ -67,6 +67,13 @@ struct DevParams {
   // FP32 copies of the constants (mixed precision)
   float inv_hf, coeff, coef_gradf;
   float etaf, eta_coeff, ktf, inv_sqrt_dtf, sqrt_2kt_etaf;
+  // mixed precision with Verlet lists: the Hu-Adams records carry n's factors
+  // times rec_scale (a power of two next to the kernel gradient's factor, so
+  // that FP32 terms keep the magnitude of the forces), and their sums take
+  // sum_scale in FP64; thermal amplitude in that unit.  rec_scale = 1 for the
+  // other laws.
+  double rec_scale, sum_scale;
+  float knoisef;
   // colloids: boundary particles carry sid 1..ncoll (0: fluid only); the
   // reference's coll_noslip, coll_rho_type, coll_translate, coll_rotate,
   // integrate_colloid_AB, coll_sub_time_step, coll_body_force(_type)
@@ -144,7 +151,36 @@ struct RepGeom {
   double cs[3];           // cell edges
   float csf[3];
   float pad2;
+  // mixed precision with Verlet lists: fixed-point positions, unit =
+  // window / 2^32 per dimension, windows = L / fxs L an integer fraction of
+  // the box (fixed_position); fhi + flo = the unit
+  double fxs[3];
+  float fhi[3], flo[3];
 };
+
+// Fixed-point windows of one box: an integer fraction of each edge, at least
+// four cut-offs wide (or the edge itself), so that a pair's difference modulo
+// the window is its nearest image's.
+inline void set_fixed_point(RepGeom& g, int dim, double cut_off) {
+  for (int d = 0; d < 3; ++d) {
+    double k = 1.0;
+    if (d < dim && g.L[d] >= 8.0 * cut_off) k = (double)(int64_t)(g.L[d] / (4.0 * cut_off));
+    g.fxs[d] = k / g.L[d];
+    const double unit = g.L[d] / k / 4294967296.0;
+    g.fhi[d] = (float)unit;
+    g.flo[d] = (float)(unit - (double)g.fhi[d]);
+  }
+}
+
+// A position in units of 2^-32 windows, modulo the window.  The difference of
+// two, as a signed 32-bit number, needs no image and no cell: its error is two
+// units (6e-9 cut-offs at most), where FP32 positions relative to a cell's
+// corner have 6e-8.
+__device__ __forceinline__ uint32_t fixed_position(const RepGeom& g, int d, double x) {
+  double t = (x - g.lo[d]) * g.fxs[d];
+  t = t - floor(t);
+  return (uint32_t)fmin(t * 4294967296.0, 4294967295.0);
+}
 
 // cell index along one dimension: PPM's FLOOR((x - x0) * rdx) with its
 // upper-face corrections (ppm_util_rank3d.F90:433-459), clamped
@@ -250,6 +286,23 @@ __device__ __forceinline__ void kernel_w_gradw_f32(int kernel_type, float s, flo
   }
 }
 
+// The FP32 kernel and its gradient without their factors, coef and 5 (Lucy:
+// 12) coef_grad, at s = r / h.
+__device__ __forceinline__ float kernel_w_f32(int kernel_type, float s) {
+  const float t1 = fmaxf(1.0f - s, 0.0f);
+  if (kernel_type != 1) return (1.0f + 3.0f * s) * (t1 * t1 * t1);
+  const float t2 = fmaxf(2.0f - s, 0.0f), t3 = fmaxf(3.0f - s, 0.0f);
+  const float q1 = (t1 * t1) * (t1 * t1), q2 = (t2 * t2) * (t2 * t2), q3 = (t3 * t3) * (t3 * t3);
+  return q3 * t3 - 6.0f * (q2 * t2) + 15.0f * (q1 * t1);
+}
+__device__ __forceinline__ float kernel_g_f32(int kernel_type, float s) {
+  const float t1 = fmaxf(1.0f - s, 0.0f);
+  if (kernel_type != 1) return s * (t1 * t1);
+  const float t2 = fmaxf(2.0f - s, 0.0f), t3 = fmaxf(3.0f - s, 0.0f);
+  const float q1 = (t1 * t1) * (t1 * t1), q2 = (t2 * t2) * (t2 * t2), q3 = (t3 * t3) * (t3 * t3);
+  return fmaxf(q3 - 6.0f * q2 + 15.0f * q1, 0.0f);
+}
+
 // 1/sqrt(x) for normal x > 0: the hardware estimate (relative error below
 // 2^-24 on gfx950) refined by one Newton step y <- y + y (1/2 - x y^2 / 2),
 // which squares the error: relative error below 2^-46.
@@ -257,6 +310,15 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-(0.5 * x) * y, y, 0.5);
   return fma(y, e, y);
+}
+
+// sqrt(x) in FP32 with one correction step: the hardware's estimate alone is
+// off by up to an ulp and 1/4 ulp on average, which shows in a sum of many
+// kernel values (the density came out 4e-8 high; with it the mean is off by 1e-9).
+__device__ __forceinline__ float sqrt_refined(float x) {
+  const float y = __builtin_amdgcn_rsqf(fmaxf(x, 1.2e-38f));
+  const float r = x * y;
+  return fmaf(fmaf(-r, r, x), 0.5f * y, r);
 }
 
 // sqrt(x) for x >= 0 with a clamp in place of sqrt_nr's selects (x below

@@ -33,9 +33,16 @@ struct DeviceState {
   // (zz, xy), (xz, yz) (2D: zz and the last plane 0)
   double *rec64;
   double *pt64;
-  float4 *vr;            // velocity, w = 1 / n^2; Oldroyd-B: w = pid bits
-  float4 *qr;            // (cell-relative x, p / n^2 or p); Oldroyd-B: (1/n^2, Pxx, Pyy, Pzz)
-  float4 *qr2;           // Oldroyd-B: (Pxy, Pxz, Pyz, 0), P = Pi / n^2
+  // FP32 records, lists rebuilt every step: velocity with w = 1 / n^2
+  // (Oldroyd-B: pid bits); (cell-relative x, p / n^2 or p), Oldroyd-B
+  // (1/n^2, Pxx, Pyy, Pzz); Oldroyd-B (Pxy, Pxz, Pyz, 0), P = Pi / n^2.
+  // Verlet lists: xq = fixed-point position and pid, vr = (v, 1/n^2), an32 =
+  // p / n^2 or p; Oldroyd-B qr = (Pxx, Pyy, Pzz, Pxy), qr2 = float2 (Pxz, Pyz)
+  float4 *vr;
+  float4 *qr;
+  float4 *qr2;
+  uint4 *xq;
+  float *an32;
   // reductions and counters
   double *partials;      // stats partial sums (blocks x 8)
   double *stats_out;     // 8 doubles

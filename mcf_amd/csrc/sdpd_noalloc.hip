@@ -110,6 +110,8 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   if (P.mixed) {
     S.vr = c.take<float4>(N);
     S.qr = c.take<float4>(N);
+    S.xq = c.take<uint4>(N);
+    S.an32 = c.take<float>(N);
   } else {
     S.rec64 = c.take<double>(8 * N);
   }
@@ -207,6 +209,7 @@ extern "C" int sdpd_evaluate_noalloc(const sdpd_params* params, int64_t step, co
     g.csf[d] = (float)P.cs[d];
     if (d < P.dim) mmax = std::max(mmax, P.length[d] + 5.0 * P.cs[d]);
   }
+  sdpd::set_fixed_point(g, P.dim, P.cut_off);
   P.nrep = 1;
   P.nrows = P.nm[1] * P.nm[2];
   // the lists a context builds for this box: Verlet candidates within the

@@ -103,6 +103,7 @@ struct Geo {
   double csd0;          // FP64 cell edge along x
   double half2;         // squared half of the shortest edge, a rounding margin less
   float cs0, cs1, cs2;  // FP32 cell edges
+  float u0h, u1h, u2h, u0l, u1l, u2l;  // units of the fixed-point positions
 };
 
 // Lees-Edwards view of a lane (P.le_g >= 0).  Rows across the upper face
@@ -264,6 +265,23 @@ __device__ __forceinline__ float mixed_s2(float d0, float d1, float d2) {
   return fmaf(d2, d2, fmaf(d1, d1, d0 * d0));
 }
 
+// FP32 separation of fixed-point positions: the integer difference is the
+// nearest image's, and the two-part unit keeps its scale exact to 2^-48 (a
+// rounded scale would shift every distance, and the pressure with them).
+template <int DIM>
+__device__ __forceinline__ void fixed_diff(const Home& h, const uint4& a, const uint4& b, float& d0,
+                                           float& d1, float& d2) {
+  const float c0 = (float)(int32_t)(a.x - b.x), c1 = (float)(int32_t)(a.y - b.y);
+  d0 = fmaf(c0, h.G.u0h, c0 * h.G.u0l);
+  d1 = fmaf(c1, h.G.u1h, c1 * h.G.u1l);
+  if (DIM == 3) {
+    const float c2 = (float)(int32_t)(a.z - b.z);
+    d2 = fmaf(c2, h.G.u2h, c2 * h.G.u2l);
+  } else {
+    d2 = 0.f;
+  }
+}
+
 // FP32 separation from cell-relative positions and the stencil offsets.
 template <int DIM>
 __device__ __forceinline__ void rel_diff(const DevParams& P, const Home& h, const float4& q,
@@ -328,6 +346,12 @@ __device__ __forceinline__ bool load_chunk(const DevParams& P, const DeviceState
   ch.G.csd0 = g.cs[0];
   const double lmin = fmin(fmin(g.L[0], g.L[1]), P.dim == 3 ? g.L[2] : g.L[1]);
   ch.G.half2 = 0.25 * lmin * lmin * (1.0 - 1e-13);
+  ch.G.u0h = g.fhi[0];
+  ch.G.u1h = g.fhi[1];
+  ch.G.u2h = g.fhi[2];
+  ch.G.u0l = g.flo[0];
+  ch.G.u1l = g.flo[1];
+  ch.G.u2l = g.flo[2];
   ch.G.cs0 = g.csf[0];
   ch.G.cs1 = g.csf[1];
   ch.G.cs2 = g.csf[2];
@@ -886,68 +910,105 @@ __device__ __forceinline__ bool mixed_inside(const DevParams& P, const DeviceSta
                            e2) < P.cut2;
 }
 
-// Per-step lists sum compensated in FP32, Verlet lists in FP64.
-template <int DIM, bool DECIDE = false>
-struct DensityMixed {
+// Per-step lists: FP32 cell-relative positions, compensated FP32 sums.
+template <int DIM>
+struct DensityMixedStep {
   const DevParams& P;
   const DeviceState& S;
   const Home& h;
-  std::conditional_t<DECIDE, WideF, KahanF> acc;
+  KahanF acc;
   int nin = 0, rechecks = 0;
   static constexpr bool kImages = false;
   // in batches of eight (the 128^3 Tait box in mixed precision: 0.59 ms in
   // fours, 0.51 in eights, 0.55 in sixteens)
   static constexpr bool kBatched = true;
   static constexpr int kBatch = 8;
-  static constexpr int kTerms = 1;
-  static constexpr int kWalk = 4;
-  struct Rec {
-    float4 q;
-    float mj;
-  };
-  __device__ __forceinline__ Rec gather(uint32_t ent) const {
-    const int j = (int)(ent & kIndexMask);
-    return {load_xyz(S.xa + j), P.density_type == 1 ? (float)S.m[j] : 1.f};
-  }
   template <int NB>
-  __device__ __forceinline__ void terms_f(const uint32_t (&e)[NB], const bool (&ok)[NB],
-                                          Rec (&rec)[NB], float (&t)[NB]) {
+  __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
+    float4 q[NB];
+    float mj[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int j = (int)(e[k] & kIndexMask);
+      q[k] = load_xyz(S.xa + j);
+      mj[k] = P.density_type == 1 ? (float)S.m[j] : 1.f;
+    }
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
       // the lane's own particle in a padding slot: code 62 is offset 0
       const Offsets o = decode_code(ok[k] ? e[k] >> kCodeShift : 62u);
       float d0, d1, d2;
-      rel_diff<DIM>(P, h, rec[k].q, o, d0, d1, d2);
-      const float s2 = mixed_s2(d0, d1, d2);
-      bool use = ok[k];
-      if (DECIDE && use) {
-        use = mixed_inside<DIM>(P, S, h, (int)(e[k] & kIndexMask), s2, rechecks);
-        nin += use ? 1 : 0;
-      }
-      const float r = __builtin_amdgcn_sqrtf(s2);
+      rel_diff<DIM>(P, h, q[k], o, d0, d1, d2);
+      const float r = __builtin_amdgcn_sqrtf(mixed_s2(d0, d1, d2));
       float w, gw;
       kernel_w_gradw_f32(P.kernel_type, r * P.inv_hf, P.coeff, P.coef_gradf, w, gw);
-      t[k] = use ? (P.density_type == 1 ? rec[k].mj * w : w) : 0.f;
+      if (ok[k]) acc.add(P.density_type == 1 ? mj[k] * w : w);
     }
+  }
+};
+
+// Verlet lists: fixed-point positions, FP32 terms (without the kernel's factor
+// coef) summed in FP64.  A candidate's in / out decision comes from its FP32
+// distance, and in a band around the cut-off from the reference's FP64
+// formula.
+template <int DIM>
+struct DensityMixed {
+  const DevParams& P;
+  const DeviceState& S;
+  const Home& h;
+  double acc;
+  int nin = 0, rechecks = 0;
+  static constexpr bool kImages = false;
+  static constexpr bool kBatched = true;
+  static constexpr int kBatch = 8;
+  static constexpr int kTerms = 1;
+  static constexpr int kWalk = 4;
+  struct Rec {
+    uint4 q;
+    float mj;
+  };
+  __device__ __forceinline__ Rec gather(uint32_t ent) const {
+    const uint32_t j = ent & kIndexMask;
+    return {load_at(S.xq, j), P.density_type == 1 ? (float)S.m[j] : 1.f};
   }
   template <int NB>
   __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
                                         Rec (&rec)[NB], double (&t)[NB][kTerms]) {
-    float f[NB];
-    terms_f(e, ok, rec, f);
+    const uint4 own = S.xq[h.ii];
+    float s2[NB];
+    bool use[NB];
+    uint64_t band = 0;
 #pragma unroll
-    for (int k = 0; k < NB; ++k) t[k][0] = (double)f[k];
+    for (int k = 0; k < NB; ++k) {
+      float d0, d1, d2;
+      fixed_diff<DIM>(h, own, rec[k].q, d0, d1, d2);
+      s2[k] = mixed_s2(d0, d1, d2);
+      use[k] = ok[k] && s2[k] < P.cut2_lo_f32;
+      band |= __ballot(s2[k] < P.cut2_hi_f32) & ~__ballot(s2[k] < P.cut2_lo_f32);
+    }
+    if (__builtin_expect(band != 0, 0)) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (ok[k])
+          use[k] = mixed_inside<DIM>(P, S, h, (int)(e[k] & kIndexMask), s2[k], rechecks);
+    }
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      nin += use[k] ? 1 : 0;
+      float w = kernel_w_f32(P.kernel_type, sqrt_refined(s2[k]) * P.inv_hf);
+      if (P.density_type == 1) w = rec[k].mj * w;
+      t[k][0] = (double)(use[k] ? w : 0.f);
+    }
   }
   template <int NB>
   __device__ __forceinline__ void body_batch(const uint32_t (&e)[NB], const bool (&ok)[NB]) {
-    float t[NB];
+    double t[NB][kTerms];
     Rec rec[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) rec[k] = gather(e[k]);
-    terms_f(e, ok, rec, t);
+    terms(e, ok, rec, t);
 #pragma unroll
-    for (int k = 0; k < NB; ++k)
-      if (DECIDE || ok[k]) acc.add(t[k]);
+    for (int k = 0; k < NB; ++k) acc = acc + t[k][0];
   }
 };
 
@@ -961,6 +1022,9 @@ struct DensityMixed {
 //   FP32 Newtonian: (cell-relative x, y, z, p/n^2 for Hu-Adams or p for the
 //   angular form) and (vx, vy, vz, 1/n^2); the pair body gathers these two
 //   and the particle id.
+//   (Both FP32 forms: lists rebuilt every step.  Verlet lists: (v, 1/n^2),
+//   p/n^2 or p apart, and for Oldroyd-B (Pxx, Pyy, Pzz, Pxy) and (Pxz, Pyz),
+//   all but p with P.rec_scale; the position and pid are in xq.)
 //   FP32 Oldroyd-B: (v, pid), (1/n^2, Pxx, Pyy, Pzz) and (Pxy, Pxz, Pyz, 0)
 //   with P = Pi / n^2, Pi = (p + G) I - G c (particles_compute_pressure_
 //   tensor.F90:114-133; c is symmetric); the position comes from xa.
@@ -970,7 +1034,19 @@ __device__ __forceinline__ void write_force_records(const DevParams& P, const De
   const int64_t n = P.n;
   if (P.mixed) {
     const float v0 = (float)S.v[i], v1 = (float)S.v[n + i], v2 = DIM == 3 ? (float)S.v[2 * n + i] : 0.f;
-    if (P.newtonian) {
+    if (P.verlet) {
+      S.vr[i] = make_float4(v0, v1, v2, (float)(bn * P.rec_scale));
+      S.an32[i] = (float)(P.force_type == 4 ? press : an * P.rec_scale);
+      if (!P.newtonian) {
+        const double b = bn * P.rec_scale;
+        auto pi = [&](int a, int c) {
+          return (float)(((a == c ? press + P.G : 0.0) - P.G * S.ct[(int64_t)(a + DIM * c) * n + i]) * b);
+        };
+        S.qr[i] = make_float4(pi(0, 0), pi(1, 1), DIM == 3 ? pi(DIM - 1, DIM - 1) : 0.f, pi(0, 1));
+        reinterpret_cast<float2*>(S.qr2)[i] =
+            DIM == 3 ? make_float2(pi(0, DIM - 1), pi(1, DIM - 1)) : make_float2(0.f, 0.f);
+      }
+    } else if (P.newtonian) {
       const float4 xa = S.xa[i];
       S.qr[i] = make_float4(xa.x, xa.y, xa.z, (float)(P.force_type == 4 ? press : an));
       S.vr[i] = make_float4(v0, v1, v2, (float)bn);
@@ -1248,13 +1324,13 @@ __device__ __forceinline__ void finish_density(const DevParams& P, const DeviceS
 // (particles_compute_density.F90:369-558).
 template <bool MIXED>
 __device__ __forceinline__ double self_density(const DevParams& P, double mi) {
-  if (MIXED) return (double)(float)(P.density_type == 1 ? P.w0 * mi : P.w0);
-  // (FP64 sums leave the kernel's factor cw to density_of)
-  return P.density_type == 1 ? P.w0q * mi : P.w0q;
+  // (the sums leave the kernel's factor to density_of)
+  const double w = MIXED ? P.w0 / P.coef : P.w0q;
+  return P.density_type == 1 ? w * mi : w;
 }
 template <bool MIXED>
 __device__ __forceinline__ double density_of(const DevParams& P, double sum) {
-  return MIXED ? sum : P.cw * sum;
+  return (MIXED ? P.coef : P.cw) * sum;
 }
 
 // One chunk slot of a density pass that scans the stencil.
@@ -1270,20 +1346,22 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
   const Home h = load_home<DIM>(P, S, ch);
   const double mi = S.m[h.ii];
   uint32_t* list = (MODE == kStore || MODE == kBuild) ? S.nlist : nullptr;
-  using Pol = std::conditional_t<MIXED, DensityMixed<DIM, kDecide>, DensityF64<DIM, kDecide>>;
+  using Pol = std::conditional_t<
+      MIXED, std::conditional_t<kDecide, DensityMixed<DIM>, DensityMixedStep<DIM>>,
+      DensityF64<DIM, kDecide>>;
   Pol pol{P, S, h, {}};
-  if constexpr (MIXED)
-    pol.acc.add((float)self_density<true>(P, mi));
+  if constexpr (MIXED && !kDecide)
+    pol.acc.add((float)(P.density_type == 1 ? P.w0 * mi : P.w0));
   else
-    pol.acc = self_density<false>(P, mi);
+    pol.acc = self_density<MIXED>(P, mi);
   int rechecks = 0;
   const int cnt =
       staged_scan<DIM, Pol, TILE, BUF, kDecide>(P, S, ch, h, pol, tile, buf, rechecks, list);
   double rho;
-  if constexpr (MIXED)
+  if constexpr (MIXED && !kDecide)
     rho = pol.acc.value();
   else
-    rho = density_of<false>(P, pol.acc);
+    rho = density_of<MIXED>(P, pol.acc);
   if (!h.active) return;
   const int i = h.i;
   if (MODE == kStore || MODE == kBuild) S.nbr_count[i] = cnt;
@@ -1296,8 +1374,9 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
 
 // The walk of the step's Verlet lists: NQ quarters of a chunk per workgroup.
 // Quarters one after the other let the epilogue (equation of state, force
-// records) run once on 64 lanes; a small box takes one quarter per workgroup
-// to fill the GPU.  QUINTIC: the quintic spline and the number density as
+// records) run once on 64 lanes (128^3 box: FP64 0.58 ms, 0.65 with one
+// quarter per workgroup; mixed 0.46 and 0.49); a small box takes one quarter
+// per workgroup to fill the GPU.  QUINTIC: the quintic spline and the number density as
 // constants, so the batch's terms carry no branches.
 template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ>
 __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState S) {
@@ -1321,7 +1400,7 @@ __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState
 #pragma unroll 1
   for (int q = 0; q < NQ && ch.p0 + kQuarter * (q0 + q) < ch.p1; ++q) {
     const Home h = load_quarter_home<DIM>(P, S, ch, q0 + q);
-    using Pol = std::conditional_t<MIXED, DensityMixed<DIM, true>, DensityF64<DIM, true>>;
+    using Pol = std::conditional_t<MIXED, DensityMixed<DIM>, DensityF64<DIM, true>>;
     Pol pol{P, S, h, {}};
     walk_quarter<DIM>(P, S, ch, q0 + q, h, pol,
                       self_density<MIXED>(P, QUINTIC ? 1.0 : S.m[h.ii]), lds);
@@ -1818,46 +1897,71 @@ struct ForceMixed {
   // Oldroyd-B: own Pi / n^2 (xx, yy, zz, xy, xz, yz), 1 / n
   float pb[6];
   float inv_ni;
+  uint4 own;               // Verlet lists: own fixed-point position
   // the acceleration's components, then the velocity gradient's: with
   // Verlet lists FP64 sums of the FP32 terms; per-step lists sum the
   // acceleration compensated in FP32
   static constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
   std::conditional_t<DECIDE, WideF, KahanF> facc[DIM];
   WideF gacc[DIM * DIM];
+  // the terms leave out the kernel gradient's factor but for the power of two
+  // in the records, and the velocity gradient's 1 / n_i (finish_pairs)
+  static constexpr bool kUnit = DECIDE && (FT == 3 || FT == 5);
   static constexpr bool kImages = false;
   // Verlet lists: the records of a lane's kWalk entries are gathered before
   // the first pair is evaluated
   static constexpr bool kBatched = DECIDE;
   static constexpr int kBatch = 2;
-  static constexpr int kWalk = FT >= 5 ? 2 : 4;
+  static constexpr int kWalk = 2;
   __device__ __forceinline__ double sum(int c) const {
     return c < DIM ? facc[c < DIM ? c : 0].value() : gacc[c < DIM ? 0 : c - DIM].value();
   }
-  // j's records: FP32 position (w: p/n^2 or p, Newtonian), velocity (w:
-  // 1/n^2, or the pid bits for Oldroyd-B), pid, and the Oldroyd-B
-  // (1/n^2, Pxx, Pyy, Pzz) and (Pxy, Pxz, Pyz, 0)
+  // j's velocity and 1/n^2, p/n^2 (p for the angular form), pid, Oldroyd-B
+  // Pi / n^2 (xx, yy, zz, xy, xz, yz), and the position: fixed-point (Verlet
+  // lists) or cell-relative
   struct Rec {
-    float4 x, v, q, q2;
-    uint32_t pid;
+    uint4 x;
+    float4 v;
+    float an;
+    float4 q;
+    float2 q2;
   };
-  __device__ __forceinline__ Rec load_rec(int j) const {
+  __device__ __forceinline__ Rec load_rec(uint32_t j) const {
     Rec r;
-    if (FT >= 5) {
-      r.v = S.vr[j];
-      r.x = load_xyz(S.xa + j);
-      r.q = S.qr[j];
-      r.q2 = S.qr2[j];
-      r.pid = __float_as_uint(r.v.w);
-    } else {
-      r.x = S.qr[j];
-      r.v = S.vr[j];
-      r.q = r.q2 = make_float4(0.f, 0.f, 0.f, 0.f);
-      r.pid = P.noise ? (uint32_t)S.pid[j] : 0u;
+    r.an = 0.f;
+    r.q = make_float4(0.f, 0.f, 0.f, 0.f);
+    r.q2 = make_float2(0.f, 0.f);
+    if (DECIDE) {
+      r.x = load_at(S.xq, j);
+      r.v = load_at(S.vr, j);
+      if (FT < 5) r.an = load_at(S.an32, j);
+      if (FT >= 5) {
+        r.q = load_at(S.qr, j);
+        r.q2 = load_at(reinterpret_cast<const float2*>(S.qr2), j);
+      }
+      return r;
     }
+    r.v = S.vr[j];
+    float4 x;
+    if (FT >= 5) {
+      x = load_xyz(S.xa + j);
+      const float4 q = S.qr[j], q2 = S.qr2[j];
+      r.x.w = __float_as_uint(r.v.w);
+      r.v.w = q.x;
+      r.q = make_float4(q.y, q.z, q.w, q2.x);
+      r.q2 = make_float2(q2.y, q2.z);
+    } else {
+      x = S.qr[j];
+      r.an = x.w;
+      r.x.w = P.noise ? (uint32_t)S.pid[j] : 0u;
+    }
+    r.x.x = __float_as_uint(x.x);
+    r.x.y = __float_as_uint(x.y);
+    r.x.z = __float_as_uint(x.z);
     return r;
   }
   __device__ __forceinline__ Rec gather(uint32_t ent) const {
-    return load_rec((int)(ent & kIndexMask));
+    return load_rec(ent & kIndexMask);
   }
   __device__ __forceinline__ void add(const float (&t)[kTerms]) {
 #pragma unroll
@@ -1869,19 +1973,38 @@ struct ForceMixed {
     }
   }
   __device__ __forceinline__ void body(uint32_t ent) {
-    const int j = (int)(ent & kIndexMask);
+    const uint32_t j = ent & kIndexMask;
     const Rec r = load_rec(j);
-    float t[kTerms];
-    eval(j, r.x, r.v, r.pid, r.q, r.q2, decode_code(ent >> kCodeShift), true, t);
+    const Offsets o = decode_code(ent >> kCodeShift);
+    float d0, d1, d2, t[kTerms];
+    rel_diff<DIM>(P, h,
+                  make_float4(__uint_as_float(r.x.x), __uint_as_float(r.x.y),
+                              __uint_as_float(r.x.z), 0.f),
+                  o, d0, d1, d2);
+    eval((int)j, r, d0, d1, d2, mixed_s2(d0, d1, d2), le_dvf(P, h, o), t);
     add(t);
   }
+  // (Verlet candidates take no in / out decision: outside the cut-off the
+  // kernel gradient is 0.  An empty slot holds the lane's own particle, moved
+  // outside.)
   template <int NB>
   __device__ __forceinline__ void terms_f(const uint32_t (&e)[NB], const bool (&ok)[NB],
                                           Rec (&r)[NB], float (&t)[NB][kTerms]) const {
+    float d[NB][3], r2[NB];
+    uint64_t empty = 0;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      fixed_diff<DIM>(h, own, r[k].x, d[k][0], d[k][1], d[k][2]);
+      r2[k] = mixed_s2(d[k][0], d[k][1], d[k][2]);
+      empty |= __ballot(!ok[k]);
+    }
+    if (__builtin_expect(empty != 0, 0)) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) r2[k] = ok[k] ? r2[k] : 4.f * P.cut2_hi_f32;
+    }
 #pragma unroll
     for (int k = 0; k < NB; ++k)
-      eval((int)(e[k] & kIndexMask), r[k].x, r[k].v, r[k].pid, r[k].q, r[k].q2,
-           decode_code(ok[k] ? e[k] >> kCodeShift : 62u), ok[k], t[k]);
+      eval((int)(e[k] & kIndexMask), r[k], d[k][0], d[k][1], d[k][2], r2[k], 0.f, t[k]);
   }
   template <int NB>
   __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
@@ -1903,33 +2026,23 @@ struct ForceMixed {
 #pragma unroll
     for (int k = 0; k < NB; ++k) add(t[k]);
   }
-  // xj: cell-relative position (w: p/n^2 for Hu-Adams, p for the angular
-  // form); vj: velocity (w: 1/n^2, Newtonian); Oldroyd-B qj: (1/n^2, Pxx,
-  // Pyy, Pzz), q2: (Pxy, Pxz, Pyz, 0)
-  __device__ __forceinline__ void eval(int jidx, const float4& xj, const float4& vj,
-                                       uint32_t pidj, const float4& qj, const float4& q2,
-                                       const Offsets& o, bool ok, float (&t)[kTerms]) const {
-    float d0, d1, d2;
-    rel_diff<DIM>(P, h, xj, o, d0, d1, d2);
-    float r2 = mixed_s2(d0, d1, d2);
-    // Verlet candidates: the pair is evaluated either way (outside the
-    // cut-off the kernel gradient is 0) and only added when inside.  The
-    // record's w is pinned to a register ahead of the decision (an empty
-    // asm), so the record arrives in one 16-byte gather with the position
-    // instead of a second 4-byte one after the decision's branch.
-    bool use = true;
-    float xjw = xj.w;
-    if (DECIDE) {
-      asm volatile("" : "+v"(xjw));
-      int rechecks = 0;
-      use = ok && mixed_inside<DIM>(P, S, h, jidx, r2, rechecks);
-      if (!ok) r2 = P.cut2_hi_f32;  // an empty slot (the lane's own particle)
-    }
+  // The terms of one pair: j's record, the separation and its square, the x
+  // velocity of j's image on top of j's own.
+  __device__ __forceinline__ void eval(int jidx, const Rec& rj, float d0, float d1, float d2,
+                                       float r2, float jump, float (&t)[kTerms]) const {
+    const float4& vj = rj.v;
+    const float xjw = rj.an, bj = rj.v.w;
+    const uint32_t pidj = rj.x.w;
     const float ir = __builtin_amdgcn_rsqf(r2);
     const float r = r2 * ir;
-    float w, gw;
-    kernel_w_gradw_f32(P.kernel_type, r * P.inv_hf, P.coeff, P.coef_gradf, w, gw);
-    const float u0 = vi0 - (vj.x + le_dvf(P, h, o)), u1 = vi1 - vj.y, u2 = vi2 - vj.z;
+    float gw;
+    if (kUnit) {
+      gw = kernel_g_f32(P.kernel_type, r * P.inv_hf);
+    } else {
+      float w;
+      kernel_w_gradw_f32(P.kernel_type, r * P.inv_hf, P.coeff, P.coef_gradf, w, gw);
+    }
+    const float u0 = vi0 - (DECIDE ? vj.x : vj.x + jump), u1 = vi1 - vj.y, u2 = vi2 - vj.z;
     float fi0, fi1, fi2;
     if (FT >= 5) {
       // rhs_force_ff_non_Newtonian_HuAdams.F90:105-131 with the records'
@@ -1937,14 +2050,14 @@ struct ForceMixed {
       // Espanol: its thermal force below; FT 7, angular: the diagonal
       // averaged, (Pi_i + Pi_j) / 2 (1/n_i^2 + 1/n_j^2), and dissipation
       // along e)
-      float sxx = pb[0] + qj.y, syy = pb[1] + qj.z, szz = pb[2] + qj.w;
+      float sxx = pb[0] + rj.q.x, syy = pb[1] + rj.q.y, szz = pb[2] + rj.q.z;
       if (FT == 7) {
-        const float bsum = bi + qj.x;
-        sxx = 0.5f * (pb[0] / bi + qj.y / qj.x) * bsum;
-        syy = 0.5f * (pb[1] / bi + qj.z / qj.x) * bsum;
-        szz = 0.5f * (pb[2] / bi + qj.w / qj.x) * bsum;
+        const float bsum = bi + bj;
+        sxx = 0.5f * (pb[0] / bi + rj.q.x / bj) * bsum;
+        syy = 0.5f * (pb[1] / bi + rj.q.y / bj) * bsum;
+        szz = 0.5f * (pb[2] / bi + rj.q.z / bj) * bsum;
       }
-      const float sxy = pb[3] + q2.x, sxz = pb[4] + q2.y, syz = pb[5] + q2.z;
+      const float sxy = pb[3] + rj.q.w, sxz = pb[4] + rj.q2.x, syz = pb[5] + rj.q2.y;
       float c0, c1, c2;
       if (DIM == 3) {
         c0 = sxx * d0 + sxy * d1 + sxz * d2;
@@ -1956,9 +2069,9 @@ struct ForceMixed {
         c2 = 0.f;
       }
       const float gir = gw * ir;
-      const float f_d = P.etaf * (bi + qj.x) * gir;
+      const float f_d = P.etaf * (bi + bj) * gir;
       if (FT == 7) {
-        const float fde = P.eta_coeff * P.etaf * (bi + qj.x) * gw * (d0 * u0 + d1 * u1 + d2 * u2) *
+        const float fde = P.eta_coeff * P.etaf * (bi + bj) * gw * (d0 * u0 + d1 * u1 + d2 * u2) *
                           (ir * ir * ir);
         fi0 = fde * d0 - c0 * gir;
         fi1 = fde * d1 - c1 * gir;
@@ -1968,19 +2081,19 @@ struct ForceMixed {
         fi1 = f_d * u1 - c1 * gir;
         fi2 = f_d * u2 - c2 * gir;
       }
-      const float gfac = gir * inv_ni;
-      const float du[3] = {-u0, -u1, -u2};
+      const float gfac = kUnit ? gir : gir * inv_ni;
+      const float ug[3] = {-u0 * gfac, -u1 * gfac, -u2 * gfac};
       const float dx[3] = {d0, d1, d2};
 #pragma unroll
       for (int b = 0; b < DIM; ++b)
 #pragma unroll
         for (int a = 0; a < DIM; ++a)
-          t[DIM + a + DIM * b] = use ? du[a] * dx[b] * gfac : 0.f;
+          t[DIM + a + DIM * b] = ug[a] * dx[b];
       if (FT == 6 && P.noise) {
         // Espanol's (A S e + B tr e) / sqrt(dt), Z = 4 kT W' / (r n_i n_j)
         float w0, w1, w2, g3;
         noise_vector<DIM, float>(P, step, pidi, pidj, d0 * ir, d1 * ir, d2 * ir, w0, w1, w2, &g3);
-        const float zij = 4.0f * P.ktf * gir * inv_ni * __builtin_amdgcn_sqrtf(qj.x);
+        const float zij = 4.0f * P.ktf * gir * inv_ni * __builtin_amdgcn_sqrtf(bj);
         const float ea = 5.0f * P.etaf / 3.0f, eb = (DIM + 2.0f) * P.etaf / 3.0f;
         const float aij = __builtin_amdgcn_sqrtf(-zij * ea) * P.inv_sqrt_dtf;
         const float bij = __builtin_amdgcn_sqrtf(-zij * DIM / 2.0f * (eb + ea * (2.0f / DIM - 1.0f))) *
@@ -1990,25 +2103,29 @@ struct ForceMixed {
         fi1 = fi1 + aij * w1 + btr * d1;
         fi2 = fi2 + aij * w2 + btr * d2;
       } else if (FT == 5 && P.noise) {
+        if constexpr (kUnit) {
+          unit_noise(pidj, f_d, d0, d1, d2, ir, fi0, fi1, fi2);
+        } else {
         float w0, w1, w2;
         noise_vector<DIM, float>(P, step, pidi, pidj, d0 * ir, d1 * ir, d2 * ir, w0, w1, w2);
         const float f_r = __builtin_amdgcn_sqrtf(-4.0f * P.ktf * f_d) * P.inv_sqrt_dtf;
         fi0 = fi0 + f_r * w0;
         fi1 = fi1 + f_r * w1;
         fi2 = fi2 + f_r * w2;
+        }
       }
     } else if (FT == 1) {
       // rhs_force_ff_Newtonian_Morris.F90:112-136 (accelerations carrying
       // the partner's mass; bi, vj.w = 1/rho)
       const float mj = (float)S.m[jidx];
       const float fcm = mj * (ai + xjw) * gw * ir;
-      const float fdm = mj * 2.0f * P.etaf * gw * bi * vj.w * ir;
+      const float fdm = mj * 2.0f * P.etaf * gw * bi * bj * ir;
       fi0 = fdm * u0 - fcm * d0;
       fi1 = fdm * u1 - fcm * d1;
       fi2 = fdm * u2 - fcm * d2;
     } else if (FT == 2) {
       // rhs_force_ff_Newtonian_Espanol.F90:152-251 (bi, vj.w = 1/n)
-      const float gnn = gw * bi * vj.w * ir;
+      const float gnn = gw * bi * bj * ir;
       const float ev = (d0 * u0 + d1 * u1 + d2 * u2) * ir;
       const float fd1 = (2.0f - 1.0f / DIM) * P.etaf * gnn;
       const float fd2 = P.etaf * (DIM + 2.0f) / DIM * gnn * ev;
@@ -2031,23 +2148,27 @@ struct ForceMixed {
         fi2 = fi2 + aij * w2 + btr * d2;
       }
     } else if (FT == 3) {
-      const float fcr = (ai + xjw) * gw * ir;
-      const float f_d = P.etaf * (bi + vj.w) * gw * ir;
+      const float fcr = kUnit ? (ai + xjw) * (gw * ir) : (ai + xjw) * gw * ir;
+      const float f_d = kUnit ? fmaf(P.etaf, bj, P.etaf * bi) * (gw * ir) : P.etaf * (bi + bj) * gw * ir;
       fi0 = f_d * u0 - fcr * d0;
       fi1 = f_d * u1 - fcr * d1;
       fi2 = f_d * u2 - fcr * d2;
       if (P.noise) {
+        if constexpr (kUnit) {
+          unit_noise(pidj, f_d, d0, d1, d2, ir, fi0, fi1, fi2);
+        } else {
         float w0, w1, w2;
         noise_vector<DIM, float>(P, step, pidi, pidj, d0 * ir, d1 * ir, d2 * ir, w0, w1, w2);
         const float f_r = __builtin_amdgcn_sqrtf(-4.0f * P.ktf * f_d) * P.inv_sqrt_dtf;
         fi0 = fi0 + f_r * w0;
         fi1 = fi1 + f_r * w1;
         fi2 = fi2 + f_r * w2;
+        }
       }
     } else {
       const float ev = (d0 * u0 + d1 * u1 + d2 * u2) * ir;
       const float pij = (pi + xjw) * 0.5f;
-      const float aij = (bi + vj.w) * gw;
+      const float aij = (bi + bj) * gw;
       const float f_c = aij * pij;
       const float f_d = P.eta_coeff * P.etaf * aij * ev * ir;
       float sc = f_d - f_c;
@@ -2062,11 +2183,31 @@ struct ForceMixed {
       fi1 = sc * d1;
       fi2 = sc * d2;
     }
-    t[0] = use ? fi0 : 0.f;
-    t[1] = use ? fi1 : 0.f;
-    if (DIM == 3) t[2] = use ? fi2 : 0.f;
+    t[0] = fi0;
+    t[1] = fi1;
+    if (DIM == 3) t[2] = fi2;
+  }
+  // f_r W e of the Hu-Adams forms in units of the kernel gradient's factor
+  // (negative: the unit turns the sign), as ForceF64 writes it on d
+  __device__ __forceinline__ void unit_noise(uint32_t pidj, float f_d, float d0, float d1, float d2,
+                                             float ir, float& f0, float& f1, float& f2) const {
+    float g[4];
+    pair_normals(P.seed, pidi < pidj ? pidi : pidj, pidi < pidj ? pidj : pidi, step, g);
+    const float fr = __builtin_amdgcn_sqrtf(P.knoisef * f_d);
+    const float sfr = pidi < pidj ? -fr : fr;
+    if (DIM == 3) {
+      const float cba = 0.81649658092772603273f * 1.41421356237309504880f - 1.0f;
+      const float k = cba * fmaf(g[2], d2, fmaf(g[1], d1, g[0] * d0)) * (ir * ir);
+      f0 = fmaf(sfr, fmaf(k, d0, g[0]), f0);
+      f1 = fmaf(sfr, fmaf(k, d1, g[1]), f1);
+      f2 = fmaf(sfr, fmaf(k, d2, g[2]), f2);
+    } else {
+      f0 = fmaf(sfr, g[0], f0);
+      f1 = fmaf(sfr, g[1], f1);
+    }
   }
 };
+
 
 template <int DIM>
 __device__ __forceinline__ void finish_force(const DevParams& P, const DeviceState& S, int i,
@@ -2125,13 +2266,23 @@ __device__ __forceinline__ ForceMixed<DIM, FT, DECIDE> mixed_policy(const DevPar
                                                                     const Home& h) {
   const int ii = h.ii;
   const float4 vi = S.vr[ii];
-  const float4 qi = S.qr[ii];
-  // Newtonian records: qi.w = p/n^2 (Hu-Adams) or p (angular), vi.w = 1/n^2
-  ForceMixed<DIM, FT, DECIDE> pol{P, S, h, vi.x, vi.y, vi.z, FT <= 3 ? qi.w : 0.f, vi.w,
-                                  FT == 4 ? qi.w : 0.f,
-                                  FT >= 5 ? __float_as_uint(vi.w) : (uint32_t)S.pid[ii],
-                                  S.step_dev[0]};
-  if (FT >= 5) {
+  const float4 qi = FT >= 5 || !DECIDE ? S.qr[ii] : make_float4(0.f, 0.f, 0.f, 0.f);
+  ForceMixed<DIM, FT, DECIDE> pol{P, S, h, vi.x, vi.y, vi.z, 0.f, vi.w, 0.f,
+                                  (uint32_t)S.pid[ii], S.step_dev[0]};
+  if (FT <= 4) {
+    // p/n^2, or p for the angular form
+    const float an = DECIDE ? S.an32[ii] : qi.w;
+    pol.ai = FT <= 3 ? an : 0.f;
+    pol.pi = FT == 4 ? an : 0.f;
+  } else if (DECIDE) {
+    const float2 q2 = reinterpret_cast<const float2*>(S.qr2)[ii];
+    pol.pb[0] = qi.x;
+    pol.pb[1] = qi.y;
+    pol.pb[2] = qi.z;
+    pol.pb[3] = qi.w;
+    pol.pb[4] = q2.x;
+    pol.pb[5] = q2.y;
+  } else {
     const float4 q2 = S.qr2[ii];
     pol.bi = qi.x;
     pol.pb[0] = qi.y;
@@ -2140,8 +2291,9 @@ __device__ __forceinline__ ForceMixed<DIM, FT, DECIDE> mixed_policy(const DevPar
     pol.pb[3] = q2.x;
     pol.pb[4] = q2.y;
     pol.pb[5] = q2.z;
-    pol.inv_ni = (float)(1.0 / S.rho[ii]);
   }
+  if (FT >= 5) pol.inv_ni = (float)(1.0 / S.rho[ii]);
+  if (DECIDE) pol.own = S.xq[ii];
   return pol;
 }
 
@@ -2185,24 +2337,31 @@ __device__ __forceinline__ ForceF64<DIM, FT, COLL, DECIDE> f64_policy(const DevP
   return pol;
 }
 
-// Acceleration (and conformation rate) of particle i from its pair sums;
-// F64: with the factors the FP64 bodies leave out.
-template <int DIM, int FT, bool F64, bool COLL>
+// Acceleration (and conformation rate) of particle i from its pair sums, with
+// the factors the bodies leave out: UNIT is that of the kernel gradient (0
+// none, 1 FP64, 2 FP32 records), GRAD whether 1 / n_i is left out of the
+// velocity gradient.
+template <int DIM, int FT, int UNIT, bool GRAD>
 __device__ __forceinline__ void finish_pairs(const DevParams& P, const DeviceState& S, int i,
                                              const double* sum, bool fluid) {
-  constexpr bool kUnit = F64 && (FT == 3 || FT == 5);
+  const double unit = UNIT == 1 ? P.cg : (UNIT == 2 ? P.sum_scale : 1.0);
   // the Morris body sums accelerations already
-  const double inv_mi = (kUnit ? P.cg : 1.0) * (FT == 1 ? 1.0 : 1.0 / S.m[i]);
+  const double inv_mi = unit * (FT == 1 ? 1.0 : 1.0 / S.m[i]);
   finish_force<DIM>(P, S, i, sum[0] * inv_mi, sum[1] * inv_mi, DIM == 3 ? sum[DIM - 1] * inv_mi : 0.0,
                     fluid);
   if (FT >= 5) {
-    const double fac = (kUnit ? P.cg : 1.0) * (F64 && !COLL ? 1.0 / S.rho[i] : 1.0);
+    // (the FP32 records' power of two scales the forces, not the gradient)
+    const double fac = (UNIT == 2 ? unit * P.rec_scale : unit) * (GRAD ? 1.0 / S.rho[i] : 1.0);
     double L[DIM * DIM];
 #pragma unroll
     for (int q = 0; q < DIM * DIM; ++q) L[q] = sum[DIM + q] * fac;
     conformation_rate<DIM>(P, S, i, L);
   }
 }
+template <int FT, bool MIXED, bool VERLET>
+constexpr int kPairUnit = (FT == 3 || FT == 5) ? (MIXED ? (VERLET ? 2 : 0) : 1) : 0;
+template <int FT, bool MIXED, bool COLL, bool VERLET>
+constexpr bool kPairGrad = MIXED ? (VERLET && FT == 5) : !COLL;
 
 // One chunk slot of a force pass with one particle per lane.  Two launches
 // over the same grid: SCAN = false takes the chunks whose lists hold every
@@ -2245,7 +2404,9 @@ __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceSta
     for (int c = 0; c < pol.kTerms; ++c) sum[c] = pol.sum[c];
     fluid = !COLL || pol.sidi == 0;
   }
-  if (h.active) finish_pairs<DIM, FT, !MIXED, COLL>(P, S, h.i, sum, fluid);
+  if (h.active)
+    finish_pairs<DIM, FT, kPairUnit<FT, MIXED, VERLET>, kPairGrad<FT, MIXED, COLL, VERLET>>(
+        P, S, h.i, sum, fluid);
 }
 
 // With Verlet lists the rescan (SCAN) has work only if a list overflowed at
@@ -2279,9 +2440,11 @@ enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
 // The FP64 Hu-Adams body is held to 128 registers, four waves per SIMD; left
 // alone the compiler interleaves more of the two pairs' noise and takes 191.
 // Two entries per lane and batch: the 128^3 box takes 1.33 ms with two, 1.47
-// with four (191 registers); it took 1.66 with one particle per lane.
+// with four (191 registers); it took 1.66 with one particle per lane.  The
+// mixed bodies fit six waves (0.87 ms, 1.14 with cell-relative positions, their
+// code decode and compensated FP32 sums, one particle per lane).
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC>
-__global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : 1) void k_force_walk(DevParams P, DeviceState S) {
+__global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? 6 : 1)) void k_force_walk(DevParams P, DeviceState S) {
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (SPEC != kAny) {
@@ -2310,7 +2473,8 @@ __global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : 1) void k
   double sum[kTerms];
 #pragma unroll
   for (int c = 0; c < kTerms; ++c) sum[c] = quarter_sum(lds, threadIdx.x, c);
-  finish_pairs<DIM, FT, !MIXED, COLL>(P, S, i, sum, !COLL || S.sid[i] == 0);
+  finish_pairs<DIM, FT, kPairUnit<FT, MIXED, true>, kPairGrad<FT, MIXED, COLL, true>>(
+      P, S, i, sum, !COLL || S.sid[i] == 0);
 }
 
 // ---------------------------------------------------------------------

@@ -105,22 +105,20 @@ __global__ void k_conformation(DevParams P, DeviceState S, double lambda) {
     S.ct[q * n + i] = S.ct[q * n + i] + S.act[q * n + i] * P.dt * lambda;
 }
 
-// Verlet lists: particle i's displacement since the lists were built and,
-// in mixed precision, its FP32 position relative to the corner of the cell
-// it was sorted into then.  Per dimension the displacement x - x_ref is
-// taken to the nearest period, so a particle that crossed a periodic face
-// keeps its build cell: its FP32 position goes on from there, unwrapped,
-// and stays consistent with the stencil offsets stored in the lists.
-// Returns the squared displacement.
+// Verlet lists: particle i's squared displacement since the lists were built,
+// per dimension taken to the nearest period.  What the walks read of the
+// positions follows here: the (x, y) plane of the FP64 records, or in mixed
+// precision the fixed-point position.
 //
-// FP64 runs without sheared faces keep the FP32 positions of the build:
-// their walks take distances from the FP64 positions, and the only readers
-// of the FP32 ones between builds (the rescans of overflowed lists and the
+// The FP32 positions relative to the build cell are kept as they were at the
+// build (without sheared faces): the walks do not read them, and the only
+// readers between builds (the rescans of overflowed lists and the
 // neighbour-set signature) screen at rc + skin.  Every particle has moved
 // at most skin / 2 since the build, so the build-time positions put every
 // pair that is within rc now inside that screen, and the exact FP64
 // decision follows.  With sheared faces the scan's windows follow the
-// current shear length and FP32 positions, which are kept current.
+// current shear length and FP32 positions, which are kept current: unwrapped
+// from the build cell.
 // A replica's corner and edges in registers.
 struct BoxFrame {
   double lo[3], L[3];
@@ -151,9 +149,12 @@ __device__ __forceinline__ double track_particle(const DevParams& P, const Devic
     const double dd = raw + w[d];
     d2 = d2 + dd * dd;
   }
-  // the (x, y) plane of the FP64 records follows the positions
-  if (!P.mixed) reinterpret_cast<double2*>(S.rec64)[i] = make_double2(xv[0], xv[1]);
-  if (P.mixed || P.le_g >= 0) {
+  if (P.mixed)
+    S.xq[i] = make_uint4(fixed_position(g, 0, xv[0]), fixed_position(g, 1, xv[1]),
+                         DIM == 3 ? fixed_position(g, 2, xv[2]) : 0u, (uint32_t)S.pid[i]);
+  else
+    reinterpret_cast<double2*>(S.rec64)[i] = make_double2(xv[0], xv[1]);
+  if (P.le_g >= 0) {
     const int kl = S.key_sorted[i] - g.cell_base;
     const int cc[3] = {kl % g.nm[0], (kl / g.nm[0]) % g.nm[1], kl / (g.nm[0] * g.nm[1])};
     float a[3] = {0.f, 0.f, 0.f};
