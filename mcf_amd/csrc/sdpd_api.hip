@@ -44,7 +44,7 @@ struct sdpd_ctx {
   std::vector<sdpd::RepGeom> geo;
   std::vector<int32_t> row_cell, row_len, row_rep;
   bool sorted_once = false;
-  // captured two-step graphs of sdpd_step, one per parity of the sort's
+  // captured graphs of sdpd_step's steps, one per parity of the sort's
   // ping-pong buffers (kernel arguments hold the buffer pointers)
   bool use_graphs = true;
   int list_cap_req = 0;      // stored neighbour entries per particle (0: automatic)
@@ -423,7 +423,7 @@ void free_state(DeviceState& S) {
                   S.key_sorted, S.xa,     S.pt64,      S.vr,        S.qr,      S.partials, S.stats_out,
                   S.nbr_count, S.recheck, S.nbr_hash, S.rkey,   S.rslot,    S.rcount,
                   S.rstart,   S.runsorted, S.rlpdx,  S.nlist,   S.nbr_sig_count,
-                  S.row_nchunk, S.row_chunk_off, S.chunk_row, S.scan_tmp, S.rec64,
+                  S.sort_ctl, S.row_chunk_off, S.chunk_row, S.scan_tmp, S.rec64,
                   (void*)S.geo, S.rep,      S.rep_alt,  S.row_cell, S.row_len,  S.row_rep,
                   S.rep_stats, S.qr2,     S.xq,       S.an32,     S.step_dev, S.time_dev, S.sid,
                   S.sid_alt,  S.slot_of,  (void*)S.coll_hot, (void*)S.coll, S.coll_start,
@@ -504,10 +504,10 @@ int alloc_state(sdpd_ctx* c, int n) {
     const size_t nrows = (size_t)P.nrows;
     const size_t nchunk = (N + 63) / 64 + nrows;
     const size_t ntile = ((size_t)std::max(P.ncell, (int32_t)nrows) + 4095) / 4096 + 1;
-    ALLOC(row_nchunk, nrows);
     ALLOC(row_chunk_off, nrows + 1);
     ALLOC(chunk_row, nchunk);
     ALLOC(scan_tmp, std::max(ntile, (size_t)((P.ncell_ref + 4095) / 4096 + 1)));
+    ALLOC(sort_ctl, 8);
   }
   c->stats_nb = sdpd::stats_blocks(n);
   ALLOC(partials, (size_t)c->stats_nb * 4);
@@ -599,18 +599,15 @@ int need_particles(sdpd_ctx* c) {
 // then swap.  Verlet lists: the sorted state is copied back (the buffers
 // stay put), the positions of the sort become the lists' reference, and
 // the next density pass builds the lists.
-int run_sort(sdpd_ctx* c, bool keys_done) {
+int run_sort(sdpd_ctx* c, bool keys_done, bool advance = false) {
   c->P.step = c->step;
   {
     PhaseMark pm(c, 1);
-    if (c->P.verlet) {
-      sdpd::launch_cell_keys(c->stream, c->P, c->S);
-      sdpd::launch_cell_sort_after_keys(c->stream, c->P, c->S, nullptr, true);
-      sdpd::launch_force_build(c->stream, c->S);
-    } else {
-      if (!keys_done) sdpd::launch_cell_keys(c->stream, c->P, c->S);
-      sdpd::launch_cell_sort_after_keys(c->stream, c->P, c->S);
-    }
+    sdpd::launch_sort(c->stream, c->P, c->S,
+                      c->P.verlet ? sdpd::SortKind::kVerletForced
+                                  : (keys_done ? sdpd::SortKind::kStepKeysDone
+                                               : sdpd::SortKind::kStep),
+                      advance);
   }
   int rc = check_launch(c, "cell sort");
   if (rc) return rc;
@@ -623,16 +620,14 @@ int run_sort(sdpd_ctx* c, bool keys_done) {
 }
 
 // Verlet lists after a drift whose displacements have been tracked: the
-// step's gate (a particle moved more than skin / 2 since the lists' build),
-// then the sort, every kernel of which returns at once unless the gate is
-// set.  Nothing here depends on the host, so captured steps replay it.
-int run_list_update(sdpd_ctx* c) {
+// sort, which returns at once unless a particle moved more than skin / 2
+// since the lists' build.  Nothing here depends on the host, so captured
+// steps replay it.
+int run_list_update(sdpd_ctx* c, bool advance = false) {
   c->P.step = c->step;
   {
     PhaseMark pm(c, 1);
-    sdpd::launch_decide(c->stream, c->P, c->S);
-    sdpd::launch_cell_keys(c->stream, c->P, c->S, c->S.gate);
-    sdpd::launch_cell_sort_after_keys(c->stream, c->P, c->S, c->S.gate, true);
+    sdpd::launch_sort(c->stream, c->P, c->S, sdpd::SortKind::kVerletGated, advance);
   }
   int rc = check_launch(c, "list update");
   if (rc) return rc;
@@ -694,7 +689,10 @@ int prime_colloids(sdpd_ctx* c) {
 int step_body(sdpd_ctx* c, int closing) {
   c->step += 1;
   c->P.step = c->step;
-  sdpd::launch_advance_step(c->stream, c->P, c->S);
+  // boxes with sheared faces and colloids read the step's time before the
+  // sort, which otherwise advances it along the way
+  const bool early = c->P.le_g >= 0 || c->P.ncoll > 0;
+  if (early) sdpd::launch_advance_step(c->stream, c->P, c->S);
   {
     PhaseMark pm(c, 0);
     // the colloid block moves only boundary particles, the drift only fluid
@@ -705,19 +703,23 @@ int step_body(sdpd_ctx* c, int closing) {
   int rc = check_launch(c, "step boundary");
   if (rc) return rc;
   c->cells_valid = false;
-  if ((rc = c->P.verlet ? run_list_update(c) : run_sort(c, true))) return rc;
+  if ((rc = c->P.verlet ? run_list_update(c, !early) : run_sort(c, true, !early))) return rc;
   if ((rc = run_density(c))) return rc;
   return run_forces(c);
 }
 
-// Records two closing-kick steps on the context stream into a graph.
+// Records kGraphSteps closing-kick steps on the context stream into a graph.
 // Nothing runs during capture: the host step counter is restored, and the
-// two sorts leave the ping-pong parity where it was.
-int capture_two_steps(sdpd_ctx* c, hipGraphExec_t* out) {
+// even number of sorts leaves the ping-pong parity where it was.
+// (A graph's launch leaves the GPU idle for a few us: the 64 x 64 wave takes
+// 59.5 us per step in graphs of 2, 58.3 of 4, 57.8 of 8; what is left over
+// runs directly, at 0 to 1 us more per step.)
+constexpr int kGraphSteps = 4;
+int capture_steps(sdpd_ctx* c, hipGraphExec_t* out) {
   const int64_t step0 = c->step;
   HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-  int rc = step_body(c, 1);
-  if (!rc) rc = step_body(c, 1);
+  int rc = SDPD_OK;
+  for (int k = 0; k < kGraphSteps && !rc; ++k) rc = step_body(c, 1);
   hipGraph_t graph = nullptr;
   hipError_t e = hipStreamEndCapture(c->stream, &graph);
   c->step = step0;
@@ -995,6 +997,8 @@ int upload_impl(sdpd_ctx* c, const double* x, const double* v, const double* m,
     sdpd::launch_set_step(c->stream, c->S, c->step, t, tle, tprev);
   }
   sdpd::launch_fill_i32(c->stream, c->S.gate, 0, 4);
+  sdpd::launch_fill_i32(c->stream, c->S.sort_ctl, 0, 8);
+  sdpd::launch_fill_i32(c->stream, c->S.count, 0, c->P.ncell);
   sdpd::launch_fill_i32(c->stream, reinterpret_cast<int32_t*>(c->S.disp), 0, 2);
   sdpd::launch_fill_f64(c->stream, c->S.f, 0.0, (int64_t)dim * n);
   sdpd::launch_fill_f64(c->stream, c->S.rho, 0.0, n);
@@ -1238,16 +1242,16 @@ int sdpd_step(sdpd_ctx* c, int32_t nsteps) {
   if (nsteps == 0) return SDPD_OK;
   // the first step opens without a closing kick (the previous call ended
   // with it); every later one starts with the closing kick of the one
-  // before, two at a time through a captured graph when possible
+  // before, kGraphSteps at a time through a captured graph when possible
   if ((rc = step_body(c, 0))) return rc;
   int32_t left = nsteps - 1;
-  if (c->use_graphs && !c->timing && left >= 2) {
+  if (c->use_graphs && !c->timing && left >= kGraphSteps) {
     hipGraphExec_t& g = c->graph[c->parity];
-    if (!g && (rc = capture_two_steps(c, &g))) return rc;
-    while (left >= 2) {
+    if (!g && (rc = capture_steps(c, &g))) return rc;
+    while (left >= kGraphSteps) {
       HIP_TRY(c, hipGraphLaunch(g, c->stream));
-      c->step += 2;
-      left -= 2;
+      c->step += kGraphSteps;
+      left -= kGraphSteps;
     }
   }
   for (; left > 0; --left)

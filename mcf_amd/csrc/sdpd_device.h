@@ -203,6 +203,17 @@ __device__ __forceinline__ double f_modulo(double a, double p) {
   return r;
 }
 
+// One marching step: step + 1, time_current + dt (marching_marching.F90:
+// 1392-1393), and the Lees-Edwards shear length is evaluated at
+// time_current + dt (marching_integrate_VV.F90:784-786).
+__device__ __forceinline__ void advance_step(int64_t* step_dev, double* time_dev, double dt) {
+  step_dev[0] = step_dev[0] + 1;
+  const double t = time_dev[0] + dt;
+  time_dev[2] = time_dev[1];
+  time_dev[0] = t;
+  time_dev[1] = t + dt;
+}
+
 // Histogram slot of key k, aggregated per wave (every lane of the wave
 // calls it; lanes with act false count nothing and get 0).  Equal keys in
 // runs of neighbouring lanes -- particles stored in cell order -- cost one

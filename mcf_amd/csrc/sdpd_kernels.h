@@ -26,8 +26,9 @@ struct DeviceState {
   // mixed precision records (cell order)
   float4 *xa;            // FP32 position relative to the own cell corner, w = cell x index
   // work map of the pair kernels (chunks of <= 64 particles of one row)
-  int32_t *row_nchunk, *row_chunk_off, *chunk_row;
+  int32_t *row_chunk_off, *chunk_row;
   int32_t *scan_tmp;     // tile sums of the exclusive scans
+  int32_t *sort_ctl;     // counters of the sort chain (8, zero between sorts)
   // FP64 records of the force pass, planes of n 16-byte entries: (x, y),
   // (z, p/n^2), (vx, vy), (vz, 1/n^2); Oldroyd-B also Pi / n^2 as (xx, yy),
   // (zz, xy), (xz, yz) (2D: zz and the last plane 0)
@@ -75,8 +76,8 @@ struct DeviceState {
   // reference-grid cell list (built on request by sdpd_get_cells)
   int32_t *rkey, *rslot, *rcount, *rstart, *runsorted, *rlpdx;
   // Verlet lists: positions at the last build (cell order), the step's
-  // gate (gate[0] = 1: the lists are rebuilt this step; gate[1] counts the
-  // builds; gate[2] = 1: a chunk's lists overflowed at the last build, so
+  // gate (gate[0] = 1: the next density pass builds the lists; gate[1] counts
+  // the builds; gate[2] = 1: a chunk's lists overflowed at the last build, so
   // the rescan passes have work), the bits of the largest squared
   // displacement since the build
   // seen this step, and the in-cut-off neighbours of each particle in the
@@ -87,21 +88,21 @@ struct DeviceState {
   int32_t* nbr_in;
 };
 
-void launch_fill_i32(hipStream_t s, int32_t* a, int32_t v, int64_t n,
-                     const int32_t* gate = nullptr);
+void launch_fill_i32(hipStream_t s, int32_t* a, int32_t v, int64_t n);
 void launch_fill_f64(hipStream_t s, double* a, double v, int64_t n);
-// key + histogram (counts zeroed first), then scan, scatter and place into
-// the *_alt buffers.  Without copy_back the caller swaps the ping-pong
-// pointers afterwards; with it the sorted state is copied back into the
-// primary buffers (and into x_ref), so the buffers never change, which lets
-// a captured graph sort on some steps only.  A non-null gate makes every
-// kernel of the sort return at once unless gate[0] != 0.
-void launch_cell_keys(hipStream_t s, const DevParams& P, const DeviceState& S,
-                      const int32_t* gate = nullptr);
-void launch_exclusive_scan(hipStream_t s, const int32_t* count, int32_t* start, int32_t m,
-                           int32_t* tile_sums, const int32_t* gate = nullptr);
-void launch_cell_sort_after_keys(hipStream_t s, const DevParams& P, const DeviceState& S,
-                                 const int32_t* gate = nullptr, bool copy_back = false);
+// The cell sort of the step grid (cell counts and sort_ctl are zero before and
+// after).  Lists rebuilt every step: the sorted state is in the *_alt buffers
+// and the caller swaps the ping-pong pointers (kStepKeysDone: the step
+// boundary has counted the cells already).  Verlet lists: the sorted state is
+// copied back into the primary buffers (and into x_ref), so the buffers never
+// change and a captured graph can hold the sort; kVerletGated runs only if the
+// lists are outdated, and either way sets gate[0] when the next density pass
+// has to build them.  advance: also k_advance_step's work.
+enum class SortKind { kStep, kStepKeysDone, kVerletGated, kVerletForced };
+void launch_sort(hipStream_t s, const DevParams& P, const DeviceState& S, SortKind kind,
+                 bool advance = false);
+// the same sort, one launch per phase, without sort_ctl and the gate
+void launch_sort_phases(hipStream_t s, const DevParams& P, const DeviceState& S, bool copy_back);
 // PPM's cell list on PPM's grid, particles ordered by upload index inside a
 // cell (ppm_util_rank3d on the particles in upload order); fills rstart and
 // rlpdx without moving the state
@@ -116,15 +117,9 @@ void launch_forces(hipStream_t s, const DevParams& P, const DeviceState& S, bool
 void launch_signature(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed);
 void launch_refresh_records(hipStream_t s, const DevParams& P, const DeviceState& S);
 
-// Verlet lists: displacement since the last build and the FP32 cell-relative
-// positions after a drift (every particle), then the step's gate: 1 when a
-// particle moved more than skin / 2 (the displacement maximum is cleared)
+// Verlet lists: displacement since the last build and the positions the walks
+// gather, after a separate drift
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S);
-void launch_decide(hipStream_t s, const DevParams& P, const DeviceState& S);
-// after a sort outside the step: gate[0] = 1 (build at the next density pass)
-void launch_force_build(hipStream_t s, const DeviceState& S);
-// after a density pass: gate[0] = 0 (the lists are current)
-void launch_lists_current(hipStream_t s, const DeviceState& S);
 void launch_kick(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);
 void launch_drift_wrap(hipStream_t s, const DevParams& P, const DeviceState& S);
 void launch_conformation(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);

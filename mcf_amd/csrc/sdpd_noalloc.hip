@@ -123,7 +123,6 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   S.time_dev = c.take<double>(4);
   const size_t nchunk = (N + 63) / 64 + nrows;
   const size_t ntile = (std::max((size_t)P.ncell, nrows) + 4095) / 4096 + 1;
-  S.row_nchunk = c.take<int32_t>(nrows);
   S.row_chunk_off = c.take<int32_t>(nrows + 1);
   S.chunk_row = c.take<int32_t>(nchunk);
   S.scan_tmp = c.take<int32_t>(ntile);
@@ -139,23 +138,29 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
 
 // Geometry tables of the single box: its RepGeom and, per row of the sort
 // grid, first cell, length and replica (0).
-__global__ void k_na_geometry(RepGeom g, int32_t nrows, RepGeom* __restrict__ geo,
-                              int32_t* __restrict__ row_cell, int32_t* __restrict__ row_len,
-                              int32_t* __restrict__ row_rep) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r == 0) *geo = g;
-  if (r >= nrows) return;
-  row_cell[r] = r * g.nm[0];
-  row_len[r] = g.nm[0];
-  row_rep[r] = 0;
-}
-
-// The caller's column-major x(dim, n), v(dim, n), m(n), id(2, n) into the
-// structure-of-arrays state in upload order.
-__global__ void k_na_ingest(int32_t n, int32_t dim, const double* __restrict__ x,
+// The noise step and the lists' gate (their build is due), the counts of the
+// cell sort cleared, and the caller's column-major x(dim, n), v(dim, n), m(n),
+// id(2, n) into the structure-of-arrays state in upload order.
+__global__ void k_na_ingest(RepGeom g, int32_t n, int32_t dim, int32_t nrows, int32_t ncell,
+                            int64_t step, const double* __restrict__ x,
                             const double* __restrict__ v, const double* __restrict__ m,
                             const int32_t* __restrict__ id, DeviceState S) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) {
+    *const_cast<RepGeom*>(S.geo) = g;
+    S.step_dev[0] = step;
+    // (the times only serve sheared faces, which this entry lacks)
+    for (int q = 0; q < 4; ++q) S.time_dev[q] = 0.0;
+    S.gate[0] = 1;
+    S.gate[1] = S.gate[2] = S.gate[3] = 0;
+  }
+  const int stride = gridDim.x * blockDim.x;
+  for (int r = i; r < nrows; r += stride) {
+    S.row_cell[r] = r * g.nm[0];
+    S.row_len[r] = g.nm[0];
+    S.row_rep[r] = 0;
+  }
+  for (int c = i; c < ncell; c += stride) S.count[c] = 0;
   if (i >= n) return;
   for (int d = 0; d < dim; ++d) {
     S.x[(int64_t)d * n + i] = x[(int64_t)dim * i + d];
@@ -243,18 +248,12 @@ extern "C" int sdpd_evaluate_noalloc(const sdpd_params* params, int64_t step, co
 
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int nb = (n + 255) / 256;
-  hipLaunchKernelGGL(k_na_geometry, dim3((P.nrows + 255) / 256), dim3(256), 0, s, g, P.nrows,
-                     const_cast<RepGeom*>(S.geo), S.row_cell, S.row_len, S.row_rep);
-  // noise step; the times only serve sheared faces, which this entry lacks
-  sdpd::launch_set_step(s, S, step, 0.0, 0.0, 0.0);
-  hipLaunchKernelGGL(k_na_ingest, dim3(nb), dim3(256), 0, s, n, P.dim, x, v, m, id, S);
+  hipLaunchKernelGGL(k_na_ingest, dim3(nb), dim3(256), 0, s, g, n, P.dim, P.nrows, P.ncell, step,
+                     x, v, m, id, S);
   // technique_build_list: the sort writes the *_alt copies, which are
-  // copied back (Verlet lists, whose build the gate then asks for) or swap
-  sdpd::launch_cell_keys(s, P, S);
-  sdpd::launch_cell_sort_after_keys(s, P, S, nullptr, P.verlet != 0);
-  if (P.verlet) {
-    sdpd::launch_force_build(s, S);
-  } else {
+  // copied back (Verlet lists) or swap
+  sdpd::launch_sort_phases(s, P, S, P.verlet != 0);
+  if (!P.verlet) {
     std::swap(S.x, S.x_alt);
     std::swap(S.v, S.v_alt);
     std::swap(S.m, S.m_alt);

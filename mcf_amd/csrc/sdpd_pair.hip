@@ -1287,15 +1287,13 @@ __device__ __forceinline__ bool chunk_meets_le_face(int le_g, const Chunk& ch, i
 // frame's state would cost the whole pass registers and occupancy).
 //
 // Modes.  kStore: the in-cut-off pairs found by the candidate scan are
-// stored; lists rebuilt every step.  Verlet lists decide in / out of the
-// cut-off per candidate on the current positions: kBuild (steps whose gate
-// is set) scans the stencil for every candidate within rc + skin and stores
-// them; kWalk (the other steps) walks the stored candidates of the chunks
-// whose lists hold them all; kRescan (those steps) scans the stencil again,
-// without storing, for the chunks with an overflowed list; kScanAll does
-// that for every chunk whatever the gate (the autotuner).  The walk and the
-// scans visit the candidates in the same order, so they give the same sums.
-enum DensityMode { kStore = 0, kBuild = 1, kRescan = 3, kScanAll = 4 };
+// summed and stored (lists rebuilt every step).  Verlet lists decide the
+// cut-off per candidate on the current positions: kScan scans the stencil,
+// on steps whose gate asks for it for every chunk, storing the candidates
+// within rc + skin, and on the others for the chunks whose lists overflowed,
+// without storing (k_density_walk takes the rest); kScanAll does the latter
+// for every chunk (autotune's timing of the scan).
+enum DensityMode { kStore = 0, kScan = 1, kScanAll = 2 };
 
 // Density epilogue of particle i with number (or mass) density sum rho.
 template <int DIM>
@@ -1336,16 +1334,17 @@ __device__ __forceinline__ double density_of(const DevParams& P, double sum) {
 // One chunk slot of a density pass that scans the stencil.
 template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
 __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceState& S, int slot,
-                                              int le_box, float4* __restrict__ tile,
+                                              int le_box, bool build,
+                                              float4* __restrict__ tile,
                                               uint32_t* __restrict__ buf) {
   constexpr bool kDecide = MODE != kStore;
   Chunk ch;
   if (!load_chunk(P, S, ch, slot)) return;
   if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
-  if (MODE == kRescan && !list_overflow(P, S, ch)) return;
+  if (MODE == kScan && !build && !list_overflow(P, S, ch)) return;
   const Home h = load_home<DIM>(P, S, ch);
   const double mi = S.m[h.ii];
-  uint32_t* list = (MODE == kStore || MODE == kBuild) ? S.nlist : nullptr;
+  uint32_t* list = (MODE == kStore || (MODE == kScan && build)) ? S.nlist : nullptr;
   using Pol = std::conditional_t<
       MIXED, std::conditional_t<kDecide, DensityMixed<DIM>, DensityMixedStep<DIM>>,
       DensityF64<DIM, kDecide>>;
@@ -1364,11 +1363,11 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
     rho = density_of<MIXED>(P, pol.acc);
   if (!h.active) return;
   const int i = h.i;
-  if (MODE == kStore || MODE == kBuild) S.nbr_count[i] = cnt;
-  if (MODE == kBuild && cnt > P.list_cap) S.gate[2] = 1;  // every writer stores 1
+  if (MODE == kStore || (MODE == kScan && build)) S.nbr_count[i] = cnt;
+  if (MODE == kScan && build && cnt > P.list_cap) S.gate[2] = 1;  // every writer stores 1
   // the shear time of the build (the copies across sheared faces drift
   // from their build positions as it advances)
-  if (MODE == kBuild && i == 0) S.time_dev[3] = S.time_dev[1];
+  if (MODE == kScan && build && i == 0) S.time_dev[3] = S.time_dev[1];
   finish_density<DIM>(P, S, i, mi, rho, kDecide ? pol.nin : cnt, rechecks + pol.rechecks);
 }
 
@@ -1423,29 +1422,27 @@ __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState
   finish_density<DIM>(P, S, i, S.m[i], density_of<MIXED>(P, rho), nin, rechecks);
 }
 
-// The rescan (kRescan) has work only after a list overflowed at the build;
-// it is launched on a reduced grid, whose workgroups take every gridDim.x-th
-// chunk slot, so that on the other steps its launch costs little.
+// kScan has work only when the lists are built or one overflowed then: its
+// workgroups take every gridDim.x-th chunk slot, so that on the other steps
+// the launch is cheap.
 template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
 __global__ __launch_bounds__(kWave) void k_density(DevParams P, DeviceState S) {
-  if (MODE == kBuild && S.gate[0] == 0) return;
-  if (MODE == kRescan && S.gate[0] != 0) return;
-  // no list overflowed at the build: nothing to rescan
-  if (MODE == kRescan && S.gate[2] == 0) return;
+  const bool build = MODE == kScan && S.gate[0] != 0;
+  if (MODE == kScan && !build && S.gate[2] == 0) return;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   __shared__ float4 tile[TILE + 1];
   // whole groups of 8 rows: the final flush stores the last group of a
   // lane's entries as 8 rows, of which those past its count are padding
   __shared__ uint32_t buf[(BUF + 7) / 8 * 8 * kWave];
-  if (MODE == kRescan) {
+  if (MODE == kScan) {
     const int slots = chunk_slots(P);
     for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
-      density_chunk<DIM, MIXED, TILE, BUF, LE, MODE>(P, S, slot, le_box, tile, buf);
+      density_chunk<DIM, MIXED, TILE, BUF, LE, MODE>(P, S, slot, le_box, build, tile, buf);
       __syncthreads();
     }
   } else {
-    density_chunk<DIM, MIXED, TILE, BUF, LE, MODE>(P, S, blockIdx.x, le_box, tile, buf);
+    density_chunk<DIM, MIXED, TILE, BUF, LE, MODE>(P, S, blockIdx.x, le_box, false, tile, buf);
   }
 }
 
@@ -2445,6 +2442,8 @@ enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
 // code decode and compensated FP32 sums, one particle per lane).
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC>
 __global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? 6 : 1)) void k_force_walk(DevParams P, DeviceState S) {
+  // the density pass has built the lists that were due
+  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (SPEC != kAny) {
@@ -2539,8 +2538,6 @@ __global__ __launch_bounds__(kWave) void k_signature(DevParams P, DeviceState S)
 // launchers: one 64-lane workgroup per chunk; the grid covers the upper
 // bound of chunks (one partial chunk per row plus n / 64 full ones)
 // ---------------------------------------------------------------------
-static inline int nchunks_max(const DevParams& P) { return chunk_slots(P); }
-
 // Chunk slots from which a density walk takes a whole chunk per workgroup.
 constexpr int kWholeChunkSlots = 4096;
 
@@ -2563,16 +2560,17 @@ static void launch_density_walk(hipStream_t s, const DevParams& P, const DeviceS
   }
 }
 
-// Workgroups of a rescan launch (a multiple of 8, at most the slots): few
-// enough that the launch is cheap on the steps without an overflowed list
-// (on the 128^3 box, whose 33k slots each took a workgroup before, the two
-// rescans now cost the step 15 us less), and enough that a step with
-// overflowed lists checks its slots 16 at a time.
-static inline dim3 rescan_grid(const DevParams& P) { return dim3(std::min(chunk_slots(P), 2048)); }
+// Workgroups of a launch that has work only after a list build or overflow (a
+// multiple of 8, at most the slots): few enough that the launch is cheap on
+// the other steps (on the 128^3 box, with 33k slots, two such launches cost
+// 15 us less than with a workgroup per slot), and enough to fill the GPU.
+static inline dim3 strided_grid(const DevParams& P) {
+  return dim3(std::min(chunk_slots(P), 4096));
+}
 
 template <int DIM, bool MIXED, bool LE, int MODE>
 static void launch_density_shape(hipStream_t s, const DevParams& P, const DeviceState& S) {
-  dim3 g(nchunks_max(P)), b(kWave);
+  const dim3 g = MODE == kScan ? strided_grid(P) : dim3(chunk_slots(P)), b(kWave);
   switch (P.density_shape) {
     case 1:
       hipLaunchKernelGGL((k_density<DIM, MIXED, 128, 16, LE, MODE>), g, b, 0, s, P, S);
@@ -2600,24 +2598,17 @@ static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceSt
     launch_density_shape<DIM, MIXED, false, kScanAll>(s, P, S);
     return;
   }
-  // Verlet lists: each kernel returns at once unless the step's gate
-  // selects it (build, or walk + rescan of overflowed chunks); a box with
-  // sheared faces splits the chunks between the Lees-Edwards and the plain
-  // instantiations, as its per-step lists do
-  const dim3 b(kWave);
+  // Verlet lists: the gate and the overflow flag decide which of the two
+  // kernels takes a chunk; a box with sheared faces splits the chunks between
+  // the Lees-Edwards and the plain instantiations, as its per-step lists do
   if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
     if (P.le_g >= 0) {
-      launch_density_shape<DIM, MIXED, true, kBuild>(s, P, S);
+      launch_density_shape<DIM, MIXED, true, kScan>(s, P, S);
       launch_density_walk<DIM, MIXED, true>(s, P, S);
-      hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, true, kRescan>), rescan_grid(P), b,
-                         0, s, P, S);
     }
   }
-  launch_density_shape<DIM, MIXED, false, kBuild>(s, P, S);
+  launch_density_shape<DIM, MIXED, false, kScan>(s, P, S);
   launch_density_walk<DIM, MIXED, false>(s, P, S);
-  hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, false, kRescan>), rescan_grid(P), b, 0,
-                     s, P, S);
-  launch_lists_current(s, S);
 }
 
 void launch_density(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed,
@@ -2645,7 +2636,7 @@ void launch_refresh_records(hipStream_t s, const DevParams& P, const DeviceState
 
 template <int DIM, int FT, bool MIXED, bool COLL>
 static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceState& S) {
-  dim3 g(nchunks_max(P)), b(kWave);
+  dim3 g(chunk_slots(P)), b(kWave);
   if (P.verlet) {
     // as the lists rebuilt every step: with colloids the chunks near a
     // sheared face take the Lees-Edwards instantiation and the others the
@@ -2654,7 +2645,7 @@ static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceStat
     if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
       if (P.le_g >= 0) {
         hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, true, kAny>), gq, b, 0, s, P, S);
-        hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, true, true, true>), rescan_grid(P), b,
+        hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, true, true, true>), strided_grid(P), b,
                            0, s, P, S);
       }
     }
@@ -2669,7 +2660,7 @@ static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceStat
       else
         hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kNoNoise>), gq, b, 0, s, P,
                            S);
-      hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, false, true, true>), rescan_grid(P), b,
+      hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, false, true, true>), strided_grid(P), b,
                          0, s, P, S);
     }
     return;
@@ -2769,7 +2760,7 @@ void launch_forces(hipStream_t s, const DevParams& P, const DeviceState& S, bool
 
 void launch_signature(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed) {
   (void)mixed;  // both modes share the decision
-  dim3 g(nchunks_max(P)), b(kWave);
+  dim3 g(chunk_slots(P)), b(kWave);
   const bool le = P.le_g >= 0;
   if (P.dim == 3) {
     if (P.verlet && le)

@@ -267,52 +267,6 @@ __global__ __launch_bounds__(256) void k_track(DevParams P, DeviceState S) {
   block_max_disp(S.disp, d2);
 }
 
-// The step's gate: rebuild the lists when a particle moved more than
-// skin / 2 since their build (a pair then may have closed in by more than
-// the skin); the displacement maximum starts again from zero.  gate[1]
-// counts the builds; gate[2], set by the build, flags lists that
-// overflowed their capacity.
-__global__ void k_decide(DevParams P, DeviceState S) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  const double d2 = __longlong_as_double((long long)S.disp[0]);
-  double lim = P.half_skin2;
-  int rebuild = 0;
-  if (P.le_g >= 0) {
-    // sheared faces: the copies across a face move by |v_upper - v_lower|
-    // per unit time against the box, so a pair across it may have closed
-    // in by that drift since the build on top of the particles' own
-    // displacements: the lists hold while 2 max |dx| + drift < skin.  A
-    // list that overflowed rebuilds every step (the rescans then always
-    // see the positions of a build).
-    const double drift = fabs(P.le_vhi - P.le_vlo) * fabs(S.time_dev[1] - S.time_dev[3]);
-    const double room = 0.5 * (P.skin - drift);
-    lim = room > 0.0 ? room * room : -1.0;
-    rebuild = S.gate[2] != 0 ? 1 : 0;
-  }
-  rebuild = rebuild | (d2 > lim ? 1 : 0);
-  // a build still pending (a sort whose lists no density pass has built
-  // yet) stays pending
-  S.gate[0] |= rebuild;
-  S.gate[1] += rebuild;
-  if (rebuild) S.gate[2] = 0;
-  S.disp[0] = 0ull;
-}
-
-// After the density pass: the lists are current (no build pending).
-__global__ void k_lists_current(DeviceState S) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
-}
-
-// A sort requested outside the step (upload, a cell-list call, a check):
-// the next density pass builds the lists.
-__global__ void k_force_build(DeviceState S) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  S.gate[0] = 1;
-  S.gate[1] += 1;
-  S.gate[2] = 0;
-  S.disp[0] = 0ull;
-}
-
 // Neumaier-compensated sum helpers
 struct KSum {
   double s, c;
@@ -401,18 +355,9 @@ __global__ void k_set_step(int64_t* __restrict__ step_dev, double* __restrict__ 
   }
 }
 
-// One marching step: step + 1, time_current + dt (marching_marching.F90:
-// 1392-1393), and the Lees-Edwards shear length is evaluated at
-// time_current + dt (marching_integrate_VV.F90:784-786).
 __global__ void k_advance_step(int64_t* __restrict__ step_dev, double* __restrict__ time_dev,
                                double dt) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    step_dev[0] = step_dev[0] + 1;
-    const double t = time_dev[0] + dt;
-    time_dev[2] = time_dev[1];
-    time_dev[0] = t;
-    time_dev[1] = t + dt;
-  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) advance_step(step_dev, time_dev, dt);
 }
 
 __global__ void k_pair_normals(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
@@ -454,7 +399,6 @@ void launch_boundary(hipStream_t s, const DevParams& P, const DeviceState& S, in
       hipLaunchKernelGGL((k_boundary<2, true>), g, b, 0, s, P, S, closing, opening);
     return;
   }
-  launch_fill_i32(s, S.count, 0, P.ncell);
   if (P.dim == 3)
     hipLaunchKernelGGL((k_boundary<3, false>), g, b, 0, s, P, S, closing, opening);
   else
@@ -463,18 +407,6 @@ void launch_boundary(hipStream_t s, const DevParams& P, const DeviceState& S, in
 
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S) {
   hipLaunchKernelGGL(k_track, dim3(nblk(P.n)), dim3(256), 0, s, P, S);
-}
-
-void launch_decide(hipStream_t s, const DevParams& P, const DeviceState& S) {
-  hipLaunchKernelGGL(k_decide, dim3(1), dim3(64), 0, s, P, S);
-}
-
-void launch_force_build(hipStream_t s, const DeviceState& S) {
-  hipLaunchKernelGGL(k_force_build, dim3(1), dim3(64), 0, s, S);
-}
-
-void launch_lists_current(hipStream_t s, const DeviceState& S) {
-  hipLaunchKernelGGL(k_lists_current, dim3(1), dim3(64), 0, s, S);
 }
 
 void launch_stats(hipStream_t s, const DevParams& P, const DeviceState& S, int nblocks) {
