@@ -120,6 +120,9 @@ void launch_refresh_records(hipStream_t s, const DevParams& P, const DeviceState
 // Verlet lists: displacement since the last build and the positions the walks
 // gather, after a separate drift
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S);
+// src (comps planes of n, cell order) -> dst (comps, n) in upload order
+void launch_to_upload_order(hipStream_t s, const DevParams& P, const DeviceState& S, int comps,
+                            const double* src, double* dst);
 void launch_kick(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);
 void launch_drift_wrap(hipStream_t s, const DevParams& P, const DeviceState& S);
 void launch_conformation(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);

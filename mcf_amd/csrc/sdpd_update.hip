@@ -360,6 +360,17 @@ __global__ void k_advance_step(int64_t* __restrict__ step_dev, double* __restric
   if (blockIdx.x == 0 && threadIdx.x == 0) advance_step(step_dev, time_dev, dt);
 }
 
+// One quantity from cell order, structure of arrays, to upload order with a
+// particle's components together.
+__global__ void k_to_upload_order(int n, int comps, const int32_t* __restrict__ perm,
+                                  const double* __restrict__ src, double* __restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t u = perm[i];
+  if (u < 0 || u >= n) return;
+  for (int q = 0; q < comps; ++q) dst[u * comps + q] = src[(int64_t)q * n + i];
+}
+
 __global__ void k_pair_normals(const uint32_t* __restrict__ lo, const uint32_t* __restrict__ hi,
                                int count, uint64_t seed, int64_t step, float* __restrict__ g) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -370,7 +381,6 @@ __global__ void k_pair_normals(const uint32_t* __restrict__ lo, const uint32_t* 
 }
 
 static inline int nblk(int64_t n) { return (int)((n + 255) / 256); }
-
 
 int stats_blocks(int n) {
   int b = nblk(n);
@@ -403,6 +413,12 @@ void launch_boundary(hipStream_t s, const DevParams& P, const DeviceState& S, in
     hipLaunchKernelGGL((k_boundary<3, false>), g, b, 0, s, P, S, closing, opening);
   else
     hipLaunchKernelGGL((k_boundary<2, false>), g, b, 0, s, P, S, closing, opening);
+}
+
+void launch_to_upload_order(hipStream_t s, const DevParams& P, const DeviceState& S, int comps,
+                            const double* src, double* dst) {
+  hipLaunchKernelGGL(k_to_upload_order, dim3(nblk(P.n)), dim3(256), 0, s, P.n, comps, S.perm, src,
+                     dst);
 }
 
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S) {
