@@ -142,35 +142,33 @@ __global__ void k_scatter(int n, const int32_t* __restrict__ key, const int32_t*
 // the sort of the step, as items of work in phases
 // ---------------------------------------------------------------------
 // Phases (each needs all of the one before):
-//   keys     cell key, slot and histogram       1024 particles per item
+//   keys     cell key, slot and histogram       ITEM particles per item
 //   sums     sums of 4096 cell counts           one tile per item
 //   starts   first particle of every cell       one tile per item, which adds
 //                                               up the sums of the tiles before
-//   scatter  unsorted[start[key] + slot] = i    1024 particles; item 0 is the
+//   scatter  unsorted[start[key] + slot] = i    ITEM particles; item 0 is the
 //                                               pair kernels' work map
 //   place    rank in the cell, state moved to the *_alt buffers, cell counts
-//            cleared for the next sort          1024 particles
+//            cleared for the next sort          ITEM particles
 //   back     the state copied back, with x_ref and the walks' positions
-//                                               1024 particles (Verlet lists)
+//                                               ITEM particles (Verlet lists)
 // The counts are zero between sorts.
 constexpr int kSortThreads = 256;
-constexpr int kSortItem = 1024;
 enum SortPhase { kKeys = 0, kSums, kStarts, kScatter, kPlace, kBack, kSortPhases };
 
 struct SortPlan {
   int32_t items[kSortPhases];
-  int32_t copy_back;
 };
 
-static SortPlan sort_plan(const DevParams& P, bool keys, bool copy_back) {
-  const int32_t blocks = (P.n + kSortItem - 1) / kSortItem;
+static SortPlan sort_plan(const DevParams& P, int item, bool keys, bool copy_back) {
+  const int32_t blocks = (P.n + item - 1) / item;
   const int32_t tiles = (P.ncell + kScanTile - 1) / kScanTile;
-  return {{keys ? blocks : 0, tiles, tiles, blocks + 1, blocks, copy_back ? blocks : 0},
-          copy_back ? 1 : 0};
+  return {{keys ? blocks : 0, tiles, tiles, blocks + 1, blocks, copy_back ? blocks : 0}};
 }
 
-// exclusive scan over the workgroup's 256 threads
-__device__ __forceinline__ int32_t block_scan_256(int32_t v, int32_t& total, int32_t* wsum) {
+// exclusive scan over the workgroup's T threads
+template <int T>
+__device__ __forceinline__ int32_t block_scan(int32_t v, int32_t& total, int32_t* wsum) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   int32_t incl = v;
 #pragma unroll
@@ -180,17 +178,23 @@ __device__ __forceinline__ int32_t block_scan_256(int32_t v, int32_t& total, int
   }
   if (lane == 63) wsum[wid] = incl;
   __syncthreads();
-  const int32_t a = wsum[0], b = wsum[1], c = wsum[2], d = wsum[3];
-  total = a + b + c + d;
-  const int32_t before = wid == 0 ? 0 : (wid == 1 ? a : (wid == 2 ? a + b : a + b + c));
+  int32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    before += w < wid ? wsum[w] : 0;
+    total += wsum[w];
+  }
   __syncthreads();
   return before + incl - v;
 }
 
+template <int T, int ITEM>
 __device__ __forceinline__ void sort_keys(const DevParams& P, const DeviceState& S, int item) {
   const int64_t n = P.n;
-  for (int q = 0; q < kSortItem / kSortThreads; ++q) {
-    const int i0 = item * kSortItem + q * kSortThreads + (int)threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < ITEM / T; ++q) {
+    const int i0 = item * ITEM + q * T + (int)threadIdx.x;
     const bool act = i0 < P.n;
     const int i = act ? i0 : P.n - 1;  // every lane takes part in the histogram
     const RepGeom& g = S.geo[S.rep[i]];
@@ -204,23 +208,26 @@ __device__ __forceinline__ void sort_keys(const DevParams& P, const DeviceState&
   }
 }
 
+template <int T>
 __device__ __forceinline__ void sort_sums(const DevParams& P, const DeviceState& S, int item,
                                           int32_t* wsum) {
-  const int64_t base = (int64_t)item * kScanTile + threadIdx.x * (kScanTile / kSortThreads);
+  const int64_t base = (int64_t)item * kScanTile + threadIdx.x * (kScanTile / T);
   int32_t local = 0;
-  for (int q = 0; q < kScanTile / kSortThreads; ++q)
+#pragma unroll
+  for (int q = 0; q < kScanTile / T; ++q)
     if (base + q < P.ncell) local += S.count[base + q];
   int32_t total;
-  (void)block_scan_256(local, total, wsum);
+  (void)block_scan<T>(local, total, wsum);
   if (threadIdx.x == 0) S.scan_tmp[item] = total;
 }
 
+template <int T>
 __device__ __forceinline__ void sort_starts(const DevParams& P, const DeviceState& S, int item,
                                             int32_t* wsum) {
   int32_t part = 0, before;
-  for (int t = threadIdx.x; t < item; t += kSortThreads) part += S.scan_tmp[t];
-  (void)block_scan_256(part, before, wsum);
-  constexpr int kPer = kScanTile / kSortThreads;
+  for (int t = threadIdx.x; t < item; t += T) part += S.scan_tmp[t];
+  (void)block_scan<T>(part, before, wsum);
+  constexpr int kPer = kScanTile / T;
   const int64_t base = (int64_t)item * kScanTile + threadIdx.x * kPer;
   int32_t v[kPer], local = 0;
 #pragma unroll
@@ -229,7 +236,7 @@ __device__ __forceinline__ void sort_starts(const DevParams& P, const DeviceStat
     local += v[q];
   }
   int32_t total;
-  int32_t ex = block_scan_256(local, total, wsum) + before;
+  int32_t ex = block_scan<T>(local, total, wsum) + before;
 #pragma unroll
   for (int q = 0; q < kPer; ++q) {
     if (base + q < P.ncell) S.start[base + q] = ex;
@@ -241,11 +248,12 @@ __device__ __forceinline__ void sort_starts(const DevParams& P, const DeviceStat
 // Work map of the pair kernels: each (y, z) row of the sort grid is cut
 // into chunks of at most 64 consecutive particles; chunk c belongs to row
 // chunk_row[c] and is the (c - row_chunk_off[row])-th chunk of that row.
+template <int T>
 __device__ __forceinline__ void sort_rows(const DevParams& P, const DeviceState& S,
-                                          int32_t* wsum) {
+                                          const int32_t* start, int32_t* wsum) {
   constexpr int kPer = 4;
   int32_t carry = 0;
-  for (int r0 = 0; r0 < P.nrows; r0 += kPer * kSortThreads) {
+  for (int r0 = 0; r0 < P.nrows; r0 += kPer * T) {
     const int base = r0 + (int)threadIdx.x * kPer;
     int32_t nc[kPer], local = 0;
 #pragma unroll
@@ -253,12 +261,12 @@ __device__ __forceinline__ void sort_rows(const DevParams& P, const DeviceState&
       nc[q] = 0;
       if (base + q < P.nrows) {
         const int c0 = S.row_cell[base + q];
-        nc[q] = (S.start[c0 + S.row_len[base + q]] - S.start[c0] + 63) / 64;
+        nc[q] = (start[c0 + S.row_len[base + q]] - start[c0] + 63) / 64;
       }
       local += nc[q];
     }
     int32_t total;
-    int32_t ex = block_scan_256(local, total, wsum) + carry;
+    int32_t ex = block_scan<T>(local, total, wsum) + carry;
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
       if (base + q < P.nrows) {
@@ -272,123 +280,170 @@ __device__ __forceinline__ void sort_rows(const DevParams& P, const DeviceState&
   if (threadIdx.x == 0) S.row_chunk_off[P.nrows] = carry;
 }
 
+template <int T, int ITEM>
 __device__ __forceinline__ void sort_scatter(const DevParams& P, const DeviceState& S, int item) {
-  for (int q = 0; q < kSortItem / kSortThreads; ++q) {
-    const int i = item * kSortItem + q * kSortThreads + (int)threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < ITEM / T; ++q) {
+    const int i = item * ITEM + q * T + (int)threadIdx.x;
     if (i < P.n) S.unsorted[S.start[S.key[i]] + S.slot[i]] = i;
   }
 }
 
+// A particle's state in registers: every load is issued before the first
+// store (the buffers may alias as far as the compiler knows).
+struct Moved {
+  double x[3], v[3], m, ct[9];
+  int32_t pid, perm, rep, sid;
+};
+__device__ __forceinline__ Moved load_moved(const DevParams& P, int i, const double* x,
+                                            const double* v, const double* m, const double* ct,
+                                            const int32_t* pid, const int32_t* perm,
+                                            const int32_t* rep, const int32_t* sid) {
+  const int64_t n = P.n;
+  Moved a;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    a.x[d] = d < P.dim ? x[d * n + i] : 0.0;
+    a.v[d] = d < P.dim ? v[d * n + i] : 0.0;
+  }
+  a.m = m[i];
+  a.pid = pid[i];
+  a.perm = perm[i];
+  a.rep = rep[i];
+  a.sid = P.ncoll ? sid[i] : 0;
+  if (!P.newtonian) {
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (q < P.dim * P.dim) a.ct[q] = ct[q * n + i];
+  }
+  return a;
+}
+__device__ __forceinline__ void store_moved(const DevParams& P, int p, const Moved& a, double* x,
+                                            double* v, double* m, double* ct, int32_t* pid,
+                                            int32_t* perm, int32_t* rep, int32_t* sid) {
+  const int64_t n = P.n;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (d < P.dim) {
+      x[d * n + p] = a.x[d];
+      v[d * n + p] = a.v[d];
+    }
+  m[p] = a.m;
+  pid[p] = a.pid;
+  perm[p] = a.perm;
+  rep[p] = a.rep;
+  if (P.ncoll) sid[p] = a.sid;
+  if (!P.newtonian) {
+#pragma unroll
+    for (int q = 0; q < 9; ++q)
+      if (q < P.dim * P.dim) ct[q * n + p] = a.ct[q];
+  }
+}
+
+// FP32 position relative to the lower corner of the own cell, the cell's x
+// index in w (records of the neighbour scan).
+__device__ __forceinline__ float4 cell_record(const DevParams& P, const RepGeom& g, int32_t k,
+                                              const double* x) {
+  const int kl = k - g.cell_base;
+  const int cx = kl % g.nm[0];
+  const int cy = (kl / g.nm[0]) % g.nm[1];
+  const int cz = kl / (g.nm[0] * g.nm[1]);
+  return make_float4((float)(x[0] - (g.lo[0] + (double)cx * g.cs[0])),
+                     (float)(x[1] - (g.lo[1] + (double)cy * g.cs[1])),
+                     P.dim == 3 ? (float)(x[2] - (g.lo[2] + (double)cz * g.cs[2])) : 0.f,
+                     __int_as_float(cx));
+}
+
+// What the walks gather of the position of slot p, and x_ref.
+__device__ __forceinline__ void store_positions(const DevParams& P, const DeviceState& S,
+                                                const RepGeom& g, int p, const Moved& a) {
+  const int64_t n = P.n;
+  if (P.mixed) {
+    S.xq[p] = make_uint4(fixed_position(g, 0, a.x[0]), fixed_position(g, 1, a.x[1]),
+                         P.dim == 3 ? fixed_position(g, 2, a.x[2]) : 0u, (uint32_t)a.pid);
+  } else {
+    reinterpret_cast<double2*>(S.rec64)[p] = make_double2(a.x[0], a.x[1]);
+  }
+  if (S.x_ref) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (d < P.dim) S.x_ref[d * n + p] = a.x[d];
+  }
+}
+
 // Rank inside the cell by index (stable order) and move the state there.
+template <int T, int ITEM>
 __device__ __forceinline__ void sort_place(const DevParams& P, const DeviceState& S, int item,
                                            int items) {
-  const int64_t n = P.n;
-  const int dim = P.dim;
   const int64_t c0 = (int64_t)P.ncell * item / items, c1 = (int64_t)P.ncell * (item + 1) / items;
-  for (int64_t c = c0 + threadIdx.x; c < c1; c += kSortThreads) S.count[c] = 0;
-  for (int qq = 0; qq < kSortItem / kSortThreads; ++qq) {
-    const int i = item * kSortItem + qq * kSortThreads + (int)threadIdx.x;
+  for (int64_t c = c0 + threadIdx.x; c < c1; c += T) S.count[c] = 0;
+  for (int qq = 0; qq < ITEM / T; ++qq) {
+    const int i = item * ITEM + qq * T + (int)threadIdx.x;
     if (i >= P.n) continue;
     const int32_t k = S.key[i];
+    const Moved a = load_moved(P, i, S.x, S.v, S.m, S.ct, S.pid, S.perm, S.rep, S.sid);
     const int32_t s = S.start[k], e = S.start[k + 1];
     int32_t r = 0;
-    for (int32_t q = s; q < e; ++q) r += S.unsorted[q] < i ? 1 : 0;
+    for (int32_t q = s; q < e; q += 8) {
+      int32_t u[8];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) u[w] = S.unsorted[min(q + w, e - 1)];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) r += (q + w < e && u[w] < i) ? 1 : 0;
+    }
     const int32_t p = s + r;
-    double xv[3] = {0.0, 0.0, 0.0};
-    for (int d = 0; d < dim; ++d) {
-      xv[d] = S.x[d * n + i];
-      S.x_alt[d * n + p] = xv[d];
-      S.v_alt[d * n + p] = S.v[d * n + i];
-    }
-    S.m_alt[p] = S.m[i];
-    S.pid_alt[p] = S.pid[i];
-    S.perm_alt[p] = S.perm[i];
-    if (P.ncoll) {
-      // colloids: species id moves with the particle; the slot of each upload
-      // index locates the boundary particles of a colloid
-      S.sid_alt[p] = S.sid[i];
-      S.slot_of[S.perm[i]] = p;
-    }
-    const int rq = S.rep[i];
-    S.rep_alt[p] = rq;
+    const float4 xa = cell_record(P, S.geo[a.rep], k, a.x);
+    store_moved(P, p, a, S.x_alt, S.v_alt, S.m_alt, S.ct_alt, S.pid_alt, S.perm_alt, S.rep_alt,
+                S.sid_alt);
     S.key_sorted[p] = k;
-    if (!P.newtonian) {
-      const int d2 = dim * dim;
-      for (int q = 0; q < d2; ++q) S.ct_alt[q * n + p] = S.ct[q * n + i];
-    }
-    // FP32 position relative to the lower corner of the own cell, the cell's
-    // x index in w (records of the neighbour scan)
-    const RepGeom& g = S.geo[rq];
-    const int kl = k - g.cell_base;
-    const int cx = kl % g.nm[0];
-    const int cy = (kl / g.nm[0]) % g.nm[1];
-    const int cz = kl / (g.nm[0] * g.nm[1]);
-    S.xa[p] = make_float4((float)(xv[0] - (g.lo[0] + (double)cx * g.cs[0])),
-                          (float)(xv[1] - (g.lo[1] + (double)cy * g.cs[1])),
-                          dim == 3 ? (float)(xv[2] - (g.lo[2] + (double)cz * g.cs[2])) : 0.f,
-                          __int_as_float(cx));
+    S.xa[p] = xa;
+    // (the slot of each upload index locates the boundary particles of a
+    // colloid)
+    if (P.ncoll) S.slot_of[a.perm] = p;
   }
 }
 
 // The sorted state back from the *_alt buffers into the primary ones, the
-// sorted positions into x_ref (the positions of the lists' build) and into
-// what the walks gather.
+// sorted positions into x_ref (the positions of the lists' build; not kept by
+// a single evaluation) and into what the walks gather.
+template <int T, int ITEM>
 __device__ __forceinline__ void sort_back(const DevParams& P, const DeviceState& S, int item) {
-  const int64_t n = P.n;
-  for (int qq = 0; qq < kSortItem / kSortThreads; ++qq) {
-    const int i = item * kSortItem + qq * kSortThreads + (int)threadIdx.x;
+  for (int qq = 0; qq < ITEM / T; ++qq) {
+    const int i = item * ITEM + qq * T + (int)threadIdx.x;
     if (i >= P.n) continue;
-    double xv[3] = {0.0, 0.0, 0.0};
-    for (int d = 0; d < P.dim; ++d) {
-      xv[d] = S.x_alt[d * n + i];
-      S.x[d * n + i] = xv[d];
-      S.x_ref[d * n + i] = xv[d];
-      S.v[d * n + i] = S.v_alt[d * n + i];
-    }
-    const int32_t pid = S.pid_alt[i], rq = S.rep_alt[i];
-    if (P.mixed) {
-      const RepGeom& g = S.geo[rq];
-      S.xq[i] = make_uint4(fixed_position(g, 0, xv[0]), fixed_position(g, 1, xv[1]),
-                           P.dim == 3 ? fixed_position(g, 2, xv[2]) : 0u, (uint32_t)pid);
-    } else {
-      reinterpret_cast<double2*>(S.rec64)[i] = make_double2(xv[0], xv[1]);
-    }
-    S.m[i] = S.m_alt[i];
-    S.pid[i] = pid;
-    S.perm[i] = S.perm_alt[i];
-    S.rep[i] = rq;
-    if (!P.newtonian) {
-      const int d2 = P.dim * P.dim;
-      for (int q = 0; q < d2; ++q) S.ct[q * n + i] = S.ct_alt[q * n + i];
-    }
-    if (P.ncoll) S.sid[i] = S.sid_alt[i];
+    const Moved a = load_moved(P, i, S.x_alt, S.v_alt, S.m_alt, S.ct_alt, S.pid_alt, S.perm_alt,
+                               S.rep_alt, S.sid_alt);
+    store_positions(P, S, S.geo[a.rep], i, a);
+    store_moved(P, i, a, S.x, S.v, S.m, S.ct, S.pid, S.perm, S.rep, S.sid);
   }
 }
 
+template <int T, int ITEM>
 __device__ __forceinline__ void sort_item(const DevParams& P, const DeviceState& S,
                                           const SortPlan& plan, int phase, int item,
                                           int32_t* wsum) {
   switch (phase) {
-    case kKeys: sort_keys(P, S, item); break;
-    case kSums: sort_sums(P, S, item, wsum); break;
-    case kStarts: sort_starts(P, S, item, wsum); break;
+    case kKeys: sort_keys<T, ITEM>(P, S, item); break;
+    case kSums: sort_sums<T>(P, S, item, wsum); break;
+    case kStarts: sort_starts<T>(P, S, item, wsum); break;
     case kScatter:
       if (item == 0)
-        sort_rows(P, S, wsum);
+        sort_rows<T>(P, S, S.start, wsum);
       else
-        sort_scatter(P, S, item - 1);
+        sort_scatter<T, ITEM>(P, S, item - 1);
       break;
-    case kPlace: sort_place(P, S, item, plan.items[kPlace]); break;
-    default: sort_back(P, S, item); break;
+    case kPlace: sort_place<T, ITEM>(P, S, item, plan.items[kPlace]); break;
+    default: sort_back<T, ITEM>(P, S, item); break;
   }
 }
 
 // One launch per phase: for callers that may overlap on the same buffers
 // (k_sort_chain's counters would not survive that).
+template <int ITEM>
 __global__ __launch_bounds__(kSortThreads) void k_sort_phase(DevParams P, DeviceState S,
                                                              SortPlan plan, int phase) {
   __shared__ int32_t wsum[4];
-  sort_item(P, S, plan, phase, blockIdx.x, wsum);
+  sort_item<kSortThreads, ITEM>(P, S, plan, phase, blockIdx.x, wsum);
 }
 
 // Whether the lists are rebuilt this step: a particle moved more than skin / 2
@@ -415,6 +470,18 @@ __device__ __forceinline__ bool lists_outdated(const DevParams& P, const DeviceS
   return moved || S.gate[0] != 0;
 }
 
+// After a sort for Verlet lists.  gate[0]: the next density pass builds the
+// lists; gate[1] counts the builds; gate[2], set by the build, flags lists that
+// overflowed.
+__device__ __forceinline__ void set_gate(const DeviceState& S, bool moved) {
+  S.gate[0] = 1;
+  if (moved) {
+    S.gate[1] += 1;
+    S.gate[2] = 0;
+    S.disp[0] = 0ull;
+  }
+}
+
 // The whole sort in one launch.  Launched one by one its 13 kernels cost a
 // step 2.6 to 4.5 us each, most of a small box's step, and with Verlet lists
 // nearly all of those launches return at once (with the gate, the list flags
@@ -431,6 +498,7 @@ __device__ __forceinline__ bool lists_outdated(const DevParams& P, const DeviceS
 // mode 0: per-step lists.  1 (Verlet lists): sorts when the lists are
 // outdated.  2 (Verlet lists): sorts in any case.  advance: also one marching
 // step (nothing else here reads the step).
+template <int ITEM>
 __global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, DeviceState S,
                                                              SortPlan plan, int mode,
                                                              int advance) {
@@ -467,7 +535,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, Device
       }
       ready = phase - 1;
     }
-    sort_item(P, S, plan, phase, item, wsum);
+    sort_item<kSortThreads, ITEM>(P, S, plan, phase, item, wsum);
     // every wave's stores have reached the L2 before thread 0 writes it back
     // (a workgroup barrier alone does not wait for them)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -481,15 +549,115 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, Device
   if (atomicAdd(&ctl[7], 1) != (int)gridDim.x - 1) return;
   // the last workgroup: every other one has read what is written here
   for (int q = 0; q < 8; ++q) ctl[q] = 0;
-  if (mode == 0) return;
-  // gate[0]: the next density pass builds the lists; gate[1] counts the
-  // builds; gate[2], set by the build, flags lists that overflowed
-  S.gate[0] = 1;
-  if (moved) {
-    S.gate[1] += 1;
-    S.gate[2] = 0;
-    S.disp[0] = 0ull;
+  if (mode != 0) set_gate(S, moved);
+}
+
+// The sort of a small box: every workgroup counts all the cells for itself in
+// LDS, so that the phases up to the placing need no exchange, and places 256
+// particles; the last one to finish copies the state back.  Nothing waits, and
+// ctl[0] alone is shared.  64 x 64 particles: 20 us, 51 with k_sort_chain,
+// 39 with the whole sort in one workgroup (one CU's issue rate).
+// mode: k_sort_chain's, and without the gate 3 as 2, 4 as 0; keys_done: the
+// step boundary has counted the cells in S.count, which are cleared.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallPer = 4;
+constexpr int kSmallParticles = kSmallThreads * kSmallPer;
+constexpr int kSmallCellsPer = 8;
+constexpr int kSmallCells = kSmallThreads * kSmallCellsPer;
+constexpr int kSmallOwn = 256;
+__global__ __launch_bounds__(kSmallThreads) void k_sort_small(DevParams P, DeviceState S, int mode,
+                                                              int keys_done, int advance) {
+  __shared__ int32_t wsum[kSmallThreads / 64];
+  __shared__ int32_t start[kSmallCells + 1];
+  __shared__ int32_t unsorted[kSmallParticles];
+  __shared__ int32_t arrived;
+  const int tid = threadIdx.x;
+  const int64_t n = P.n;
+  bool moved = mode == 2;
+  if (advance && blockIdx.x == 0 && tid == 0) advance_step(S.step_dev, S.time_dev, P.dt);
+  if (mode == 1 && !lists_outdated(P, S, moved)) return;
+  double x[kSmallPer][3];
+  int32_t rep[kSmallPer], key[kSmallPer], slot[kSmallPer];
+#pragma unroll
+  for (int q = 0; q < kSmallPer; ++q) {
+    const int i = min(q * kSmallThreads + tid, P.n - 1);
+    rep[q] = S.rep[i];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) x[q][d] = d < P.dim ? S.x[d * n + i] : 0.0;
   }
+  // the particles that this workgroup places, 256 of its threads one each
+  constexpr int kOwners = kSmallThreads / kSmallOwn;
+  const int mine = (int)blockIdx.x / kOwners;  // which of a thread's particles
+  const int own = mine * kSmallThreads + tid;
+  const bool owner = tid / kSmallOwn == (int)blockIdx.x % kOwners && own < P.n;
+  Moved a;
+  if (owner) a = load_moved(P, own, S.x, S.v, S.m, S.ct, S.pid, S.perm, S.rep, S.sid);
+  for (int c = tid; c <= P.ncell; c += kSmallThreads) start[c] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSmallPer; ++q) {
+    key[q] = cell_key_geo(S.geo[rep[q]], P.dim, x[q][0], x[q][1], x[q][2]);
+    slot[q] = q * kSmallThreads + tid < P.n ? atomicAdd(&start[key[q]], 1) : 0;
+  }
+  __syncthreads();
+  {
+    int32_t v[kSmallCellsPer], local = 0, total;
+    const int c0 = tid * kSmallCellsPer;
+#pragma unroll
+    for (int u = 0; u < kSmallCellsPer; ++u) {
+      v[u] = c0 + u < P.ncell ? start[c0 + u] : 0;
+      local += v[u];
+    }
+    int32_t ex = block_scan<kSmallThreads>(local, total, wsum);
+#pragma unroll
+    for (int u = 0; u < kSmallCellsPer; ++u) {
+      if (c0 + u < P.ncell) {
+        start[c0 + u] = ex;
+        if (blockIdx.x == 0) S.start[c0 + u] = ex;
+      }
+      ex += v[u];
+    }
+    if (tid == 0) start[P.ncell] = total;
+    if (tid == 0 && blockIdx.x == 0) S.start[P.ncell] = total;
+  }
+  __syncthreads();
+  int32_t k = 0;
+#pragma unroll
+  for (int q = 0; q < kSmallPer; ++q) {
+    const int i = q * kSmallThreads + tid;
+    if (i < P.n) unsorted[start[key[q]] + slot[q]] = i;
+    if (q == mine) k = key[q];
+  }
+  if (blockIdx.x == 0) sort_rows<kSmallThreads>(P, S, start, wsum);
+  __syncthreads();
+  if (owner) {
+    const int s = start[k], e = start[k + 1];
+    int p = s;
+    for (int w = s; w < e; ++w) p += unsorted[w] < own ? 1 : 0;
+    const float4 xa = cell_record(P, S.geo[a.rep], k, a.x);
+    store_moved(P, p, a, S.x_alt, S.v_alt, S.m_alt, S.ct_alt, S.pid_alt, S.perm_alt, S.rep_alt,
+                S.sid_alt);
+    S.key_sorted[p] = k;
+    S.xa[p] = xa;
+    if (P.ncoll) S.slot_of[a.perm] = p;
+  }
+  // (as in k_sort_chain)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    arrived = __hip_atomic_fetch_add(&S.sort_ctl[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+  if (arrived != (int)gridDim.x - 1) return;
+  if (mode != 0 && mode != 4)
+    for (int q = 0; q < kSmallPer; ++q) sort_back<kSmallThreads, kSmallThreads>(P, S, q);
+  if (keys_done)
+    for (int c = tid; c < P.ncell; c += kSmallThreads) S.count[c] = 0;
+  if (tid != 0) return;
+  S.sort_ctl[0] = 0;
+  if (mode == 1 || mode == 2) set_gate(S, moved);
 }
 
 // ---------------------------------------------------------------------
@@ -545,6 +713,18 @@ void launch_fill_f64(hipStream_t s, double* a, double v, int64_t n) {
   hipLaunchKernelGGL(k_fill_f64, dim3(nb), dim3(256), 0, s, a, v, n);
 }
 
+static inline bool sort_small(const DevParams& P) {
+  return P.n <= kSmallParticles && P.ncell <= kSmallCells;
+}
+static inline dim3 small_grid(const DevParams& P) {
+  return dim3((P.n + kSmallOwn - 1) / kSmallOwn);
+}
+
+// Particles per item: 256 as long as that leaves the tickets few (32^3: 28
+// us for the six phases, 47 with 1024), 1024 beyond.
+constexpr int kSmallItem = 256, kLargeItem = 1024;
+constexpr int kSmallItems = 1 << 17;
+
 // Workgroups of the chain: up to four per CU, no more than its longest phase
 // has items.
 static inline dim3 sort_grid(const SortPlan& plan) {
@@ -557,18 +737,32 @@ void launch_sort(hipStream_t s, const DevParams& P, const DeviceState& S, SortKi
                  bool advance) {
   const bool keys = kind != SortKind::kStepKeysDone;
   const bool verlet = kind == SortKind::kVerletGated || kind == SortKind::kVerletForced;
-  const SortPlan plan = sort_plan(P, keys, verlet);
   const int mode = !verlet ? 0 : (kind == SortKind::kVerletGated ? 1 : 2);
-  hipLaunchKernelGGL(k_sort_chain, sort_grid(plan), dim3(kSortThreads), 0, s, P, S, plan, mode,
-                     advance ? 1 : 0);
+  if (sort_small(P)) {
+    hipLaunchKernelGGL(k_sort_small, small_grid(P), dim3(kSmallThreads), 0, s, P, S, mode,
+                       keys ? 0 : 1, advance ? 1 : 0);
+  } else if (P.n <= kSmallItems) {
+    const SortPlan plan = sort_plan(P, kSmallItem, keys, verlet);
+    hipLaunchKernelGGL(k_sort_chain<kSmallItem>, sort_grid(plan), dim3(kSortThreads), 0, s, P, S,
+                       plan, mode, advance ? 1 : 0);
+  } else {
+    const SortPlan plan = sort_plan(P, kLargeItem, keys, verlet);
+    hipLaunchKernelGGL(k_sort_chain<kLargeItem>, sort_grid(plan), dim3(kSortThreads), 0, s, P, S,
+                       plan, mode, advance ? 1 : 0);
+  }
 }
 
 void launch_sort_phases(hipStream_t s, const DevParams& P, const DeviceState& S, bool copy_back) {
-  const SortPlan plan = sort_plan(P, true, copy_back);
+  if (sort_small(P)) {
+    hipLaunchKernelGGL(k_sort_small, small_grid(P), dim3(kSmallThreads), 0, s, P, S,
+                       copy_back ? 3 : 4, 0, 0);
+    return;
+  }
+  const SortPlan plan = sort_plan(P, kSmallItem, true, copy_back);
   for (int p = 0; p < kSortPhases; ++p)
     if (plan.items[p] > 0)
-      hipLaunchKernelGGL(k_sort_phase, dim3(plan.items[p]), dim3(kSortThreads), 0, s, P, S, plan,
-                         p);
+      hipLaunchKernelGGL(k_sort_phase<kSmallItem>, dim3(plan.items[p]), dim3(kSortThreads), 0, s,
+                         P, S, plan, p);
 }
 
 void launch_reference_cells(hipStream_t s, const DevParams& P, const DeviceState& S) {

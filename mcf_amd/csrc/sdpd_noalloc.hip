@@ -126,6 +126,7 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   S.row_chunk_off = c.take<int32_t>(nrows + 1);
   S.chunk_row = c.take<int32_t>(nchunk);
   S.scan_tmp = c.take<int32_t>(ntile);
+  S.sort_ctl = c.take<int32_t>(8);
   S.nbr_count = c.take<int32_t>(N);
   S.nbr_in = c.take<int32_t>(N);
   S.recheck = c.take<int32_t>(N);
@@ -151,6 +152,7 @@ __global__ void k_na_ingest(RepGeom g, int32_t n, int32_t dim, int32_t nrows, in
     S.step_dev[0] = step;
     // (the times only serve sheared faces, which this entry lacks)
     for (int q = 0; q < 4; ++q) S.time_dev[q] = 0.0;
+    S.sort_ctl[0] = 0;
     S.gate[0] = 1;
     S.gate[1] = S.gate[2] = S.gate[3] = 0;
   }

@@ -56,3 +56,14 @@ def test_sort(oracle, shape, n, skin):
     assert np.abs(x - st.x).max() < 1e-10 * max(shape)
     assert vec_err(v, st.v) < 1e-10
     assert vec_err(f, st.f) < 1e-10
+
+
+@pytest.mark.parametrize("shape,n", [((17, 16), 255), ((17, 16), 256), ((17, 16), 257),
+                                     ((33, 33), 1025), ((64, 64), 4096), ((65, 64), 4097),
+                                     ((16, 16, 17), 4096), ((50, 50, 50), 4000),
+                                     ((56, 57, 60), 4000)])
+@pytest.mark.parametrize("skin", [0.0, 1e-9])
+def test_small_sort(oracle, shape, n, skin):
+    # k_sort_small where its 256 particles per workgroup, its four particles
+    # per thread and its cells in LDS end
+    test_sort(oracle, shape, n, skin)
