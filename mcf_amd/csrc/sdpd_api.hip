@@ -527,9 +527,7 @@ int alloc_state(sdpd_ctx* c, int n) {
   ALLOC(gate, 4);
   ALLOC(disp, 1);
   if (P.verlet) ALLOC(x_ref, dim * N);
-  // neighbour lists: one block of list_cap x 64 entries per chunk of the
-  // sort grid (at most N / 64 + rows chunks, rounded up to 8)
-  ALLOC(nlist, (size_t)P.list_cap * 64 * (((N + 63) / 64 + (size_t)P.nrows + 7) / 8 * 8));
+  ALLOC(nlist, sdpd::list_entries(P, n));
   ALLOC(recheck, N);
   ALLOC(nbr_hash, N);
   if (P.ncoll > 0) {

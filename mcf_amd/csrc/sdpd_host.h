@@ -17,6 +17,11 @@ int derive_params(const sdpd_params& p, DevParams& P, const char*& err);
 // five sort-grid cells is at most mmax.
 void set_cut_band(DevParams& P, double mmax);
 
+// Entries of the stored neighbour lists of n particles: the blocks' and those
+// that the last block's walk may read past it.
+inline size_t list_entries(const DevParams& P, int64_t n) {
+  return (size_t)P.list_cap * (size_t)n + 8 * 64;
+}
 // Automatic capacity of the stored neighbour lists for n particles in the
 // given volume (the cut-off sphere plus the Verlet skin).
 int auto_list_capacity(const DevParams& P, double volume, int64_t n);

@@ -130,11 +130,30 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   S.nbr_count = c.take<int32_t>(N);
   S.nbr_in = c.take<int32_t>(N);
   S.recheck = c.take<int32_t>(N);
-  S.nlist = c.take<uint32_t>((size_t)P.list_cap * 64 * ((nchunk + 7) / 8 * 8));
+  S.nlist = c.take<uint32_t>(sdpd::list_entries(P, P.n));
   S.gate = c.take<int32_t>(4);
   S.disp = c.take<unsigned long long>(1);
-  if (P.verlet) S.x_ref = c.take<double>(dim * N);
   return c.used;
+}
+
+// The bytes by which a box is refused: those of lists of capacity 8 in blocks
+// of whole chunks, with their rows' counters, and of reference positions.
+// carve_state takes no more at that capacity.
+size_t bytes_asked(DevParams P) {
+  P.list_cap = 8;
+  DeviceState S{};
+  const size_t N = (size_t)P.n, nrows = (size_t)P.nrows;
+  Carver with{nullptr}, without{nullptr};
+  with.take<uint32_t>((size_t)8 * 64 * (((N + 63) / 64 + nrows + 7) / 8 * 8));
+  with.take<int32_t>(nrows);
+  if (P.verlet) with.take<double>((size_t)P.dim * N);
+  without.take<uint32_t>(sdpd::list_entries(P, P.n));
+  without.take<int32_t>(8);
+  if (P.mixed) {
+    without.take<uint4>(N);
+    without.take<float>(N);
+  }
+  return carve_state(nullptr, P, S) + with.used - without.used;
 }
 
 // Geometry tables of the single box: its RepGeom and, per row of the sort
@@ -233,16 +252,18 @@ extern "C" int sdpd_evaluate_noalloc(const sdpd_params* params, int64_t step, co
   double volume = 1.0;
   for (int d = 0; d < P.dim; ++d) volume *= P.length[d];
 
-  // the automatic list capacity, smaller if the array cannot hold it (any
-  // capacity gives the same results: chunks whose lists overflow are
-  // scanned again by the force pass)
+  // the automatic list capacity, or the largest that the array can hold (any
+  // capacity gives the same results: chunks whose lists overflow are scanned
+  // again)
   DeviceState S{};
-  P.list_cap = sdpd::auto_list_capacity(P, volume, n);
-  while (carve_state(nullptr, P, S) > kScratchBytes && P.list_cap > 8)
-    P.list_cap = std::max(8, (P.list_cap / 2 + 7) / 8 * 8);
-  if (carve_state(nullptr, P, S) > kScratchBytes)
+  P.list_cap = 8;
+  const size_t least = carve_state(nullptr, P, S);
+  if (bytes_asked(P) > kScratchBytes || least > kScratchBytes)
     return reject(SDPD_ERR_ARG,
                   "the box needs more than the 32 MiB scratch array (too many particles or cells)");
+  const size_t room = (kScratchBytes - least) / (8 * sizeof(uint32_t) * (size_t)n);
+  P.list_cap = std::min(sdpd::auto_list_capacity(P, volume, n), 8 + 8 * (int)std::min<size_t>(room, 512));
+  while (P.list_cap > 8 && carve_state(nullptr, P, S) > kScratchBytes) P.list_cap -= 8;
 
   unsigned char* base = nullptr;
   if ((rc = scratch_address(&base)) != SDPD_OK) return reject(rc, "no scratch array on this device");

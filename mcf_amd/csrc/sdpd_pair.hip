@@ -365,16 +365,18 @@ __device__ __forceinline__ bool load_chunk(const DevParams& P, const DeviceState
   return true;
 }
 
-// Neighbour list block of a chunk: list_cap / 8 groups, each 64 lanes x 8
-// entries; a lane's group g holds its entries 8g .. 8g+7.  Verlet lists
-// store them as (0, 4), (1, 5), (2, 6), (3, 7): four lanes walk a particle's
-// list, lane s takes the entries s and s + 4 of a group in one 8-byte load,
-// and a wave's 64 loads are contiguous.
+// Neighbour list block of a chunk of m particles: list_cap / 8 groups, each m
+// lanes x 8 entries; a lane's group g holds its entries 8g .. 8g+7.  Verlet
+// lists store them as (0, 4), (1, 5), (2, 6), (3, 7): four lanes walk a
+// particle's list, lane s takes the entries s and s + 4 of a group in one
+// 8-byte load, and a wave's 64 loads are contiguous.  The blocks follow the
+// particles without padding (list_entries: the last lanes of the last block
+// may read, not use, entries past it).
 __device__ __forceinline__ uint32_t* list_block(const DevParams& P, uint32_t* list, const Chunk& ch) {
-  return list + (int64_t)ch.c * P.list_cap * kWave;
+  return list + (int64_t)ch.p0 * P.list_cap;
 }
-__device__ __forceinline__ int64_t group_offset(int q, int lane) {
-  return ((int64_t)(q >> 3) * kWave + lane) * 8;
+__device__ __forceinline__ int64_t group_offset(const Chunk& ch, int q, int lane) {
+  return ((q >> 3) * (ch.p1 - ch.p0) + lane) * 8;
 }
 
 template <int DIM>
@@ -598,7 +600,7 @@ __device__ __forceinline__ int staged_scan(const DevParams& P, const DeviceState
           hi.y = buf[(q + (SKIN ? 6 : 5)) * kWave + lane];
           hi.z = buf[(q + (SKIN ? 3 : 6)) * kWave + lane];
           hi.w = buf[(q + 7) * kWave + lane];
-          uint4* dst = reinterpret_cast<uint4*>(blk + group_offset(stored + q, lane));
+          uint4* dst = reinterpret_cast<uint4*>(blk + group_offset(ch, stored + q, lane));
           dst[0] = lo;
           dst[1] = hi;
         }
@@ -718,6 +720,184 @@ __device__ __forceinline__ int staged_scan(const DevParams& P, const DeviceState
   return stored;
 }
 
+// The scan of a list build: the entries of staged_scan with SKIN, in the same
+// order, stored and not evaluated (the walk of the same step does that).
+// A wave per chunk leaves small boxes a chain of latencies, so nothing waits
+// within a row: lane r looks up stencil row r before the first one starts, and
+// a row's records and window bounds load while the row before is scanned.
+// A build without its sums takes 83 us instead of 185 in a 32^3 box (mixed
+// precision) and 0.97 ms instead of 2.2 in the 128^3 one (1.53 with the
+// registers of two waves per SIMD); the walk adds 22 us and 0.58 ms.
+// tile holds TILE + 3 records (the last three only serve lanes past their
+// window).
+template <int DIM, bool IMAGES, int TILE, int BUF>
+__device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& S,
+                                         const Chunk& ch, const Home& h,
+                                         float4* __restrict__ tile, uint32_t* __restrict__ buf,
+                                         uint32_t* __restrict__ blk) {
+  constexpr int kRows = DIM == 3 ? 25 : 5;
+  constexpr int kAhead = (TILE + kWave - 1) / kWave;  // records per lane of a row's first batch
+  constexpr int kStep = 4;                            // candidates per lane and pass
+  constexpr int kRing = (BUF + 7) / 8 * 8;            // rows of buf: a ring of whole groups
+  static_assert((kRing & (kRing - 1)) == 0 && kRing >= 8 + kStep, "");
+  const int lane = threadIdx.x;
+  const int nm0 = h.G.nm0;
+  const int32_t* __restrict__ start = S.start;
+  const uint32_t self_flag = (IMAGES && P.ncoll && S.sid[h.ii] != 0) ? kBoundaryBit : 0u;
+  const RowPieces mine = row_pieces<DIM>(P, S, ch, h, lane < kRows ? lane : kRows - 1);
+  auto row_of = [&](int row) {
+    RowPieces rp;
+    auto get = [&](int v) { return __builtin_amdgcn_readlane(v, row); };
+    rp.rb = get(mine.rb);
+    rp.my = get(mine.my);
+    rp.mz = get(mine.mz);
+    rp.sigma = get(mine.sigma);
+    rp.vlo = get(mine.vlo);
+    rp.a1 = get(mine.a1);
+    rp.a2 = get(mine.a2);
+    rp.aend = get(mine.aend);
+    rp.m0 = get(mine.m0);
+    rp.g0 = get(mine.g0);
+    rp.len0 = get(mine.len0);
+    rp.g1 = get(mine.g1);
+    rp.len1 = get(mine.len1);
+    rp.g2 = get(mine.g2);
+    rp.len2 = get(mine.len2);
+    rp.tot = get(mine.tot);
+    return rp;
+  };
+  // a record of the row's sequence with its entry, ready for the tile
+  struct Rec {
+    float4 q;
+    int sid;
+  };
+  auto fetch = [&](const RowPieces& rp, int t) {
+    const int g = seq_particle(rp, min(t, rp.tot - 1));
+    Rec r;
+    r.q = S.xa[g];
+    r.sid = (IMAGES && P.ncoll) ? S.sid[g] : 0;
+    return r;
+  };
+  auto place = [&](const RowPieces& rp, int t, const Rec& r, float4* __restrict__ to) {
+    const int g = seq_particle(rp, t);
+    const int piece = t < rp.len0 ? 0 : (t < rp.len0 + rp.len1 ? 1 : 2);
+    const int v = __float_as_int(r.q.w) + (rp.m0 + piece) * nm0;
+    const int vrel = v - rp.vlo;
+    uint32_t code = IMAGES ? image_field(v, nm0, 0) : (uint32_t)vrel << kCodeShift;
+    if (IMAGES && P.ncoll && r.sid != 0) code |= kBoundaryBit;
+    *to = make_float4(fmaf((float)vrel, h.G.cs0, r.q.x), r.q.y, r.q.z,
+                      __uint_as_float((uint32_t)g | code));
+  };
+  // the lane's entries so far, and those of them (whole groups of 8) in its
+  // list; entry q waits in row q mod kRing of buf
+  int cnt = 0, stored = 0;
+  auto flush = [&](int least) {
+    if (cnt - stored >= least) {
+      if (stored + 8 <= P.list_cap) {
+        const uint32_t* __restrict__ from = buf + (stored & (kRing - 1)) * kWave + lane;
+        // (pairs for the four-lane walk)
+        uint4 lo, hi;
+        lo.x = from[0 * kWave];
+        lo.y = from[4 * kWave];
+        lo.z = from[1 * kWave];
+        lo.w = from[5 * kWave];
+        hi.x = from[2 * kWave];
+        hi.y = from[6 * kWave];
+        hi.z = from[3 * kWave];
+        hi.w = from[7 * kWave];
+        uint4* dst = reinterpret_cast<uint4*>(blk + group_offset(ch, stored, lane));
+        dst[0] = lo;
+        dst[1] = hi;
+      }
+      stored += 8;
+    }
+  };
+  // what a row needs, loaded while the row before is scanned
+  RowPieces rp = row_of(0);
+  Rec ahead[kAhead];
+  int wc = 0, tb = 0, te = 0;
+  auto prepare = [&]() {
+    wc = rp.sigma >= 0 ? h.le.wc(rp.sigma) : h.cx;
+    // this lane's window: virtual cells wc-2 .. wc+2 as a range of the row
+    // sequence
+    tb = te = 0;
+    if (h.active) {
+      tb = seq_of(rp, start, nm0, wc - 2);
+      te = seq_of(rp, start, nm0, wc + 3);
+    }
+    if (rp.tot > 0) {
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) ahead[k] = fetch(rp, lane + k * kWave);
+    }
+  };
+  prepare();
+#pragma unroll 1
+  for (int row = 0; row < kRows; ++row) {
+    const RowPieces now = rp;
+    const int wc_now = wc, tb_now = tb, te_now = te;
+    const int dy = row % 5 - 2, dz = DIM == 3 ? row / 5 - 2 : 0;
+    // Positions in the tile are relative to the corner of virtual cell vlo in
+    // x and to the candidate's own cell in y and z (staged_scan).
+    const bool le_row = now.sigma >= 0;
+    const int crel = wc_now - now.vlo;
+    const float ax = (le_row ? h.a.x + h.le.dxf(now.sigma) : h.a.x) + (float)crel * h.G.cs0;
+    const uint32_t self_w =
+        le_row ? 0xFFFFFFFFu
+               : (IMAGES ? ((uint32_t)h.ii | self_flag)
+                         : ((uint32_t)h.ii | ((uint32_t)crel << kCodeShift)));
+    const float ay = h.a.y - (float)dy * h.G.cs1;
+    const float az = DIM == 3 ? h.a.z - (float)dz * h.G.cs2 : 0.f;
+    const uint32_t kadd =
+        IMAGES
+            ? image_field(h.cy + dy, h.G.nm1, 1) | (DIM == 3 ? image_field(h.cz + dz, h.G.nm2, 2) : 0u)
+            : (uint32_t)(2 - crel + 5 * (dy + 2) + 25 * (dz + 2)) << kCodeShift;
+    for (int base = 0; base < now.tot; base += TILE) {
+      const int bend = min(now.tot, base + TILE);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int t = base + lane + k * kWave;
+        if (k * kWave + lane < TILE && t < bend) {
+          if (base > 0) ahead[k] = fetch(now, t);
+          place(now, t, ahead[k], tile + (t - base));
+        }
+      }
+      __syncthreads();
+      if (bend == now.tot && row + 1 < kRows) {
+        rp = row_of(row + 1);
+        prepare();
+      }
+      const int lb = max(tb_now, base) - base, le = min(te_now, bend) - base;
+      for (int t = lb; __ballot(t < le) != 0ull; t += kStep) {
+        if (__ballot(cnt - stored > kRing - kStep) != 0ull) flush(8);
+        const float4* __restrict__ tp = tile + min(t, TILE - 1);
+#pragma unroll
+        for (int u = 0; u < kStep; ++u) {
+          const float4 q = tp[u];
+          const uint32_t wv = __float_as_uint(q.w);
+          const float d0 = ax - q.x;
+          const float d1 = ay - q.y;
+          float s2 = fmaf(d1, d1, d0 * d0);
+          if (DIM == 3) {
+            const float d2 = az - q.z;
+            s2 = fmaf(d2, d2, s2);
+          }
+          // (written in any case: the next entry overwrites it unless it counts)
+          buf[(cnt & (kRing - 1)) * kWave + lane] = wv + kadd;
+          cnt += (t + u < le && wv != self_w && s2 < P.skin2_hi_f32) ? 1 : 0;
+        }
+      }
+      __syncthreads();
+    }
+    if (now.tot == 0 && row + 1 < kRows) {
+      rp = row_of(row + 1);
+      prepare();
+    }
+  }
+  flush(8);
+  flush(1);
+  return cnt;
+}
+
 // FP32 terms summed in FP64 (each add rounds once, at FP64 precision)
 struct WideF {
   double s = 0.0;
@@ -800,7 +980,7 @@ struct DensityF64 {
   int nin = 0, rechecks = 0;
   static constexpr bool kImages = true;
   static constexpr bool kBatched = DECIDE;
-  static constexpr int kBatch = 8;
+  static constexpr int kBatch = 2;  // (larger ones cost the scan kernels registers)
   static constexpr int kTerms = 1;
   static constexpr int kWalk = 4;
   __device__ __forceinline__ void body(uint32_t ent) {
@@ -960,7 +1140,7 @@ struct DensityMixed {
   int nin = 0, rechecks = 0;
   static constexpr bool kImages = false;
   static constexpr bool kBatched = true;
-  static constexpr int kBatch = 8;
+  static constexpr int kBatch = 2;  // (larger ones cost the scan kernels registers)
   static constexpr int kTerms = 1;
   static constexpr int kWalk = 4;
   struct Rec {
@@ -1115,7 +1295,7 @@ __device__ __forceinline__ void for_each_listed(const DevParams& P, const Device
       // padding inside the row and are not evaluated.  The group goes to
       // LDS (entry u of a lane at buf[u * 64 + lane], conflict-free), and
       // the loop reads one entry per pair, the next one ahead of the body.
-      const uint4* src = reinterpret_cast<const uint4*>(blk + group_offset(q, lane));
+      const uint4* src = reinterpret_cast<const uint4*>(blk + group_offset(ch, q, lane));
       const uint4 lo = src[0], hi = src[1];
       buf[0 * kWave + lane] = lo.x;
       buf[1 * kWave + lane] = lo.y;
@@ -1187,12 +1367,12 @@ __device__ __forceinline__ void walk_quarter(const DevParams& P, const DeviceSta
   if (s == 0) sum[0] = start;
   // the next batch's entries are loaded behind the current batch's gathers,
   // without a branch (a group past the list's capacity reads its last one)
-  const int last = (P.list_cap >> 3) - 1;
+  const int last = (P.list_cap >> 3) - 1, stride = (ch.p1 - ch.p0) * 8;
   uint2 nx[NB / 2];
   auto fetch = [&](int q) {
 #pragma unroll
     for (int g = 0; g < NB / 2; ++g)
-      nx[g] = *reinterpret_cast<const uint2*>(src + (int64_t)min((q >> 3) + g, last) * (8 * kWave));
+      nx[g] = *reinterpret_cast<const uint2*>(src + min((q >> 3) + g, last) * stride);
   };
   fetch(0);
   for (int q = 0; __ballot(q < cnt) != 0ull; q += 4 * NB) {
@@ -1288,11 +1468,12 @@ __device__ __forceinline__ bool chunk_meets_le_face(int le_g, const Chunk& ch, i
 //
 // Modes.  kStore: the in-cut-off pairs found by the candidate scan are
 // summed and stored (lists rebuilt every step).  Verlet lists decide the
-// cut-off per candidate on the current positions: kScan scans the stencil,
-// on steps whose gate asks for it for every chunk, storing the candidates
-// within rc + skin, and on the others for the chunks whose lists overflowed,
-// without storing (k_density_walk takes the rest); kScanAll does the latter
-// for every chunk (autotune's timing of the scan).
+// cut-off per candidate on the current positions: k_density_walk walks the
+// lists of the chunks that hold them all, and kScan, before it, stores the
+// candidates within rc + skin of every chunk on steps whose gate asks for it,
+// and scans the stencil for the sums of the chunks whose lists overflowed;
+// kScanAll does the latter for every chunk (the autotuner).  The walk and the
+// scans visit the candidates in the same order, so they give the same sums.
 enum DensityMode { kStore = 0, kScan = 1, kScanAll = 2 };
 
 // Density epilogue of particle i with number (or mass) density sum rho.
@@ -1343,8 +1524,18 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
   if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
   if (MODE == kScan && !build && !list_overflow(P, S, ch)) return;
   const Home h = load_home<DIM>(P, S, ch);
+  if (MODE == kScan && build) {
+    const int cnt = list_scan<DIM, !MIXED, TILE, BUF>(P, S, ch, h, tile, buf,
+                                                      list_block(P, S.nlist, ch));
+    if (h.active) S.nbr_count[h.i] = cnt;
+    // the shear time of the build (the copies across sheared faces drift
+    // from their build positions as it advances)
+    if (h.active && h.i == 0) S.time_dev[3] = S.time_dev[1];
+    if (__ballot(h.active && cnt > P.list_cap) == 0ull) return;
+    if (threadIdx.x == 0) S.gate[2] = 1;  // every writer stores 1
+  }
   const double mi = S.m[h.ii];
-  uint32_t* list = (MODE == kStore || (MODE == kScan && build)) ? S.nlist : nullptr;
+  uint32_t* list = MODE == kStore ? S.nlist : nullptr;
   using Pol = std::conditional_t<
       MIXED, std::conditional_t<kDecide, DensityMixed<DIM>, DensityMixedStep<DIM>>,
       DensityF64<DIM, kDecide>>;
@@ -1363,11 +1554,7 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
     rho = density_of<MIXED>(P, pol.acc);
   if (!h.active) return;
   const int i = h.i;
-  if (MODE == kStore || (MODE == kScan && build)) S.nbr_count[i] = cnt;
-  if (MODE == kScan && build && cnt > P.list_cap) S.gate[2] = 1;  // every writer stores 1
-  // the shear time of the build (the copies across sheared faces drift
-  // from their build positions as it advances)
-  if (MODE == kScan && build && i == 0) S.time_dev[3] = S.time_dev[1];
+  if (MODE == kStore) S.nbr_count[i] = cnt;
   finish_density<DIM>(P, S, i, mi, rho, kDecide ? pol.nin : cnt, rechecks + pol.rechecks);
 }
 
@@ -1379,7 +1566,8 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
 // constants, so the batch's terms carry no branches.
 template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ>
 __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState S) {
-  if (S.gate[0] != 0) return;
+  // the lists are current
+  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
   __shared__ __align__(16) double lds[kTermWords<1>];
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
@@ -1426,12 +1614,12 @@ __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState
 // workgroups take every gridDim.x-th chunk slot, so that on the other steps
 // the launch is cheap.
 template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
-__global__ __launch_bounds__(kWave) void k_density(DevParams P, DeviceState S) {
+__global__ __launch_bounds__(kWave, MODE == kScan ? 4 : 1) void k_density(DevParams P, DeviceState S) {
   const bool build = MODE == kScan && S.gate[0] != 0;
   if (MODE == kScan && !build && S.gate[2] == 0) return;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
-  __shared__ float4 tile[TILE + 1];
+  __shared__ float4 tile[TILE + 3];
   // whole groups of 8 rows: the final flush stores the last group of a
   // lane's entries as 8 rows, of which those past its count are padding
   __shared__ uint32_t buf[(BUF + 7) / 8 * 8 * kWave];
@@ -2442,8 +2630,6 @@ enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
 // code decode and compensated FP32 sums, one particle per lane).
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC>
 __global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? 6 : 1)) void k_force_walk(DevParams P, DeviceState S) {
-  // the density pass has built the lists that were due
-  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (SPEC != kAny) {
@@ -2598,16 +2784,15 @@ static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceSt
     launch_density_shape<DIM, MIXED, false, kScanAll>(s, P, S);
     return;
   }
-  // Verlet lists: the gate and the overflow flag decide which of the two
-  // kernels takes a chunk; a box with sheared faces splits the chunks between
+  // Verlet lists: a box with sheared faces splits the chunks between
   // the Lees-Edwards and the plain instantiations, as its per-step lists do
   if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
-    if (P.le_g >= 0) {
-      launch_density_shape<DIM, MIXED, true, kScan>(s, P, S);
-      launch_density_walk<DIM, MIXED, true>(s, P, S);
-    }
+    if (P.le_g >= 0) launch_density_shape<DIM, MIXED, true, kScan>(s, P, S);
   }
   launch_density_shape<DIM, MIXED, false, kScan>(s, P, S);
+  if constexpr (!MIXED) {
+    if (P.le_g >= 0) launch_density_walk<DIM, MIXED, true>(s, P, S);
+  }
   launch_density_walk<DIM, MIXED, false>(s, P, S);
 }
 
