@@ -110,8 +110,9 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   if (P.mixed) {
     S.vr = c.take<float4>(N);
     S.qr = c.take<float4>(N);
-    S.xq = c.take<uint4>(N);
-    S.an32 = c.take<float>(N);
+    // (both of Verlet lists only; the cell keys are spent after the sort)
+    S.xq = c.take<uint4>(P.verlet ? N : 0);
+    S.an32 = reinterpret_cast<float*>(S.key);
   } else {
     S.rec64 = c.take<double>(8 * N);
   }
@@ -149,10 +150,7 @@ size_t bytes_asked(DevParams P) {
   if (P.verlet) with.take<double>((size_t)P.dim * N);
   without.take<uint32_t>(sdpd::list_entries(P, P.n));
   without.take<int32_t>(8);
-  if (P.mixed) {
-    without.take<uint4>(N);
-    without.take<float>(N);
-  }
+  if (P.mixed) without.take<uint4>(P.verlet ? N : 0);
   return carve_state(nullptr, P, S) + with.used - without.used;
 }
 
