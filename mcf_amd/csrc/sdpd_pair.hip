@@ -722,17 +722,25 @@ __device__ __forceinline__ int staged_scan(const DevParams& P, const DeviceState
 
 // The scan of a list build: the entries of staged_scan with SKIN, in the same
 // order, stored and not evaluated (the walk of the same step does that).
+// LANES: with 1 a wave takes the chunk, a lane per particle.  With 4 it takes 16
+// of the chunk's particles (ch is cut to them), and four lanes test four
+// candidates of a particle at a time; a ballot gives each its place, so the
+// entries stand in the same order.  stride, own: particles of the chunk and the
+// lane's particle among them (the layout of the lists).
+//
 // A wave per chunk leaves small boxes a chain of latencies, so nothing waits
 // within a row: lane r looks up stencil row r before the first one starts, and
 // a row's records and window bounds load while the row before is scanned.
 // A build without its sums takes 83 us instead of 185 in a 32^3 box (mixed
 // precision) and 0.97 ms instead of 2.2 in the 128^3 one (1.53 with the
 // registers of two waves per SIMD); the walk adds 22 us and 0.58 ms.
-// tile holds TILE + 3 records (the last three only serve lanes past their
-// window).
-template <int DIM, bool IMAGES, int TILE, int BUF>
+// tile holds TILE + kTilePad<LANES> records (the last ones only serve lanes
+// past their window).
+template <int LANES>
+constexpr int kTilePad = LANES == 4 ? 7 : 3;
+template <int DIM, bool IMAGES, int TILE, int BUF, int LANES = 1>
 __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& S,
-                                         const Chunk& ch, const Home& h,
+                                         const Chunk& ch, const Home& h, int stride, int own,
                                          float4* __restrict__ tile, uint32_t* __restrict__ buf,
                                          uint32_t* __restrict__ blk) {
   constexpr int kRows = DIM == 3 ? 25 : 5;
@@ -741,6 +749,17 @@ __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& 
   constexpr int kRing = (BUF + 7) / 8 * 8;            // rows of buf: a ring of whole groups
   static_assert((kRing & (kRing - 1)) == 0 && kRing >= 8 + kStep, "");
   const int lane = threadIdx.x;
+  // four lanes per particle: buf holds kDeep entries of each of 16 particles
+  constexpr int kDeep = 4 * kRing;
+  const int part = lane >> 2, sub = lane & 3;
+  // the waves of a workgroup share nothing here (one wave: LDS operations
+  // complete in order)
+  auto sync = [&]() {
+    if constexpr (LANES == 1)
+      __syncthreads();
+    else
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
   const int nm0 = h.G.nm0;
   const int32_t* __restrict__ start = S.start;
   const uint32_t self_flag = (IMAGES && P.ncoll && S.sid[h.ii] != 0) ? kBoundaryBit : 0u;
@@ -792,6 +811,20 @@ __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& 
   // list; entry q waits in row q mod kRing of buf
   int cnt = 0, stored = 0;
   auto flush = [&](int least) {
+    if constexpr (LANES == 4) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      while (__ballot(cnt - stored >= least) != 0ull) {
+        if (cnt - stored >= least) {
+          if (stored + 8 <= P.list_cap)
+            *reinterpret_cast<uint2*>(blk + ((stored >> 3) * stride + own) * 8 + 2 * sub) =
+                make_uint2(buf[((stored + sub) & (kDeep - 1)) * 16 + part],
+                           buf[((stored + sub + 4) & (kDeep - 1)) * 16 + part]);
+          stored += 8;
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      return;
+    }
     if (cnt - stored >= least) {
       if (stored + 8 <= P.list_cap) {
         const uint32_t* __restrict__ from = buf + (stored & (kRing - 1)) * kWave + lane;
@@ -805,7 +838,7 @@ __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& 
         hi.y = from[6 * kWave];
         hi.z = from[3 * kWave];
         hi.w = from[7 * kWave];
-        uint4* dst = reinterpret_cast<uint4*>(blk + group_offset(ch, stored, lane));
+        uint4* dst = reinterpret_cast<uint4*>(blk + ((stored >> 3) * stride + own) * 8);
         dst[0] = lo;
         dst[1] = hi;
       }
@@ -861,12 +894,36 @@ __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& 
           place(now, t, ahead[k], tile + (t - base));
         }
       }
-      __syncthreads();
+      sync();
       if (bend == now.tot && row + 1 < kRows) {
         rp = row_of(row + 1);
         prepare();
       }
       const int lb = max(tb_now, base) - base, le = min(te_now, bend) - base;
+      if constexpr (LANES == 4) {
+        for (int t = lb; __ballot(t < le) != 0ull; t += 8) {
+          if (__ballot(cnt - stored > kDeep - 8) != 0ull) flush(8);
+          const float4* __restrict__ tp = tile + min(t, TILE - 1) + sub;
+          const float4 qq[2] = {tp[0], tp[4]};
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const float4 q = qq[u];
+            const uint32_t wv = __float_as_uint(q.w);
+            const float d0 = ax - q.x;
+            const float d1 = ay - q.y;
+            float s2 = fmaf(d1, d1, d0 * d0);
+            if (DIM == 3) {
+              const float d2 = az - q.z;
+              s2 = fmaf(d2, d2, s2);
+            }
+            const bool in = t + 4 * u + sub < le && wv != self_w && s2 < P.skin2_hi_f32;
+            const uint32_t four = (uint32_t)(__ballot(in) >> (lane & 60)) & 15u;
+            if (in)
+              buf[((cnt + __popc(four & ((1u << sub) - 1u))) & (kDeep - 1)) * 16 + part] = wv + kadd;
+            cnt += __popc(four);
+          }
+        }
+      } else
       for (int t = lb; __ballot(t < le) != 0ull; t += kStep) {
         if (__ballot(cnt - stored > kRing - kStep) != 0ull) flush(8);
         const float4* __restrict__ tp = tile + min(t, TILE - 1);
@@ -886,7 +943,7 @@ __device__ __forceinline__ int list_scan(const DevParams& P, const DeviceState& 
           cnt += (t + u < le && wv != self_w && s2 < P.skin2_hi_f32) ? 1 : 0;
         }
       }
-      __syncthreads();
+      sync();
     }
     if (now.tot == 0 && row + 1 < kRows) {
       rp = row_of(row + 1);
@@ -1318,49 +1375,59 @@ __device__ __forceinline__ void for_each_listed(const DevParams& P, const Device
 }
 
 // ---------------------------------------------------------------------
-// the walk of Verlet lists: four lanes per particle
+// the walk of Verlet lists: four or sixteen lanes per particle
 // ---------------------------------------------------------------------
-// A wave takes 16 consecutive particles of a chunk (a "quarter"), lane
-// 4 p + s every fourth entry of particle p.  Against one particle per lane,
+// A wave takes 64 / LANES consecutive particles of a chunk (a "part"), a lane
+// every LANES-th entry of one particle.  Against one particle per lane,
 // neighbouring lanes gather neighbouring list entries (fewer lines per
-// gather), a wave runs as long as the longest of 16 lists instead of 64,
-// and a small box has four times the waves, each a quarter as long.
+// gather), a wave runs as long as the longest of 16 (4) lists instead of 64,
+// and a small box has 4 (16) times the waves, each as much shorter.
 //
-// The terms are still added in list order: a group's four lanes put their
-// terms into LDS, and lane s adds component s (4 + s, 8 + s) of its particle's
-// four entries one after another.  So a particle's sum does not depend on
-// where its in-cut-off pairs stand among the candidates, and equals the
-// one-particle-per-lane sums of the candidate scans bit for bit.  Four FP64
-// adds per four components and group; the matrix cores' v_mfma_f64_4x4x4
-// (an fma chain over k, the same order) takes 4 CU cycles per component, and
-// on the 128^3 box the force walk took 1.54 ms with it.
-constexpr int kQuarter = 16;
+// The terms are still added in list order: a group's lanes put their terms
+// into LDS, and lane s of a particle adds component s (with four lanes also
+// 4 + s, 8 + s) of its entries one after another.  So a particle's sum does not
+// depend on where its in-cut-off pairs stand among the candidates, and equals
+// the one-particle-per-lane sums of the candidate scans bit for bit.  With four
+// lanes four FP64 adds per four components and 64 entries; the matrix cores'
+// v_mfma_f64_4x4x4 (an fma chain over k, the same order) takes 4 CU cycles per
+// component, and on the 128^3 box the force walk took 1.54 ms with it.  With
+// sixteen lanes 16 adds per 64 entries, and a prologue for every 4 particles.
+template <int LANES>
+constexpr int kPart = kWave / LANES;  // particles of a wave
 // a component's row of 64 lanes' terms: 66 doubles, so that the 16-byte reads
 // of the four lanes' rows fall on different banks
 constexpr int kTermRow = 66;
 template <int TERMS>
-constexpr int kTermWords = (TERMS + 3) / 4 * 4 * kTermRow;
+constexpr int kTermRows = (TERMS + 3) / 4 * 4 * kTermRow;
+// (sixteen lanes: entries 0 .. 3 of the groups and entries 4 .. 7)
+template <int TERMS, int LANES>
+constexpr int kTermWords = kTermRows<TERMS> * (LANES == 16 ? 2 : 1);
 
-// the sums of the 16 particles after the walk: component c of particle p
-__device__ __forceinline__ double& quarter_sum(double* lds, int p, int c) {
+// the sums of a wave's particles after the walk: component c of particle p
+__device__ __forceinline__ double& part_sum(double* lds, int p, int c) {
   return lds[c * kTermRow + p];
 }
 
-// start: what the sum of component 0 starts from (lane 4 p).  Leaves the sums
-// in lds (quarter_sum).
-template <int DIM, class Pol>
-__device__ __forceinline__ void walk_quarter(const DevParams& P, const DeviceState& S,
-                                             const Chunk& ch, int quarter, const Home& h, Pol& pol,
-                                             double start, double* __restrict__ lds) {
-  constexpr int NB = Pol::kWalk;  // entries per lane and batch (even)
-  constexpr int T = Pol::kTerms, M = (T + 3) / 4;
+// start: what the sum of component 0 starts from (a particle's first lane).
+// Leaves the sums in lds (part_sum).
+template <int DIM, int LANES, class Pol>
+__device__ __forceinline__ void walk_part(const DevParams& P, const DeviceState& S,
+                                          const Chunk& ch, int part, const Home& h, Pol& pol,
+                                          double start, double* __restrict__ lds) {
+  static_assert(LANES == 4 || LANES == 16, "");
+  constexpr int NB = LANES == 4 ? Pol::kWalk : 2;  // entries per lane and batch (even)
+  constexpr int T = Pol::kTerms, M = (T + LANES - 1) / LANES;
+  constexpr int kGroups = LANES / 4;  // list groups of 8 that two of a lane's entries span
   const int lane = threadIdx.x;
-  const int s = lane & 3, p = lane >> 2;
+  const int s = lane & (LANES - 1), p = lane / LANES;
+  const int s4 = s & 3, gl = s >> 2;
   const int cnt = h.active ? S.nbr_count[h.i] : 0;
   const uint32_t* __restrict__ src =
-      list_block(P, S.nlist, ch) + (kQuarter * quarter + p) * 8 + 2 * s;
+      list_block(P, S.nlist, ch) + (kPart<LANES> * part + p) * 8 + 2 * s4;
   double* __restrict__ put = lds + lane;
-  const double2* __restrict__ get = reinterpret_cast<const double2*>(lds + s * kTermRow + 4 * p);
+  // (lanes past the components repeat the last one's sum, unused)
+  const double2* __restrict__ get = reinterpret_cast<const double2*>(
+      lds + (LANES == 4 ? s : min(s, T - 1)) * kTermRow + LANES * p);
   double sum[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) sum[m] = 0.0;
@@ -1372,21 +1439,22 @@ __device__ __forceinline__ void walk_quarter(const DevParams& P, const DeviceSta
   auto fetch = [&](int q) {
 #pragma unroll
     for (int g = 0; g < NB / 2; ++g)
-      nx[g] = *reinterpret_cast<const uint2*>(src + min((q >> 3) + g, last) * stride);
+      nx[g] = *reinterpret_cast<const uint2*>(
+          src + min((q >> 3) + g * kGroups + gl, last) * stride);
   };
   fetch(0);
-  for (int q = 0; __ballot(q < cnt) != 0ull; q += 4 * NB) {
+  for (int q = 0; __ballot(q < cnt) != 0ull; q += LANES * NB) {
     uint32_t e[NB];
     bool ok[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-      ok[k] = q + 4 * k + s < cnt;
+      ok[k] = q + 8 * (k / 2 * kGroups + gl) + 4 * (k & 1) + s4 < cnt;
       e[k] = ok[k] ? ((k & 1) ? nx[k / 2].y : nx[k / 2].x) : (uint32_t)h.ii;
     }
     typename Pol::Rec r[NB];
 #pragma unroll
     for (int k = 0; k < NB; ++k) r[k] = pol.gather(e[k]);
-    fetch(q + 4 * NB);
+    fetch(q + LANES * NB);
     // (the density bodies are short: the scheduler would sink some of these
     // loads to their first use, one wait each -- the FP64 walk of the 128^3
     // box takes 0.78 instead of 0.58 ms then)
@@ -1394,34 +1462,55 @@ __device__ __forceinline__ void walk_quarter(const DevParams& P, const DeviceSta
     double t[NB][T];
     pol.terms(e, ok, r, t);
     // (one wave per workgroup: its LDS operations complete in order)
+    if constexpr (LANES == 4) {
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int k = 0; k < NB; ++k) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int c = 0; c < T; ++c) put[c * kTermRow] = t[k][c];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int c = 0; c < T; ++c) put[c * kTermRow] = t[k][c];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int m = 0; m < M; ++m) {
-        const double2 a = get[2 * m * kTermRow], b = get[2 * m * kTermRow + 1];
-        sum[m] = sum[m] + a.x;
-        sum[m] = sum[m] + a.y;
-        sum[m] = sum[m] + b.x;
-        sum[m] = sum[m] + b.y;
+        for (int m = 0; m < M; ++m) {
+          const double2 a = get[2 * m * kTermRow], b = get[2 * m * kTermRow + 1];
+          sum[m] = sum[m] + a.x;
+          sum[m] = sum[m] + a.y;
+          sum[m] = sum[m] + b.x;
+          sum[m] = sum[m] + b.y;
+        }
       }
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int c = 0; c < T; ++c) put[k * kTermRows<T> + c * kTermRow] = t[k][c];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const double2 a = get[k * kTermRows<T> / 2 + 2 * g];
+          const double2 b = get[k * kTermRows<T> / 2 + 2 * g + 1];
+          sum[0] = sum[0] + a.x;
+          sum[0] = sum[0] + a.y;
+          sum[0] = sum[0] + b.x;
+          sum[0] = sum[0] + b.y;
+        }
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-  for (int m = 0; m < M; ++m) quarter_sum(lds, p, 4 * m + s) = sum[m];
+  for (int m = 0; m < M; ++m)
+    if (LANES == 4 || s < T) part_sum(lds, p, LANES * m + s) = sum[m];
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// The home particle of a lane in the walk of a quarter.
-template <int DIM>
-__device__ __forceinline__ Home load_quarter_home(const DevParams& P, const DeviceState& S,
-                                                  const Chunk& ch, int quarter) {
+// The home particle of a lane in the walk of a part.
+template <int DIM, int LANES>
+__device__ __forceinline__ Home load_part_home(const DevParams& P, const DeviceState& S,
+                                               const Chunk& ch, int part) {
   Home h;
-  h.i = ch.p0 + kQuarter * quarter + ((int)threadIdx.x >> 2);
+  h.i = ch.p0 + kPart<LANES> * part + (int)threadIdx.x / LANES;
   h.active = h.i < ch.p1;
   h.ii = h.active ? h.i : ch.p0;
   const int64_t n = P.n;
@@ -1442,12 +1531,11 @@ __device__ __forceinline__ Home load_quarter_home(const DevParams& P, const Devi
   return h;
 }
 
-// Chunk slot and first quarter of a workgroup that takes NQ quarters: the
-// workgroups of a chunk are 8 apart, so they share an XCD.
-template <int NQ>
-__device__ __forceinline__ int quarter_slot(int b, int& quarter) {
-  constexpr int G = 4 / NQ;
-  quarter = (b / 8) % G * NQ;
+// Chunk slot of a workgroup and which of the chunk's G workgroups it is: they
+// are 8 apart, so they share an XCD.
+template <int G>
+__device__ __forceinline__ int part_slot(int b, int& which) {
+  which = (b / 8) % G;
   return b / (8 * G) * 8 + b % 8;
 }
 
@@ -1512,28 +1600,13 @@ __device__ __forceinline__ double density_of(const DevParams& P, double sum) {
   return (MIXED ? P.coef : P.cw) * sum;
 }
 
-// One chunk slot of a density pass that scans the stencil.
-template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
-__device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceState& S, int slot,
-                                              int le_box, bool build,
-                                              float4* __restrict__ tile,
-                                              uint32_t* __restrict__ buf) {
+// The density sums of a chunk by a scan of the stencil.
+template <int DIM, bool MIXED, int TILE, int BUF, int MODE>
+__device__ __forceinline__ void scan_density(const DevParams& P, const DeviceState& S,
+                                             const Chunk& ch, const Home& h,
+                                             float4* __restrict__ tile,
+                                             uint32_t* __restrict__ buf, bool store) {
   constexpr bool kDecide = MODE != kStore;
-  Chunk ch;
-  if (!load_chunk(P, S, ch, slot)) return;
-  if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
-  if (MODE == kScan && !build && !list_overflow(P, S, ch)) return;
-  const Home h = load_home<DIM>(P, S, ch);
-  if (MODE == kScan && build) {
-    const int cnt = list_scan<DIM, !MIXED, TILE, BUF>(P, S, ch, h, tile, buf,
-                                                      list_block(P, S.nlist, ch));
-    if (h.active) S.nbr_count[h.i] = cnt;
-    // the shear time of the build (the copies across sheared faces drift
-    // from their build positions as it advances)
-    if (h.active && h.i == 0) S.time_dev[3] = S.time_dev[1];
-    if (__ballot(h.active && cnt > P.list_cap) == 0ull) return;
-    if (threadIdx.x == 0) S.gate[2] = 1;  // every writer stores 1
-  }
   const double mi = S.m[h.ii];
   uint32_t* list = MODE == kStore ? S.nlist : nullptr;
   using Pol = std::conditional_t<
@@ -1552,23 +1625,98 @@ __device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceSt
     rho = pol.acc.value();
   else
     rho = density_of<MIXED>(P, pol.acc);
-  if (!h.active) return;
+  if (!h.active || !store) return;
   const int i = h.i;
   if (MODE == kStore) S.nbr_count[i] = cnt;
   finish_density<DIM>(P, S, i, mi, rho, kDecide ? pol.nin : cnt, rechecks + pol.rechecks);
 }
 
-// The walk of the step's Verlet lists: NQ quarters of a chunk per workgroup.
-// Quarters one after the other let the epilogue (equation of state, force
-// records) run once on 64 lanes (128^3 box: FP64 0.58 ms, 0.65 with one
-// quarter per workgroup; mixed 0.46 and 0.49); a small box takes one quarter
-// per workgroup to fill the GPU.  QUINTIC: the quintic spline and the number density as
-// constants, so the batch's terms carry no branches.
-template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ>
+// One chunk slot of a density pass that scans the stencil.
+template <int DIM, bool MIXED, int TILE, int BUF, bool LE, int MODE>
+__device__ __forceinline__ void density_chunk(const DevParams& P, const DeviceState& S, int slot,
+                                              int le_box, bool build,
+                                              float4* __restrict__ tile,
+                                              uint32_t* __restrict__ buf) {
+  Chunk ch;
+  if (!load_chunk(P, S, ch, slot)) return;
+  if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
+  if (MODE == kScan && !build && !list_overflow(P, S, ch)) return;
+  const Home h = load_home<DIM>(P, S, ch);
+  if (MODE == kScan && build) {
+    const int cnt = list_scan<DIM, !MIXED, TILE, BUF>(P, S, ch, h, ch.p1 - ch.p0, threadIdx.x, tile,
+                                                      buf, list_block(P, S.nlist, ch));
+    if (h.active) S.nbr_count[h.i] = cnt;
+    // the shear time of the build (the copies across sheared faces drift
+    // from their build positions as it advances)
+    if (h.active && h.i == 0) S.time_dev[3] = S.time_dev[1];
+    if (__ballot(h.active && cnt > P.list_cap) == 0ull) return;
+    if (threadIdx.x == 0) S.gate[2] = 1;  // every writer stores 1
+  }
+  scan_density<DIM, MIXED, TILE, BUF, MODE>(P, S, ch, h, tile, buf, true);
+}
+
+// The build of small boxes: a workgroup of four waves per chunk, 16 particles
+// each, so that a wave's chain of rows is shorter and there are four times as
+// many.  The chunk's waves sum overflowed lists alike, each in its own LDS, and
+// the first one stores.
+template <int DIM, bool MIXED>
+__global__ __launch_bounds__(4 * kWave, 4) void k_density_split(DevParams P, DeviceState S) {
+  const bool build = S.gate[0] != 0;
+  if (!build && S.gate[2] == 0) return;
+  P.le_g = -1;
+  __shared__ float4 tiles[4][kTile + kTilePad<4>];
+  __shared__ uint32_t bufs[4][kBuf * kWave];
+  __shared__ int over;
+  const int wave = threadIdx.y;
+  float4* __restrict__ tile = tiles[wave];
+  uint32_t* __restrict__ buf = bufs[wave];
+  const int slots = chunk_slots(P);
+  for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
+    Chunk ch;
+    if (!load_chunk(P, S, ch, slot)) continue;
+    if (build) {
+      if (wave == 0 && threadIdx.x == 0) over = 0;
+      __syncthreads();
+      Chunk own = ch;
+      own.p0 = ch.p0 + kPart<4> * wave;
+      own.p1 = min(own.p0 + kPart<4>, ch.p1);
+      if (own.p0 < own.p1) {
+        own.xmin = (S.key_sorted[own.p0] - ch.G.cell_base) % ch.G.nm0;
+        own.xmax = (S.key_sorted[own.p1 - 1] - ch.G.cell_base) % ch.G.nm0;
+        const Home h = load_part_home<DIM, 4>(P, S, ch, wave);
+        const int cnt = list_scan<DIM, !MIXED, kTile, kBuf, 4>(
+            P, S, own, h, ch.p1 - ch.p0, kPart<4> * wave + (int)threadIdx.x / 4, tile, buf,
+            list_block(P, S.nlist, ch));
+        if (h.active && (threadIdx.x & 3) == 0) S.nbr_count[h.i] = cnt;
+        if (h.active && h.i == 0) S.time_dev[3] = S.time_dev[1];
+        if (h.active && cnt > P.list_cap) over = 1;  // every writer stores 1
+      }
+      __syncthreads();
+      const bool scan = over != 0;
+      __syncthreads();
+      if (!scan) continue;
+      if (threadIdx.x == 0) S.gate[2] = 1;
+    } else if (!list_overflow(P, S, ch)) {
+      continue;
+    }
+    scan_density<DIM, MIXED, kTile, kBuf, kScan>(P, S, ch, load_home<DIM>(P, S, ch), tile, buf,
+                                                 wave == 0);
+    __syncthreads();
+  }
+}
+
+// The walk of the step's Verlet lists: NQ parts of a chunk per workgroup.
+// Quarters of a chunk one after the other let the epilogue (equation of state,
+// force records) run once on 64 lanes (128^3 box: FP64 0.58 ms, 0.65 with one
+// quarter per workgroup; mixed 0.46 and 0.49); a small box takes one part per
+// workgroup to fill the GPU.  QUINTIC: the quintic spline and the number density
+// as constants, so the batch's terms carry no branches.
+template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ, int LANES>
 __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState S) {
   // the lists are current
   if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
-  __shared__ __align__(16) double lds[kTermWords<1>];
+  __shared__ __align__(16) double lds[kTermWords<1, LANES>];
+  constexpr int kOwn = kPart<LANES>;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (QUINTIC) {
@@ -1577,36 +1725,38 @@ __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState
   }
   int q0;
   Chunk ch;
-  if (!load_chunk(P, S, ch, quarter_slot<NQ>(blockIdx.x, q0))) return;
-  if (ch.p0 + kQuarter * q0 >= ch.p1) return;
+  if (!load_chunk(P, S, ch, part_slot<LANES / NQ>(blockIdx.x, q0))) return;
+  q0 *= NQ;
+  if (ch.p0 + kOwn * q0 >= ch.p1) return;
   if (le_box >= 0 && chunk_meets_le_face(le_box, ch, 2) != LE) return;
   if (S.gate[2] != 0 && list_overflow(P, S, ch)) return;
   const int lane = threadIdx.x;
   double rho = 0.0;
   int nin = 0, rechecks = 0;
 #pragma unroll 1
-  for (int q = 0; q < NQ && ch.p0 + kQuarter * (q0 + q) < ch.p1; ++q) {
-    const Home h = load_quarter_home<DIM>(P, S, ch, q0 + q);
+  for (int q = 0; q < NQ && ch.p0 + kOwn * (q0 + q) < ch.p1; ++q) {
+    const Home h = load_part_home<DIM, LANES>(P, S, ch, q0 + q);
     using Pol = std::conditional_t<MIXED, DensityMixed<DIM>, DensityF64<DIM, true>>;
     Pol pol{P, S, h, {}};
-    walk_quarter<DIM>(P, S, ch, q0 + q, h, pol,
-                      self_density<MIXED>(P, QUINTIC ? 1.0 : S.m[h.ii]), lds);
+    walk_part<DIM, LANES>(P, S, ch, q0 + q, h, pol,
+                          self_density<MIXED>(P, QUINTIC ? 1.0 : S.m[h.ii]), lds);
     int in = pol.nin, re = pol.rechecks;
-    in += __shfl_xor(in, 1);
-    re += __shfl_xor(re, 1);
-    in += __shfl_xor(in, 2);
-    re += __shfl_xor(re, 2);
-    const double r = quarter_sum(lds, lane & 15, 0);
-    in = __shfl(in, 4 * (lane & 15));
-    re = __shfl(re, 4 * (lane & 15));
-    if ((lane >> 4) == q) {
+#pragma unroll
+    for (int off = 1; off < LANES; off *= 2) {
+      in += __shfl_xor(in, off);
+      re += __shfl_xor(re, off);
+    }
+    const double r = part_sum(lds, lane & (kOwn - 1), 0);
+    in = __shfl(in, LANES * (lane & (kOwn - 1)));
+    re = __shfl(re, LANES * (lane & (kOwn - 1)));
+    if (lane / kOwn == q) {
       rho = r;
       nin = in;
       rechecks = re;
     }
   }
-  const int i = ch.p0 + kQuarter * q0 + lane;
-  if (lane >= kQuarter * NQ || i >= ch.p1) return;
+  const int i = ch.p0 + kOwn * q0 + lane;
+  if (lane >= kOwn * NQ || i >= ch.p1) return;
   finish_density<DIM>(P, S, i, S.m[i], density_of<MIXED>(P, rho), nin, rechecks);
 }
 
@@ -2616,7 +2766,7 @@ __global__ __launch_bounds__(kWave) void k_forces(DevParams P, DeviceState S) {
   }
 }
 
-// The force walk of Verlet lists: one quarter of a chunk per workgroup.
+// The force walk of Verlet lists: 64 / LANES particles of a chunk per workgroup.
 // SPEC: the quintic spline as a constant, with (kNoisy) or without (kQuiet)
 // thermal noise, so that a batch's pairs form one block without run-time
 // branches; kAny leaves both to the parameters.
@@ -2628,24 +2778,25 @@ enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
 // with four (191 registers); it took 1.66 with one particle per lane.  The
 // mixed bodies fit six waves (0.87 ms, 1.14 with cell-relative positions, their
 // code decode and compensated FP32 sums, one particle per lane).
-template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC>
-__global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? 6 : 1)) void k_force_walk(DevParams P, DeviceState S) {
+template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC, int LANES>
+__global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? (FT >= 5 && LANES == 16 ? 3 : 6) : 1)) void k_force_walk(DevParams P, DeviceState S) {
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (SPEC != kAny) {
     P.kernel_type = 1;
     P.noise = SPEC == kNoisy ? 1 : 0;
   }
-  int quarter;
+  constexpr int kOwn = kPart<LANES>;
+  int part;
   Chunk ch;
-  if (!load_chunk(P, S, ch, quarter_slot<1>(blockIdx.x, quarter))) return;
-  if (ch.p0 + kQuarter * quarter >= ch.p1) return;
+  if (!load_chunk(P, S, ch, part_slot<LANES>(blockIdx.x, part))) return;
+  if (ch.p0 + kOwn * part >= ch.p1) return;
   if (COLL && le_box >= 0 && chunk_meets_le_face(le_box, ch, P.coll_le_cells) != LE) return;
   if (S.gate[2] != 0 && list_overflow(P, S, ch)) return;
-  const Home h = load_quarter_home<DIM>(P, S, ch, quarter);
+  const Home h = load_part_home<DIM, LANES>(P, S, ch, part);
   constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
-  __shared__ __align__(16) double lds[kTermWords<kTerms>];
-  auto walk = [&](auto& pol) { walk_quarter<DIM>(P, S, ch, quarter, h, pol, 0.0, lds); };
+  __shared__ __align__(16) double lds[kTermWords<kTerms, LANES>];
+  auto walk = [&](auto& pol) { walk_part<DIM, LANES>(P, S, ch, part, h, pol, 0.0, lds); };
   if constexpr (MIXED) {
     auto pol = mixed_policy<DIM, FT, true>(P, S, h);
     walk(pol);
@@ -2653,11 +2804,11 @@ __global__ __launch_bounds__(kWave, (!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? 
     auto pol = f64_policy<DIM, FT, COLL, true>(P, S, h);
     walk(pol);
   }
-  const int i = ch.p0 + kQuarter * quarter + (int)threadIdx.x;
-  if (threadIdx.x >= kQuarter || i >= ch.p1) return;
+  const int i = ch.p0 + kOwn * part + (int)threadIdx.x;
+  if (threadIdx.x >= kOwn || i >= ch.p1) return;
   double sum[kTerms];
 #pragma unroll
-  for (int c = 0; c < kTerms; ++c) sum[c] = quarter_sum(lds, threadIdx.x, c);
+  for (int c = 0; c < kTerms; ++c) sum[c] = part_sum(lds, threadIdx.x, c);
   finish_pairs<DIM, FT, kPairUnit<FT, MIXED, true>, kPairGrad<FT, MIXED, COLL, true>>(
       P, S, i, sum, !COLL || S.sid[i] == 0);
 }
@@ -2726,22 +2877,43 @@ __global__ __launch_bounds__(kWave) void k_signature(DevParams P, DeviceState S)
 // ---------------------------------------------------------------------
 // Chunk slots from which a density walk takes a whole chunk per workgroup.
 constexpr int kWholeChunkSlots = 4096;
+// A box that leaves the 1024 SIMDs idle splits its work further.
+// Sixteen lanes per particle while the four-lane walk has less than a wave per
+// SIMD (density), three (forces); us per step with four lanes, and with sixteen
+// in the density, in both: 12^3 47, 39, 28; 26^3 57, 56, 48 (30^3 with sixteen
+// in the forces alone 50 instead of 59); 37 x 29 x 41 87, 91, 87 (84); 45^3 137,
+// 146, 145; 128 x 128 52, 53, 52; Oldroyd-B 12^3 57, 49, 33, 26^3 71, 70, 61,
+// 41^3 148, 154, 154.
+constexpr int kWideDensity = 16 * 1024, kWideForces = 3 * 16 * 1024;
+// Builds by four waves per chunk while a wave per chunk is less than one per
+// SIMD; us per evaluation with one and with four: 12^3 177 and 129, 32^3 191
+// and 170, mixed 175 and 161, 64 x 64 59 and 56; build and walk of 45^3 171
+// and 209.
+constexpr int kSplitSlots = 1024;
 
 template <int DIM, bool MIXED, bool LE>
 static void launch_density_walk(hipStream_t s, const DevParams& P, const DeviceState& S) {
   const int slots = chunk_slots(P);
   const dim3 b(kWave);
   const bool quintic = P.kernel_type == 1 && P.density_type == 2;
+  if constexpr (!LE) {
+    if (quintic && P.n < kWideDensity) {
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 1, 16>), dim3(16 * slots), b, 0, s,
+                         P, S);
+      return;
+    }
+  }
   if (slots >= kWholeChunkSlots) {
     if (quintic)
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 4>), dim3(slots), b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 4, 4>), dim3(slots), b, 0, s, P, S);
     else
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 4>), dim3(slots), b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 4, 4>), dim3(slots), b, 0, s, P, S);
   } else {
     if (quintic)
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 1>), dim3(4 * slots), b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 1, 4>), dim3(4 * slots), b, 0, s, P,
+                         S);
     else
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 1>), dim3(4 * slots), b, 0, s, P,
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 1, 4>), dim3(4 * slots), b, 0, s, P,
                          S);
   }
 }
@@ -2789,7 +2961,10 @@ static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceSt
   if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
     if (P.le_g >= 0) launch_density_shape<DIM, MIXED, true, kScan>(s, P, S);
   }
-  launch_density_shape<DIM, MIXED, false, kScan>(s, P, S);
+  if (P.le_g < 0 && chunk_slots(P) < kSplitSlots)
+    hipLaunchKernelGGL((k_density_split<DIM, MIXED>), strided_grid(P), dim3(kWave, 4), 0, s, P, S);
+  else
+    launch_density_shape<DIM, MIXED, false, kScan>(s, P, S);
   if constexpr (!MIXED) {
     if (P.le_g >= 0) launch_density_walk<DIM, MIXED, true>(s, P, S);
   }
@@ -2829,7 +3004,7 @@ static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceStat
     const dim3 gq(4 * chunk_slots(P));
     if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
       if (P.le_g >= 0) {
-        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, true, kAny>), gq, b, 0, s, P, S);
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, true, kAny, 4>), gq, b, 0, s, P, S);
         hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, true, true, true>), strided_grid(P), b,
                            0, s, P, S);
       }
@@ -2837,13 +3012,25 @@ static void launch_forces_le(hipStream_t s, const DevParams& P, const DeviceStat
     if (P.le_g < 0 || COLL) {
       constexpr int kWithNoise = !COLL && FT != 1 && FT != 7 ? kNoisy : kAny;
       constexpr int kNoNoise = !COLL ? kQuiet : kAny;
-      if (P.kernel_type != 1)
-        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kAny>), gq, b, 0, s, P, S);
+      // (the common laws only: a variant of every law would double the library)
+      constexpr bool kHasWide = !COLL && (FT == 3 || FT == 4 || FT == 5);
+      const dim3 gw(16 * chunk_slots(P));
+      if (kHasWide && P.kernel_type == 1 && P.n <= kWideForces) {
+        if constexpr (kHasWide) {
+          if (P.noise)
+            hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kWithNoise, 16>), gw, b,
+                               0, s, P, S);
+          else
+            hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kNoNoise, 16>), gw, b, 0,
+                               s, P, S);
+        }
+      } else if (P.kernel_type != 1)
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kAny, 4>), gq, b, 0, s, P, S);
       else if (P.noise)
-        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kWithNoise>), gq, b, 0, s, P,
-                           S);
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kWithNoise, 4>), gq, b, 0, s,
+                           P, S);
       else
-        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kNoNoise>), gq, b, 0, s, P,
+        hipLaunchKernelGGL((k_force_walk<DIM, FT, MIXED, COLL, false, kNoNoise, 4>), gq, b, 0, s, P,
                            S);
       hipLaunchKernelGGL((k_forces<DIM, FT, MIXED, COLL, false, true, true>), strided_grid(P), b,
                          0, s, P, S);
