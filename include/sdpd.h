@@ -335,11 +335,11 @@ int sdpd_sync(sdpd_ctx *ctx);
  * no sheared faces); positions must lie in [min_phys, max_phys).  The work
  * is queued on `stream` (a hipStream_t, NULL for the null stream) and the
  * call returns without waiting.  Its working buffers come from one static
- * device array of 32 MiB that every device the library runs on holds until
+ * device array of 64 MiB that every device the library runs on holds until
  * the process ends; each call overwrites it, so calls that overlap on one
  * device race.  More than SDPD_NOALLOC_MAX_PARTICLES particles, or a box
- * whose cell tables and neighbour lists do not fit the array, are refused
- * with SDPD_ERR_ARG and a message on stderr. */
+ * whose buffers take more than 32 MiB with the shortest neighbour lists,
+ * are refused with SDPD_ERR_ARG and a message on stderr. */
 int sdpd_evaluate_noalloc(const sdpd_params *params, int64_t step, const double *x,
                           const double *v, const double *m, const int32_t *id, int32_t n,
                           double *rho, double *p, double *f, void *stream);
