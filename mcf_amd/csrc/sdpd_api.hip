@@ -479,10 +479,12 @@ int alloc_state(sdpd_ctx* c, int n) {
   ALLOC(xa, N);
   if (c->prm.precision == SDPD_PRECISION_MIXED) {
     ALLOC(vr, N);
-    ALLOC(qr, N);
+    if (!P.verlet || !P.newtonian) ALLOC(qr, N);
     if (!P.newtonian) ALLOC(qr2, N);
-    ALLOC(xq, N);
-    ALLOC(an32, N);
+    if (P.verlet) {
+      ALLOC(xq, N);
+      ALLOC(an32, N);
+    }
   } else {
     ALLOC(rec64, 8 * N);
     if (!P.newtonian) ALLOC(pt64, 6 * N);
