@@ -2903,11 +2903,13 @@ static void launch_density_walk(hipStream_t s, const DevParams& P, const DeviceS
       return;
     }
   }
-  if (slots >= kWholeChunkSlots) {
+  // (the chunks next to sheared faces are few in any box: 64^3 with colloids 117
+  // us with whole chunks, 57 with quarters)
+  if (!LE && slots >= kWholeChunkSlots) {
     if (quintic)
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 4, 4>), dim3(slots), b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, false, true, 4, 4>), dim3(slots), b, 0, s, P, S);
     else
-      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, false, 4, 4>), dim3(slots), b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density_walk<DIM, MIXED, false, false, 4, 4>), dim3(slots), b, 0, s, P, S);
   } else {
     if (quintic)
       hipLaunchKernelGGL((k_density_walk<DIM, MIXED, LE, true, 1, 4>), dim3(4 * slots), b, 0, s, P,
