@@ -78,8 +78,8 @@ struct DeviceState {
   // Verlet lists: positions at the last build (cell order), the step's
   // gate (gate[0] = 1: the next density pass builds the lists; gate[1] counts
   // the builds; gate[2] = 1: a chunk's lists overflowed at the last build, so
-  // the rescan passes have work), the bits of the largest squared
-  // displacement since the build
+  // the rescan passes have work; gate[3]: workgroups of k_stats done, 0 between
+  // launches), the bits of the largest squared displacement since the build
   // seen this step, and the in-cut-off neighbours of each particle in the
   // last density pass (every mode)
   double* x_ref;

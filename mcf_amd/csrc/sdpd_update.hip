@@ -280,10 +280,50 @@ __device__ __forceinline__ void kadd(KSum& k, double v) {
   k.s = t;
 }
 
-// Block partial sums of (E_k, P_x, P_y, P_z) over fluid particles; a
-// second pass reduces the partials in a fixed order.
-__global__ __launch_bounds__(256) void k_stats_partial(DevParams P, DeviceState S) {
-  __shared__ double sh[4][256];
+// Two compensated sums added.
+__device__ __forceinline__ void kmerge(KSum& k, double s, double c) {
+  kadd(k, s);
+  k.c += c;
+}
+
+// The workgroup's sums of its 256 threads' (E_k, P_x, P_y, P_z); threads 0 to 3
+// return one each.  A tree of lanes, then of the four waves (adding 256 values
+// one after another took 10 us, and 17 us in a second launch over the 106 partials
+// of 27000 particles; now 16 us in one launch).
+__device__ __forceinline__ double block_stats(KSum (&acc)[4], double (&sh)[4][8]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    double s[4], c[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      s[q] = __shfl_down(acc[q].s, off);
+      c[q] = __shfl_down(acc[q].c, off);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) kmerge(acc[q], s[q], c[q]);
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      sh[wave][2 * q] = acc[q].s;
+      sh[wave][2 * q + 1] = acc[q].c;
+    }
+  }
+  __syncthreads();
+  KSum t = {0, 0};
+  if (threadIdx.x < 4)
+    for (int w = 0; w < 4; ++w) kmerge(t, sh[w][2 * threadIdx.x], sh[w][2 * threadIdx.x + 1]);
+  __syncthreads();
+  return t.s + t.c;
+}
+
+// (E_k, P_x, P_y, P_z) over fluid particles: a partial sum per workgroup, which
+// the last one to finish adds up in their order (gate[3] counts them, zero
+// between launches).
+__global__ __launch_bounds__(256) void k_stats(DevParams P, DeviceState S) {
+  __shared__ double sh[4][8];
+  __shared__ int arrived;
   const int64_t n = P.n;
   const int dim = P.dim;
   KSum acc[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
@@ -298,27 +338,31 @@ __global__ __launch_bounds__(256) void k_stats_partial(DevParams P, DeviceState 
     }
     kadd(acc[0], 0.5 * mi * v2);
   }
-  for (int q = 0; q < 4; ++q) sh[q][threadIdx.x] = acc[q].s + acc[q].c;
+  const double part = block_stats(acc, sh);
+  if (threadIdx.x < 4) S.partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = part;
+  // the stores have reached the L2 before thread 0 writes it back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x < 4) {
-    KSum t = {0, 0};
-    for (int k = 0; k < 256; ++k) kadd(t, sh[threadIdx.x][k]);
-    S.partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = t.s + t.c;
+  if (threadIdx.x == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    arrived = __hip_atomic_fetch_add(&S.gate[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
-}
-
-__global__ void k_stats_final(int nblocks, DeviceState S) {
-  if (threadIdx.x < 4) {
-    KSum t = {0, 0};
-    for (int b = 0; b < nblocks; ++b) kadd(t, S.partials[(int64_t)b * 4 + threadIdx.x]);
-    S.stats_out[threadIdx.x] = t.s + t.c;
-  }
+  __syncthreads();
+  if (arrived != (int)gridDim.x - 1) return;
+  KSum all[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += 256)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) kadd(all[q], S.partials[(int64_t)b * 4 + q]);
+  const double sum = block_stats(all, sh);
+  if (threadIdx.x < 4) S.stats_out[threadIdx.x] = sum;
+  if (threadIdx.x == 0) S.gate[3] = 0;
 }
 
 // Per-replica (E_k, P) with one workgroup per replica over its particles,
 // which are contiguous in cell order: [start[cell_base_q], start[cell_base_q+1]).
 __global__ __launch_bounds__(256) void k_replica_stats(DevParams P, DeviceState S) {
-  __shared__ double sh[4][256];
+  __shared__ double sh[4][8];
   const int q = blockIdx.x;
   const int64_t n = P.n;
   const int dim = P.dim;
@@ -336,13 +380,8 @@ __global__ __launch_bounds__(256) void k_replica_stats(DevParams P, DeviceState 
     }
     kadd(acc[0], 0.5 * mi * v2);
   }
-  for (int k = 0; k < 4; ++k) sh[k][threadIdx.x] = acc[k].s + acc[k].c;
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    KSum t = {0, 0};
-    for (int k = 0; k < 256; ++k) kadd(t, sh[threadIdx.x][k]);
-    S.rep_stats[(int64_t)q * 4 + threadIdx.x] = t.s + t.c;
-  }
+  const double sum = block_stats(acc, sh);
+  if (threadIdx.x < 4) S.rep_stats[(int64_t)q * 4 + threadIdx.x] = sum;
 }
 
 __global__ void k_set_step(int64_t* __restrict__ step_dev, double* __restrict__ time_dev,
@@ -426,8 +465,7 @@ void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S) {
 }
 
 void launch_stats(hipStream_t s, const DevParams& P, const DeviceState& S, int nblocks) {
-  hipLaunchKernelGGL(k_stats_partial, dim3(nblocks), dim3(256), 0, s, P, S);
-  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(64), 0, s, nblocks, S);
+  hipLaunchKernelGGL(k_stats, dim3(nblocks), dim3(256), 0, s, P, S);
 }
 
 void launch_replica_stats(hipStream_t s, const DevParams& P, const DeviceState& S) {
