@@ -527,7 +527,7 @@ int alloc_state(sdpd_ctx* c, int n) {
   ALLOC(nbr_count, N);
   ALLOC(nbr_in, N);
   ALLOC(nbr_sig_count, N);
-  ALLOC(gate, 4);
+  ALLOC(gate, 8);
   ALLOC(disp, 1);
   if (P.verlet) ALLOC(x_ref, dim * N);
   ALLOC(nlist, sdpd::list_entries(P, n));
@@ -1084,7 +1084,7 @@ int upload_impl(sdpd_ctx* c, const double* x, const double* v, const double* m,
     marching_time(c->step, c->P.dt, &t, &tle, &tprev);
     sdpd::launch_set_step(c->stream, c->S, c->step, t, tle, tprev);
   }
-  sdpd::launch_fill_i32(c->stream, c->S.gate, 0, 4);
+  sdpd::launch_fill_i32(c->stream, c->S.gate, 0, 8);
   sdpd::launch_fill_i32(c->stream, c->S.sort_ctl, 0, 8);
   sdpd::launch_fill_i32(c->stream, c->S.count, 0, c->P.ncell);
   sdpd::launch_fill_i32(c->stream, reinterpret_cast<int32_t*>(c->S.disp), 0, 2);

@@ -79,7 +79,8 @@ struct DeviceState {
   // gate (gate[0] = 1: the next density pass builds the lists; gate[1] counts
   // the builds; gate[2] = 1: a chunk's lists overflowed at the last build, so
   // the rescan passes have work; gate[3]: workgroups of k_stats done, 0 between
-  // launches), the bits of the largest squared displacement since the build
+  // launches; gate[4] = 1: the step's force walk came to sums that are not
+  // finite, so the rescan of the forces has work), the bits of the largest squared displacement since the build
   // seen this step, and the in-cut-off neighbours of each particle in the
   // last density pass (every mode)
   double* x_ref;

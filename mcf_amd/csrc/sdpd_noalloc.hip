@@ -137,7 +137,7 @@ size_t carve_state(unsigned char* base, const DevParams& P, DeviceState& S) {
   S.nbr_in = c.take<int32_t>(N);
   S.recheck = c.take<int32_t>(N);
   S.nlist = c.take<uint32_t>(sdpd::list_entries(P, P.n));
-  S.gate = c.take<int32_t>(4);
+  S.gate = c.take<int32_t>(8);
   S.disp = c.take<unsigned long long>(1);
   return c.used;
 }
@@ -176,7 +176,7 @@ __global__ void k_na_ingest(RepGeom g, int32_t n, int32_t dim, int32_t nrows, in
     for (int q = 0; q < 4; ++q) S.time_dev[q] = 0.0;
     S.sort_ctl[0] = 0;
     S.gate[0] = 1;
-    S.gate[1] = S.gate[2] = S.gate[3] = 0;
+    for (int q = 1; q < 8; ++q) S.gate[q] = 0;
   }
   const int stride = gridDim.x * blockDim.x;
   for (int r = i; r < nrows; r += stride) {

@@ -1713,8 +1713,8 @@ __global__ __launch_bounds__(4 * kWave, 4) void k_density_split(DevParams P, Dev
 // as constants, so the batch's terms carry no branches.
 template <int DIM, bool MIXED, bool LE, bool QUINTIC, int NQ, int LANES>
 __global__ __launch_bounds__(kWave) void k_density_walk(DevParams P, DeviceState S) {
-  // the lists are current
-  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = 0;
+  // the lists are current, and no force walk has left the scan anything yet
+  if (blockIdx.x == 0 && threadIdx.x == 0) S.gate[0] = S.gate[4] = 0;
   __shared__ __align__(16) double lds[kTermWords<1, LANES>];
   constexpr int kOwn = kPart<LANES>;
   const int le_box = P.le_g;
@@ -1862,12 +1862,30 @@ __device__ __forceinline__ RecF64 load_rec(const DevParams& P, const DeviceState
   return r;
 }
 
+// The pair bodies of Verlet lists without colloids (kStraight) take no in / out
+// decision: a candidate outside the cut-off adds its kernel gradient, 0, times
+// the rest.  That is 0 only while the rest is finite.  A wave whose sums do not
+// all come out finite (a velocity, pressure or tensor of a neighbour, a
+// candidate or the particle itself is not) sums again, or leaves its chunk to the
+// scan of overflowed lists, with bodies (LEAVE) that leave out the candidates
+// outside the cut-off, as the reference does.
+__device__ __forceinline__ bool not_finite(double a) { return !(fabs(a) < __builtin_inf()); }
+// the terms of the lanes in out become 0
+template <int NB, int T, class F>
+__device__ __forceinline__ void leave_out(const uint64_t (&out)[NB], F (&t)[NB][T]) {
+  const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+  for (int k = 0; k < NB; ++k)
+#pragma unroll
+    for (int c = 0; c < T; ++c) t[k][c] = ((out[k] >> lane) & 1) != 0 ? F(0) : t[k][c];
+}
+
 // force types: 3 Hu-Adams, 4 Hu-Adams angular, 5 Oldroyd-B (non-Newtonian
 // Hu-Adams).  The bodies sum m_i times the acceleration (and the Oldroyd-B
 // velocity gradient); finish_force divides by m_i once.  DECIDE (Verlet
 // lists): the entries are candidates within rc + skin; those outside the
 // cut-off add 0.
-template <int DIM, int FT, bool COLL = false, bool DECIDE = false>
+template <int DIM, int FT, bool COLL = false, bool DECIDE = false, bool LEAVE = false>
 struct ForceF64 {
   const DevParams& P;
   const DeviceState& S;
@@ -1964,6 +1982,11 @@ struct ForceF64 {
           r2[k] = square(d[k][0], d[k][1], d[k][2]);
         }
       }
+      uint64_t out[NB] = {};
+      if constexpr (LEAVE) {
+#pragma unroll
+        for (int k = 0; k < NB; ++k) out[k] = __ballot(!(ok[k] && r2[k] < P.cut2));
+      }
       // an empty slot holds the lane's own particle, no separation and no
       // velocity difference: at a squared distance outside the cut-off it
       // adds 0
@@ -1974,6 +1997,7 @@ struct ForceF64 {
 #pragma unroll
       for (int k = 0; k < NB; ++k)
         eval(e[k], r[k], d[k][0], d[k][1], d[k][2], r2[k], 0.0, t[k]);
+      if constexpr (LEAVE) leave_out(out, t);
     } else {
 #pragma unroll
       for (int k = 0; k < NB; ++k) {
@@ -2221,7 +2245,7 @@ struct ForceF64 {
   }
 };
 
-template <int DIM, int FT, bool DECIDE = false>
+template <int DIM, int FT, bool DECIDE = false, bool LEAVE = false>
 struct ForceMixed {
   const DevParams& P;
   const DeviceState& S;
@@ -2333,6 +2357,11 @@ struct ForceMixed {
       r2[k] = mixed_s2(d[k][0], d[k][1], d[k][2]);
       empty |= __ballot(!ok[k]);
     }
+    uint64_t out[NB] = {};
+    if constexpr (LEAVE) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) out[k] = __ballot(!(ok[k] && r2[k] < (float)P.cut2));
+    }
     if (__builtin_expect(empty != 0, 0)) {
 #pragma unroll
       for (int k = 0; k < NB; ++k) r2[k] = ok[k] ? r2[k] : 4.f * P.cut2_hi_f32;
@@ -2340,6 +2369,7 @@ struct ForceMixed {
 #pragma unroll
     for (int k = 0; k < NB; ++k)
       eval((int)(e[k] & kIndexMask), r[k], d[k][0], d[k][1], d[k][2], r2[k], 0.f, t[k]);
+    if constexpr (LEAVE) leave_out(out, t);
   }
   template <int NB>
   __device__ __forceinline__ void terms(const uint32_t (&e)[NB], const bool (&ok)[NB],
@@ -2595,15 +2625,15 @@ __device__ __forceinline__ void conformation_rate(const DevParams& P, const Devi
 constexpr int kForceLdsWordsF64 = 2048;
 
 // What the pair bodies need of the home particle ii.
-template <int DIM, int FT, bool DECIDE>
-__device__ __forceinline__ ForceMixed<DIM, FT, DECIDE> mixed_policy(const DevParams& P,
-                                                                    const DeviceState& S,
-                                                                    const Home& h) {
+template <int DIM, int FT, bool DECIDE, bool LEAVE>
+__device__ __forceinline__ ForceMixed<DIM, FT, DECIDE, LEAVE> mixed_policy(const DevParams& P,
+                                                                           const DeviceState& S,
+                                                                           const Home& h) {
   const int ii = h.ii;
   const float4 vi = S.vr[ii];
   const float4 qi = FT >= 5 || !DECIDE ? S.qr[ii] : make_float4(0.f, 0.f, 0.f, 0.f);
-  ForceMixed<DIM, FT, DECIDE> pol{P, S, h, vi.x, vi.y, vi.z, 0.f, vi.w, 0.f,
-                                  (uint32_t)S.pid[ii], S.step_dev[0]};
+  ForceMixed<DIM, FT, DECIDE, LEAVE> pol{P, S, h, vi.x, vi.y, vi.z, 0.f, vi.w, 0.f,
+                                         (uint32_t)S.pid[ii], S.step_dev[0]};
   if (FT <= 4) {
     // p/n^2, or p for the angular form
     const float an = DECIDE ? S.an32[ii] : qi.w;
@@ -2632,13 +2662,13 @@ __device__ __forceinline__ ForceMixed<DIM, FT, DECIDE> mixed_policy(const DevPar
   return pol;
 }
 
-template <int DIM, int FT, bool COLL, bool DECIDE>
-__device__ __forceinline__ ForceF64<DIM, FT, COLL, DECIDE> f64_policy(const DevParams& P,
-                                                                      const DeviceState& S,
-                                                                      const Home& h) {
+template <int DIM, int FT, bool COLL, bool DECIDE, bool LEAVE>
+__device__ __forceinline__ ForceF64<DIM, FT, COLL, DECIDE, LEAVE> f64_policy(const DevParams& P,
+                                                                             const DeviceState& S,
+                                                                             const Home& h) {
   const int ii = h.ii;
   const int64_t n = P.n;
-  ForceF64<DIM, FT, COLL, DECIDE> pol{P, S, h};
+  ForceF64<DIM, FT, COLL, DECIDE, LEAVE> pol{P, S, h};
   if (COLL) {
     pol.sidi = S.sid[ii];
     pol.le_t = S.time_dev[1];
@@ -2698,6 +2728,21 @@ constexpr int kPairUnit = (FT == 3 || FT == 5) ? (MIXED ? (VERLET ? 2 : 0) : 1) 
 template <int FT, bool MIXED, bool COLL, bool VERLET>
 constexpr bool kPairGrad = MIXED ? (VERLET && FT == 5) : !COLL;
 
+// Whether the walk has left particles of a chunk to the scan: their forces (or
+// velocity gradients) are not finite, and gate[4] says that there are some.
+template <int DIM, int FT>
+__device__ __forceinline__ bool lost_forces(const DeviceState& S, int64_t n, const Chunk& ch) {
+  if (S.gate[4] == 0) return false;
+  const int i = ch.p0 + (int)threadIdx.x;
+  bool lost = false;
+  if (i < ch.p1) {
+    for (int d = 0; d < DIM; ++d) lost |= not_finite(S.f[d * n + i]);
+    if (FT >= 5)
+      for (int q = 0; q < DIM * DIM; ++q) lost |= not_finite(S.vgt[q * n + i]);
+  }
+  return __ballot(lost) != 0ull;
+}
+
 // One chunk slot of a force pass with one particle per lane.  Two launches
 // over the same grid: SCAN = false takes the chunks whose lists hold every
 // neighbour and walks them (per-step lists), SCAN = true takes the others
@@ -2705,14 +2750,19 @@ constexpr bool kPairGrad = MIXED ? (VERLET && FT == 5) : !COLL;
 // With colloids a box with sheared faces splits the chunks once more: the
 // Lees-Edwards instantiation takes the rows within coll_le_cells of a face,
 // the plain one (a quarter fewer registers) the interior.  VERLET: the scan
-// takes the Verlet candidates.
+// takes the Verlet candidates, and the chunks whose walk left it particles
+// (lost_forces).
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, bool SCAN, bool VERLET>
 __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceState& S, int slot,
                                              int le_box, float4* __restrict__ tile,
                                              uint32_t* __restrict__ buf) {
   Chunk ch;
   if (!load_chunk(P, S, ch, slot)) return;
-  if (list_overflow(P, S, ch) != SCAN) return;
+  if (SCAN && VERLET && !COLL) {
+    if (!list_overflow(P, S, ch) && !lost_forces<DIM, FT>(S, P.n, ch)) return;
+  } else if (list_overflow(P, S, ch) != SCAN) {
+    return;
+  }
   if (COLL && le_box >= 0 && chunk_meets_le_face(le_box, ch, P.coll_le_cells) != LE) return;
   const Home h = load_home<DIM>(P, S, ch);
   double sum[DIM + DIM * DIM];
@@ -2728,12 +2778,12 @@ __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceSta
     }
   };
   if constexpr (MIXED) {
-    auto pol = mixed_policy<DIM, FT, VERLET>(P, S, h);
+    auto pol = mixed_policy<DIM, FT, VERLET, SCAN && VERLET>(P, S, h);
     visit(pol);
 #pragma unroll
     for (int c = 0; c < pol.kTerms; ++c) sum[c] = pol.sum(c);
   } else {
-    auto pol = f64_policy<DIM, FT, COLL, VERLET>(P, S, h);
+    auto pol = f64_policy<DIM, FT, COLL, VERLET, SCAN && VERLET>(P, S, h);
     visit(pol);
 #pragma unroll
     for (int c = 0; c < pol.kTerms; ++c) sum[c] = pol.sum[c];
@@ -2745,12 +2795,12 @@ __device__ __forceinline__ void forces_chunk(const DevParams& P, const DeviceSta
 }
 
 // With Verlet lists the rescan (SCAN) has work only if a list overflowed at
-// the build; it is launched on a reduced grid, whose workgroups take every
-// gridDim.x-th chunk slot, so that on the other steps its launch costs
-// little.
+// the build or the walk has left it some; it is launched on a reduced grid,
+// whose workgroups take every gridDim.x-th chunk slot, so that on the other
+// steps its launch costs little.
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, bool SCAN, bool VERLET = false>
 __global__ __launch_bounds__(kWave) void k_forces(DevParams P, DeviceState S) {
-  if (SCAN && VERLET && S.gate[2] == 0) return;
+  if (SCAN && VERLET && S.gate[2] == 0 && (COLL || S.gate[4] == 0)) return;
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   __shared__ float4 tile[SCAN ? kTile + 1 : 1];
@@ -2781,10 +2831,12 @@ enum ForceSpec { kAny = 0, kNoisy = 1, kQuiet = 2 };
 //
 // RESCAN (boxes with little more than a wave per SIMD, where registers cost
 // nothing): a chunk whose lists overflowed is scanned again by its first
-// workgroup, and k_forces is not launched (12^3 29.3 -> 27.9 us per step, 64 x 64
-// 37.9 -> 36.4).
+// workgroup, a wave whose sums are not finite walks its lists again, and
+// k_forces is not launched (12^3 29.3 -> 27.9 us per step, 64 x 64 37.9 -> 36.4).
+// The other boxes' walks leave such sums to k_forces: a second walk in them took
+// registers (10 to 35, and with them a wave per SIMD).
 template <int DIM, int FT, bool MIXED, bool COLL, bool LE, int SPEC, int LANES, bool RESCAN = false>
-__global__ __launch_bounds__(kWave, RESCAN ? 2 : ((!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? (FT >= 5 && LANES == 16 ? 3 : 6) : 1))) void k_force_walk(DevParams P, DeviceState S) {
+__global__ __launch_bounds__(kWave, RESCAN ? (SPEC == kQuiet && FT <= 4 ? 4 : 2) : ((!MIXED && !COLL && FT == 3) ? 4 : (MIXED ? (FT >= 5 && LANES == 16 ? 3 : 6) : 1))) void k_force_walk(DevParams P, DeviceState S) {
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   if (SPEC != kAny) {
@@ -2809,21 +2861,38 @@ __global__ __launch_bounds__(kWave, RESCAN ? 2 : ((!MIXED && !COLL && FT == 3) ?
   const Home h = load_part_home<DIM, LANES>(P, S, ch, part);
   constexpr int kTerms = DIM + (FT >= 5 ? DIM * DIM : 0);
   __shared__ __align__(16) double lds[kTermWords<kTerms, LANES>];
-  auto walk = [&](auto& pol) { walk_part<DIM, LANES>(P, S, ch, part, h, pol, 0.0, lds); };
-  if constexpr (MIXED) {
-    auto pol = mixed_policy<DIM, FT, true>(P, S, h);
-    walk(pol);
-  } else {
-    auto pol = f64_policy<DIM, FT, COLL, true>(P, S, h);
-    walk(pol);
-  }
   const int i = ch.p0 + kOwn * part + (int)threadIdx.x;
-  if (threadIdx.x >= kOwn || i >= ch.p1) return;
-  double sum[kTerms];
+  const bool mine = threadIdx.x < kOwn && i < ch.p1;
+  // true when a particle's sums are not finite
+  auto pass = [&](auto leave) {
+    constexpr bool kLeave = decltype(leave)::value;
+    auto walk = [&](auto&& pol) { walk_part<DIM, LANES>(P, S, ch, part, h, pol, 0.0, lds); };
+    if constexpr (MIXED)
+      walk(mixed_policy<DIM, FT, true, kLeave>(P, S, h));
+    else
+      walk(f64_policy<DIM, FT, COLL, true, kLeave>(P, S, h));
+    bool bad = false;
+    if (mine) {
+      double sum[kTerms];
 #pragma unroll
-  for (int c = 0; c < kTerms; ++c) sum[c] = part_sum(lds, threadIdx.x, c);
-  finish_pairs<DIM, FT, kPairUnit<FT, MIXED, true>, kPairGrad<FT, MIXED, COLL, true>>(
-      P, S, i, sum, !COLL || S.sid[i] == 0);
+      for (int c = 0; c < kTerms; ++c) {
+        sum[c] = part_sum(lds, threadIdx.x, c);
+        bad |= not_finite(sum[c]);
+      }
+      finish_pairs<DIM, FT, kPairUnit<FT, MIXED, true>, kPairGrad<FT, MIXED, COLL, true>>(
+          P, S, i, sum, !COLL || S.sid[i] == 0);
+    }
+    return __ballot(bad) != 0ull;
+  };
+  const bool bad = pass(std::false_type{});
+  if constexpr (!COLL) {
+    if (__builtin_expect(bad, 0)) {
+      if constexpr (RESCAN)
+        (void)pass(std::true_type{});
+      else if (threadIdx.x == 0)
+        S.gate[4] = 1;  // every writer stores 1
+    }
+  }
 }
 
 // ---------------------------------------------------------------------
