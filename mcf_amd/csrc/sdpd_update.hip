@@ -119,6 +119,10 @@ __global__ void k_conformation(DevParams P, DeviceState S, double lambda) {
 // decision follows.  With sheared faces the scan's windows follow the
 // current shear length and FP32 positions, which are kept current: unwrapped
 // from the build cell.
+//
+// A position that is not finite any more has no fixed-point value (the FP64
+// walks leave out its separations): the step it turns up in rebuilds the lists,
+// and the build's screen on the FP32 positions leaves the particle out of them.
 // A replica's corner and edges in registers.
 struct BoxFrame {
   double lo[3], L[3];
@@ -140,15 +144,18 @@ __device__ __forceinline__ double track_particle(const DevParams& P, const Devic
                                                  const double* xv) {
   const int64_t n = P.n;
   double w[3] = {0.0, 0.0, 0.0};
-  double d2 = 0.0;
+  double d2 = 0.0, ref = 0.0;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
     const double L = f.L[d];
-    const double raw = xv[d] - S.x_ref[d * n + i];
+    const double xr = S.x_ref[d * n + i];
+    const double raw = xv[d] - xr;
     w[d] = raw > 0.5 * L ? -L : (raw < -0.5 * L ? L : 0.0);
     const double dd = raw + w[d];
     d2 = d2 + dd * dd;
+    ref = ref + fabs(xr);
   }
+  if (P.mixed && isnan(d2) && ref < __builtin_inf()) d2 = __builtin_inf();
   if (P.mixed)
     S.xq[i] = make_uint4(fixed_position(g, 0, xv[0]), fixed_position(g, 1, xv[1]),
                          DIM == 3 ? fixed_position(g, 2, xv[2]) : 0u, (uint32_t)S.pid[i]);

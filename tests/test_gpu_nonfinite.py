@@ -92,3 +92,35 @@ def test_velocity_between_sheared_faces():
     box.prm = box.prm.replace(le_dim=2, le_v_lower=[-0.3, 0, 0], le_v_upper=[0.3, 0, 0])
     print("not finite: sheared faces", flush=True)
     check(box)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_position(mixed):
+    # A particle without neighbours, whose lists hold particles in the skin,
+    # moves to a position that is not a number: the others go on as without it.
+    # (Fixed-point units are 3e-9 and the velocities of the records 6e-8 of
+    # theirs: 1e-6 for densities, 1e-5 for forces; a neighbour adds 1e-3.)
+    box = W.tait_box_3d(12, kt=1e-3)
+    i = box.n - 1
+    box.x[i] = 11.3
+    r = distances(box.x, i, box.prm)
+    keep = (r > 1.001 * box.prm.cut_off) | (np.arange(box.n) == i)
+    assert (r[keep] < box.prm.cut_off + 0.8).sum() > 10
+    prm = W.mixed(box).prm if mixed else box.prm
+    x, v, m, pid = box.x[keep], box.v[keep], box.m[keep], box.pid[keep]
+    out = []
+    for vi in (0.0, np.nan):
+        v[-1] = vi
+        with SDPD(prm) as g:
+            g.set_skin(0.9)
+            g.upload(x, v, m, pid)
+            g.integrate_VV(3)
+            out.append((g.download()[0], g.download_density()[0], g.download_force()))
+            builds = g.list_builds()
+    (x0, rho0, f0), (x1, rho1, f1) = out
+    assert np.isnan(x1[-1]).all()
+    assert np.abs(x1[:-1] - x0[:-1]).max() < 1e-8
+    assert np.abs(rho1[:-1] / rho0[:-1] - 1.0).max() < 1e-6
+    assert np.abs(f1[:-1] - f0[:-1]).max() < 1e-5 * np.abs(f0).max()
+    # the lists are rebuilt once, without it
+    assert builds == (2 if mixed else 1)
