@@ -1564,6 +1564,17 @@ __device__ __forceinline__ bool chunk_meets_le_face(int le_g, const Chunk& ch, i
 // scans visit the candidates in the same order, so they give the same sums.
 enum DensityMode { kStore = 0, kScan = 1, kScanAll = 2 };
 
+// The pressure of particle i and its factors of the pair forces: p/n^2 and 1/n^2
+// (Newtonian Morris and Espanol, whose viscous terms divide by n_i n_j: 1/n).
+__device__ __forceinline__ void store_pressure(const DevParams& P, const DeviceState& S, int i,
+                                               double rho, double press, double& an, double& bn) {
+  an = press / (rho * rho);
+  bn = (P.newtonian && P.force_type <= 2) ? 1.0 / rho : 1.0 / (rho * rho);
+  S.p[i] = press;
+  S.an[i] = an;
+  S.bn[i] = bn;
+}
+
 // Density epilogue of particle i with number (or mass) density sum rho.
 template <int DIM>
 __device__ __forceinline__ void finish_density(const DevParams& P, const DeviceState& S, int i,
@@ -1575,13 +1586,8 @@ __device__ __forceinline__ void finish_density(const DevParams& P, const DeviceS
     rho = P.density_type == 1 ? P.rho0 : P.rho0 / mi;
   const double press = eos_pressure(P, P.density_type == 2 ? rho * mi : rho);
   S.rho[i] = rho;
-  S.p[i] = press;
-  // per-particle factors of the pair forces: p/n^2 and 1/n^2 (Newtonian
-  // Morris and Espanol, whose viscous terms divide by n_i n_j: 1/n)
-  const double an = press / (rho * rho);
-  const double bn = (P.newtonian && P.force_type <= 2) ? 1.0 / rho : 1.0 / (rho * rho);
-  S.an[i] = an;
-  S.bn[i] = bn;
+  double an, bn;
+  store_pressure(P, S, i, rho, press, an, bn);
   S.nbr_in[i] = nin;
   S.recheck[i] = rechecks;
   write_force_records<DIM>(P, S, i, an, bn, press);
@@ -1788,10 +1794,8 @@ __global__ void k_eos(DevParams P, DeviceState S) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= P.n) return;
   const double r = S.rho[i];
-  const double press = eos_pressure(P, P.density_type == 2 ? r * S.m[i] : r);
-  S.p[i] = press;
-  S.an[i] = press / (r * r);
-  S.bn[i] = 1.0 / (r * r);
+  double an, bn;
+  store_pressure(P, S, i, r, eos_pressure(P, P.density_type == 2 ? r * S.m[i] : r), an, bn);
 }
 
 // Force-pass records after the velocities or the pressure changed between
