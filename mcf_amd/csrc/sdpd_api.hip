@@ -58,7 +58,8 @@ struct sdpd_ctx {
   double mmax = 0.0;         // largest box extent plus five cells (the FP32 band)
   int parity = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
-  // pinned pieces of the downloads (from the first one on), each with an event
+  // pinned pieces of the downloads (from the first one on), each with an event;
+  // an int32 behind them that the reordering sets to 1 on a corrupt permutation
   char* stage = nullptr;
   size_t stage_bytes = 0;
   hipEvent_t stage_done[kStageSlots] = {};
@@ -774,7 +775,8 @@ bool have_staging(sdpd_ctx* c, size_t bytes) {
                                   : std::min(pieces, (size_t)kStageSlots) * kPiece;
   if (c->stage && c->stage_bytes >= want) return true;
   release_staging(c);
-  bool ok = hipHostMalloc((void**)&c->stage, want, hipHostMallocDefault) == hipSuccess;
+  bool ok = hipHostMalloc((void**)&c->stage, want + sizeof(int32_t), hipHostMallocDefault) ==
+            hipSuccess;
   if (ok)
     c->stage_bytes = want;
   else
@@ -792,10 +794,10 @@ bool have_staging(sdpd_ctx* c, size_t bytes) {
 // thread four times the transfer: each slot has a thread that copies its piece
 // out while the others' pieces are in flight (50 MB: 12.2 ms in one hipMemcpy,
 // 10.6 through pinned memory with one thread, 3.3 with eight).
-int copy_out(sdpd_ctx* c, const double* dev, size_t bytes, void* host) {
+int copy_out(sdpd_ctx* c, const double* dev, size_t bytes, void* host, bool pinned) {
   const char* src = reinterpret_cast<const char*>(dev);
   char* dst = static_cast<char*>(host);
-  if (!have_staging(c, bytes)) {
+  if (!pinned) {
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     HIP_TRY(c, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return SDPD_OK;
@@ -835,10 +837,20 @@ int copy_out(sdpd_ctx* c, const double* dev, size_t bytes, void* host) {
 // between sorts; host loops took 20 of the 128^3 box's 43 ms).
 int download_vec(sdpd_ctx* c, const double* dev, int comps, double* host) {
   double* tmp = comps > c->P.dim ? c->S.ct_alt : c->S.x_alt;
-  sdpd::launch_to_upload_order(c->stream, c->P, c->S, comps, dev, tmp);
+  const size_t bytes = (size_t)comps * c->n * sizeof(double);
+  const bool pinned = have_staging(c, bytes);
+  int32_t* corrupt = pinned ? reinterpret_cast<int32_t*>(c->stage + c->stage_bytes) : c->S.gate + 5;
+  if (pinned) *corrupt = 0;
+  sdpd::launch_to_upload_order(c->stream, c->n, comps, c->S.perm, dev, tmp, corrupt);
   int rc = check_launch(c, "download");
+  if (!rc) rc = copy_out(c, tmp, bytes, host, pinned);
   if (rc) return rc;
-  return copy_out(c, tmp, (size_t)comps * c->n * sizeof(double), host);
+  int32_t bad = 0;
+  if (pinned)
+    bad = *corrupt;
+  else
+    HIP_TRY(c, hipMemcpy(&bad, corrupt, sizeof(bad), hipMemcpyDeviceToHost));
+  return bad ? fail(c, SDPD_ERR_STATE, "corrupt permutation") : SDPD_OK;
 }
 
 }  // namespace

@@ -80,7 +80,8 @@ struct DeviceState {
   // the builds; gate[2] = 1: a chunk's lists overflowed at the last build, so
   // the rescan passes have work; gate[3]: workgroups of k_stats done, 0 between
   // launches; gate[4] = 1: the step's force walk came to sums that are not
-  // finite, so the rescan of the forces has work), the bits of the largest squared displacement since the build
+  // finite, so the rescan of the forces has work; gate[5] = 1: a download met a
+  // corrupt permutation), the bits of the largest squared displacement since the build
   // seen this step, and the in-cut-off neighbours of each particle in the
   // last density pass (every mode)
   double* x_ref;
@@ -121,9 +122,10 @@ void launch_refresh_records(hipStream_t s, const DevParams& P, const DeviceState
 // Verlet lists: displacement since the last build and the positions the walks
 // gather, after a separate drift
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S);
-// src (comps planes of n, cell order) -> dst (comps, n) in upload order
-void launch_to_upload_order(hipStream_t s, const DevParams& P, const DeviceState& S, int comps,
-                            const double* src, double* dst);
+// src (comps planes of n, cell order) -> dst (comps, n) in upload order; corrupt
+// (device or pinned memory, 0) becomes 1 if an index of perm is out of range
+void launch_to_upload_order(hipStream_t s, int n, int comps, const int32_t* perm,
+                            const double* src, double* dst, int32_t* corrupt);
 void launch_kick(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);
 void launch_drift_wrap(hipStream_t s, const DevParams& P, const DeviceState& S);
 void launch_conformation(hipStream_t s, const DevParams& P, const DeviceState& S, double lambda);

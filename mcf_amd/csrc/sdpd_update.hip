@@ -407,13 +407,18 @@ __global__ void k_advance_step(int64_t* __restrict__ step_dev, double* __restric
 }
 
 // One quantity from cell order, structure of arrays, to upload order with a
-// particle's components together.
+// particle's components together.  corrupt is set to 1 if an upload index is out
+// of range.
 __global__ void k_to_upload_order(int n, int comps, const int32_t* __restrict__ perm,
-                                  const double* __restrict__ src, double* __restrict__ dst) {
+                                  const double* __restrict__ src, double* __restrict__ dst,
+                                  int32_t* __restrict__ corrupt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t u = perm[i];
-  if (u < 0 || u >= n) return;
+  if (u < 0 || u >= n) {
+    *corrupt = 1;
+    return;
+  }
   for (int q = 0; q < comps; ++q) dst[u * comps + q] = src[(int64_t)q * n + i];
 }
 
@@ -461,10 +466,10 @@ void launch_boundary(hipStream_t s, const DevParams& P, const DeviceState& S, in
     hipLaunchKernelGGL((k_boundary<2, false>), g, b, 0, s, P, S, closing, opening);
 }
 
-void launch_to_upload_order(hipStream_t s, const DevParams& P, const DeviceState& S, int comps,
-                            const double* src, double* dst) {
-  hipLaunchKernelGGL(k_to_upload_order, dim3(nblk(P.n)), dim3(256), 0, s, P.n, comps, S.perm, src,
-                     dst);
+void launch_to_upload_order(hipStream_t s, int n, int comps, const int32_t* perm,
+                            const double* src, double* dst, int32_t* corrupt) {
+  hipLaunchKernelGGL(k_to_upload_order, dim3(nblk(n)), dim3(256), 0, s, n, comps, perm, src, dst,
+                     corrupt);
 }
 
 void launch_track(hipStream_t s, const DevParams& P, const DeviceState& S) {
