@@ -8,14 +8,13 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <utility>
 #include <vector>
 
 #include "../../include/sdpd.h"
 #include "sdpd_host.h"
 #include "sdpd_kernels.h"
+#include "sdpd_threads.h"
 
 using sdpd::DevParams;
 using sdpd::DeviceState;
@@ -817,17 +816,8 @@ int copy_out(sdpd_ctx* c, const double* dev, size_t bytes, void* host, bool pinn
     }
     if (e != hipSuccess) error = (int)e;
   };
-  std::thread helper[kStageSlots];
-  for (int slot = 1; slot < kStageSlots && (size_t)slot < pieces; ++slot) {
-    try {
-      helper[slot] = std::thread(work, slot);
-    } catch (const std::system_error&) {
-      break;  // the threads there are take all the pieces
-    }
-  }
-  work(0);
-  for (std::thread& t : helper)
-    if (t.joinable()) t.join();
+  // (the threads there are take all the pieces)
+  sdpd::run_slots<kStageSlots>((int)std::min(pieces, (size_t)kStageSlots), work);
   HIP_TRY(c, (hipError_t)error.load());
   return SDPD_OK;
 }
