@@ -216,15 +216,16 @@ int sdpd_set_colloids(sdpd_ctx *ctx, const sdpd_colloid_params *prm, int32_t num
 int sdpd_get_colloids(sdpd_ctx *ctx, double *x, double *v, double *omega, double *drag,
                       double *torque);
 
-/* sdpd_step runs pairs of steps through a captured HIP graph (default on,
- * and off while phase timing is enabled); enable = 0 launches every kernel
+/* sdpd_step runs four steps at a time through a captured HIP graph (default
+ * on, and off while phase timing is enabled); enable = 0 launches every kernel
  * directly.  Results are identical either way. */
 int sdpd_set_graphs(sdpd_ctx *ctx, int32_t enable);
 
 /* Launch shapes of the pair kernels.  No counterpart in the reference
- * (its loops have no tunable shape).  density_shape picks the candidate
- * scan's LDS tile and per-lane list buffer: 0 = 224 records / 16 entries
- * (default), 1 = 128 / 16, 2 = 224 / 12, 3 = 128 / 12; chunk_order 1 lets
+ * (its loops have no tunable shape).  density_shape picks the LDS tile and
+ * per-lane list buffer of the candidate scan of lists rebuilt every step:
+ * 0 = 224 records / 16 entries (default, and what Verlet lists are built
+ * with whatever is set), 1 = 128 / 16, 2 = 224 / 12, 3 = 128 / 12; chunk_order 1 lets
  * each XCD work through a contiguous eighth of the chunks (default), 0
  * hands chunk b to workgroup b.  Every choice gives identical results. */
 typedef struct sdpd_tuning {
@@ -272,8 +273,7 @@ int sdpd_get_list_builds(sdpd_ctx *ctx, int64_t *builds);
  * shape (the simulation does not advance), applies the fastest and returns
  * it with its time per density + force pass pair (ms).  Lists rebuilt every
  * step: density + force pass pairs for every shape.  Verlet lists: the
- * chunk order on pass pairs that walk the lists (each step's cost), then
- * the density shape on candidate scans of every chunk (each build's). */
+ * chunk order on pass pairs that walk the lists (density_shape 0). */
 int sdpd_autotune(sdpd_ctx *ctx, int32_t reps, sdpd_tuning *best, double *ms_best);
 
 /* Noise step counter (the reference's marching step). */

@@ -648,11 +648,11 @@ int run_list_update(sdpd_ctx* c, bool advance = false) {
   return SDPD_OK;
 }
 
-int run_density(sdpd_ctx* c, bool scan_all = false) {
+int run_density(sdpd_ctx* c) {
   c->P.step = c->step;
   {
     PhaseMark pm(c, 2);
-    sdpd::launch_density(c->stream, c->P, c->S, c->P.mixed != 0, scan_all);
+    sdpd::launch_density(c->stream, c->P, c->S, c->P.mixed != 0);
   }
   int rc = check_launch(c, "density");
   if (rc) return rc;
@@ -1601,14 +1601,11 @@ int sdpd_autotune(sdpd_ctx* c, int32_t reps, sdpd_tuning* best, double* ms_best)
     release_saved();
     return fail(c, SDPD_ERR_DEVICE, "sdpd_autotune: event creation failed");
   }
-  // reps timed passes after an untimed one, at the current positions (the
-  // state is recomputed identically each time): SCAN times the candidate
-  // scan of every chunk (the density pass of a Verlet build), otherwise a
-  // density + force pass pair as a step runs it.  Returns the time in ms,
-  // or -1 after an error (rc set).
-  auto time_passes = [&](bool scan) -> float {
+  // reps timed density + force pass pairs as a step runs them, after an
+  // untimed one, at the current positions (the state is recomputed identically
+  // each time).  Returns the time in ms, or -1 after an error (rc set).
+  auto time_passes = [&]() -> float {
     auto pass = [&]() -> int {
-      if (scan) return run_density(c, true);
       int r = run_density(c);
       if (!r) r = run_forces(c);
       return r;
@@ -1641,27 +1638,17 @@ int sdpd_autotune(sdpd_ctx* c, int32_t reps, sdpd_tuning* best, double* ms_best)
   float tbest = -1.f;
   if (c->P.verlet) {
     // Verlet lists: a step walks the lists, whose cost depends on the chunk
-    // order alone; the density shape serves the candidate scan of the
-    // builds.  The order is chosen on walk passes, then the shape on scans.
+    // order alone; their builds have one shape.
     float t_order[2] = {-1.f, -1.f};
     for (int k = 0; k < 4 && rc == SDPD_OK; ++k) {
       const int order = k == 0 || k == 3 ? 1 : 0;
       c->P.xcd_order = order;
-      keep_min(t_order[order], time_passes(false));
+      keep_min(t_order[order], time_passes());
     }
     if (rc == SDPD_OK) {
       pick.chunk_order = t_order[0] < kOrderMargin * t_order[1] ? 0 : 1;
       tbest = t_order[pick.chunk_order];
     }
-    c->P.xcd_order = pick.chunk_order;
-    float t_shape[4] = {-1.f, -1.f, -1.f, -1.f};
-    for (int k = 0; k < 8 && rc == SDPD_OK; ++k) {
-      const int shape = k < 4 ? k : 7 - k;
-      c->P.density_shape = shape;
-      keep_min(t_shape[shape], time_passes(true));
-    }
-    for (int shape = 1; shape < 4; ++shape)
-      if (t_shape[shape] < t_shape[pick.density_shape]) pick.density_shape = shape;
   } else {
     // lists rebuilt every step: the density pass is the scan itself
     float t[2][4] = {{-1.f, -1.f, -1.f, -1.f}, {-1.f, -1.f, -1.f, -1.f}};
@@ -1670,7 +1657,7 @@ int sdpd_autotune(sdpd_ctx* c, int32_t reps, sdpd_tuning* best, double* ms_best)
       const int order = 1 - m / 4, shape = m % 4;
       c->P.density_shape = shape;
       c->P.xcd_order = order;
-      keep_min(t[order][shape], time_passes(false));
+      keep_min(t[order][shape], time_passes());
     }
     if (rc == SDPD_OK) {
       int s_order[2] = {0, 0};

@@ -110,10 +110,7 @@ void launch_sort_phases(hipStream_t s, const DevParams& P, const DeviceState& S,
 // rlpdx without moving the state
 void launch_reference_cells(hipStream_t s, const DevParams& P, const DeviceState& S);
 
-// scan_all (Verlet lists, the autotuner): every chunk scans its stencil,
-// without storing lists, whatever the step's gate
-void launch_density(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed,
-                    bool scan_all = false);
+void launch_density(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed);
 void launch_eos(hipStream_t s, const DevParams& P, const DeviceState& S);
 void launch_forces(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed);
 void launch_signature(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed);

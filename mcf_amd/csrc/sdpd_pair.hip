@@ -39,8 +39,8 @@
 namespace sdpd {
 
 constexpr int kWave = 64;
-// Defaults of the two tunable shapes of the candidate scan (the density
-// kernel is instantiated for the autotuner's other choices too):
+// Defaults of the two tunable shapes of the candidate scan (the density kernel of
+// lists rebuilt every step is instantiated for the autotuner's other choices too):
 constexpr int kBuf = 16;          // LDS list entries per lane between flushes (>= 10)
 constexpr int kTile = 224;        // staged candidate records per stencil row batch
 constexpr int kCodeShift = 25;    // list entry = j | (stencil code << 25)
@@ -1559,10 +1559,10 @@ __device__ __forceinline__ bool chunk_meets_le_face(int le_g, const Chunk& ch, i
 // cut-off per candidate on the current positions: k_density_walk walks the
 // lists of the chunks that hold them all, and kScan, before it, stores the
 // candidates within rc + skin of every chunk on steps whose gate asks for it,
-// and scans the stencil for the sums of the chunks whose lists overflowed;
-// kScanAll does the latter for every chunk (the autotuner).  The walk and the
-// scans visit the candidates in the same order, so they give the same sums.
-enum DensityMode { kStore = 0, kScan = 1, kScanAll = 2 };
+// and scans the stencil for the sums of the chunks whose lists overflowed.  The
+// walk and the scans visit the candidates in the same order, so they give the
+// same sums.
+enum DensityMode { kStore = 0, kScan = 1 };
 
 // The pressure of particle i and its factors of the pair forces: p/n^2 and 1/n^2
 // (Newtonian Morris and Espanol, whose viscous terms divide by n_i n_j: 1/n).
@@ -3014,63 +3014,66 @@ static inline dim3 strided_grid(const DevParams& P) {
   return dim3(std::min(chunk_slots(P), 4096));
 }
 
-template <int DIM, bool MIXED, bool LE, int MODE>
+// Lists rebuilt every step, in the shape asked for.  (Verlet lists are built in
+// the default one.  The build holds four waves per SIMD with either tile, and the
+// larger one takes a row's records in one batch; a list buffer of 12 is the same
+// ring of 16.  Density pass with a build, tiles of 224 and 128: 128^3 1.53 and
+// 1.59 ms, 100^3 0.81 and 0.86, 45^3 150 and 184 us, Oldroyd-B 41^3 137 and 157,
+// 256 x 256 36 and 37.)
+template <int DIM, bool MIXED, bool LE>
 static void launch_density_shape(hipStream_t s, const DevParams& P, const DeviceState& S) {
-  const dim3 g = MODE == kScan ? strided_grid(P) : dim3(chunk_slots(P)), b(kWave);
+  const dim3 g(chunk_slots(P)), b(kWave);
   switch (P.density_shape) {
     case 1:
-      hipLaunchKernelGGL((k_density<DIM, MIXED, 128, 16, LE, MODE>), g, b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density<DIM, MIXED, 128, 16, LE, kStore>), g, b, 0, s, P, S);
       break;
     case 2:
-      hipLaunchKernelGGL((k_density<DIM, MIXED, 224, 12, LE, MODE>), g, b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density<DIM, MIXED, 224, 12, LE, kStore>), g, b, 0, s, P, S);
       break;
     case 3:
-      hipLaunchKernelGGL((k_density<DIM, MIXED, 128, 12, LE, MODE>), g, b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density<DIM, MIXED, 128, 12, LE, kStore>), g, b, 0, s, P, S);
       break;
     default:
-      hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, LE, MODE>), g, b, 0, s, P, S);
+      hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, LE, kStore>), g, b, 0, s, P, S);
   }
 }
 
 template <int DIM, bool MIXED>
-static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceState& S,
-                               bool scan_all) {
+static void launch_density_dim(hipStream_t s, const DevParams& P, const DeviceState& S) {
   if (!P.verlet) {
-    if (P.le_g >= 0) launch_density_shape<DIM, MIXED, true, kStore>(s, P, S);
-    launch_density_shape<DIM, MIXED, false, kStore>(s, P, S);
-    return;
-  }
-  if (scan_all) {
-    launch_density_shape<DIM, MIXED, false, kScanAll>(s, P, S);
+    if (P.le_g >= 0) launch_density_shape<DIM, MIXED, true>(s, P, S);
+    launch_density_shape<DIM, MIXED, false>(s, P, S);
     return;
   }
   // Verlet lists: a box with sheared faces splits the chunks between
   // the Lees-Edwards and the plain instantiations, as its per-step lists do
   if constexpr (!MIXED) {  // mixed precision keeps per-step lists in sheared boxes
-    if (P.le_g >= 0) launch_density_shape<DIM, MIXED, true, kScan>(s, P, S);
+    if (P.le_g >= 0)
+      hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, true, kScan>), strided_grid(P),
+                         dim3(kWave), 0, s, P, S);
   }
   if (P.le_g < 0 && chunk_slots(P) < kSplitSlots)
     hipLaunchKernelGGL((k_density_split<DIM, MIXED>), strided_grid(P), dim3(kWave, 4), 0, s, P, S);
   else
-    launch_density_shape<DIM, MIXED, false, kScan>(s, P, S);
+    hipLaunchKernelGGL((k_density<DIM, MIXED, kTile, kBuf, false, kScan>), strided_grid(P),
+                       dim3(kWave), 0, s, P, S);
   if constexpr (!MIXED) {
     if (P.le_g >= 0) launch_density_walk<DIM, MIXED, true>(s, P, S);
   }
   launch_density_walk<DIM, MIXED, false>(s, P, S);
 }
 
-void launch_density(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed,
-                    bool scan_all) {
+void launch_density(hipStream_t s, const DevParams& P, const DeviceState& S, bool mixed) {
   if (P.dim == 3) {
     if (mixed)
-      launch_density_dim<3, true>(s, P, S, scan_all);
+      launch_density_dim<3, true>(s, P, S);
     else
-      launch_density_dim<3, false>(s, P, S, scan_all);
+      launch_density_dim<3, false>(s, P, S);
   } else {
     if (mixed)
-      launch_density_dim<2, true>(s, P, S, scan_all);
+      launch_density_dim<2, true>(s, P, S);
     else
-      launch_density_dim<2, false>(s, P, S, scan_all);
+      launch_density_dim<2, false>(s, P, S);
   }
 }
 
