@@ -103,7 +103,9 @@ void launch_fill_f64(hipStream_t s, double* a, double v, int64_t n);
 enum class SortKind { kStep, kStepKeysDone, kVerletGated, kVerletForced };
 void launch_sort(hipStream_t s, const DevParams& P, const DeviceState& S, SortKind kind,
                  bool advance = false);
-// the same sort, one launch per phase, without sort_ctl and the gate
+// the same sort for callers without a gate that may overlap on one device: one
+// launch per phase (small boxes: one launch, which counts its workgroups in
+// sort_ctl[0], zero before; nothing waits)
 void launch_sort_phases(hipStream_t s, const DevParams& P, const DeviceState& S, bool copy_back);
 // PPM's cell list on PPM's grid, particles ordered by upload index inside a
 // cell (ppm_util_rank3d on the particles in upload order); fills rstart and
