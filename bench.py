@@ -376,7 +376,7 @@ def main() -> int:
     force_gbs = head["force_bytes_per_particle"] * head["particles"] / t_force / 1e9
     roofline = {
         "bound": "hbm",
-        "kernel": "pair forces (k_forces list walk + overflow rescan)",
+        "kernel": "pair forces (k_force_walk, and k_forces for lists that overflowed)",
         "achieved": force_gbs,
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
