@@ -29,9 +29,10 @@ struct DeviceState {
   int32_t *row_chunk_off, *chunk_row;
   int32_t *scan_tmp;     // tile sums of the exclusive scans
   int32_t *sort_ctl;     // counters of the sort chain (8, zero between sorts)
-  // FP64 records of the force pass, planes of n 16-byte entries: (x, y),
-  // (z, p/n^2), (vx, vy), (vz, 1/n^2); Oldroyd-B also Pi / n^2 as (xx, yy),
-  // (zz, xy), (xz, yz) (2D: zz and the last plane 0)
+  // FP64 records of the force pass, four 16-byte entries: (x, y), (z, p/n^2),
+  // (vx, vy), (vz, 1/n^2); Oldroyd-B also Pi / n^2 as (xx, yy), (zz, xy),
+  // (xz, yz) (2D: zz and the last entry 0).  Verlet lists: in planes of n
+  // entries; lists rebuilt every step: a particle's entries together
   double *rec64;
   double *pt64;
   // FP32 records, lists rebuilt every step: velocity with w = 1 / n^2

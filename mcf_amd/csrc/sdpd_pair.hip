@@ -1250,12 +1250,16 @@ struct DensityMixed {
 };
 
 // Records of the force pass, written once the density is known.
-//   FP64: four planes of n 16-byte entries, (x, y), (z, p/n^2), (vx, vy) and
-//   (vz, 1/n^2).  Neighbours in a list are near each other in memory, so the
-//   lanes of a 16-byte gather share lines: gathers alone at the 128^3 box's
-//   lists take 151 CU cycles per wave-entry this way and 221 from 64-byte
-//   records (four lanes per particle).  With Verlet lists the (x, y) plane
-//   follows the positions (boundary, sort, track) and is not written here.
+//   FP64, Verlet lists: four planes of n 16-byte entries, (x, y), (z, p/n^2),
+//   (vx, vy) and (vz, 1/n^2).  Neighbours in a list are near each other in
+//   memory, so the lanes of a 16-byte gather share lines: gathers alone at the
+//   128^3 box's lists take 151 CU cycles per wave-entry this way and 221 from
+//   64-byte records (four lanes per particle).  The (x, y) plane follows the
+//   positions (boundary, sort, track) and is not written here.
+//   FP64, lists rebuilt every step: the same 64 bytes per particle together.  A
+//   lane of that walk takes a whole list, and a record costs it four lines from
+//   planes, one this way: forces of the 128^3 box 2.20 and 1.70 ms, 64^3 264 and
+//   220 us, Oldroyd-B 64^3 434 and 354.
 //   FP32 Newtonian: (cell-relative x, y, z, p/n^2 for Hu-Adams or p for the
 //   angular form) and (vx, vy, vz, 1/n^2); the pair body gathers these two
 //   and the particle id.
@@ -1302,11 +1306,13 @@ __device__ __forceinline__ void write_force_records(const DevParams& P, const De
       }
     }
   } else {
-    double2* pl = reinterpret_cast<double2*>(S.rec64);
-    if (!P.verlet) pl[i] = make_double2(S.x[i], S.x[n + i]);
-    pl[n + i] = make_double2(DIM == 3 ? S.x[2 * n + i] : 0.0, an);
-    pl[2 * n + i] = make_double2(S.v[i], S.v[n + i]);
-    pl[3 * n + i] = make_double2(DIM == 3 ? S.v[2 * n + i] : 0.0, bn);
+    // entry q of the record is at pl[q * step]
+    double2* pl = reinterpret_cast<double2*>(S.rec64) + (P.verlet ? i : 4 * (int64_t)i);
+    const int64_t step = P.verlet ? n : 1;
+    if (!P.verlet) pl[0] = make_double2(S.x[i], S.x[n + i]);
+    pl[step] = make_double2(DIM == 3 ? S.x[2 * n + i] : 0.0, an);
+    pl[2 * step] = make_double2(S.v[i], S.v[n + i]);
+    pl[3 * step] = make_double2(DIM == 3 ? S.v[2 * n + i] : 0.0, bn);
     if (!P.newtonian) {
       // Oldroyd-B: Pi / n^2 as (xx, yy, zz, xy, xz, yz), Pi = (p + G) I - G c
       // (particles_compute_pressure_tensor.F90:114-133; c is symmetric)
@@ -1314,15 +1320,15 @@ __device__ __forceinline__ void write_force_records(const DevParams& P, const De
         const double c = S.ct[(int64_t)(a + DIM * b) * n + i];
         return ((a == b ? press + P.G : 0.0) - P.G * c) * bn;
       };
-      double2* q = reinterpret_cast<double2*>(S.pt64) + i;
+      double2* q = reinterpret_cast<double2*>(S.pt64) + (P.verlet ? i : 3 * (int64_t)i);
       if (DIM == 3) {
         q[0] = make_double2(pib(0, 0), pib(1, 1));
-        q[n] = make_double2(pib(2, 2), pib(0, 1));
-        q[2 * n] = make_double2(pib(0, 2), pib(1, 2));
+        q[step] = make_double2(pib(2, 2), pib(0, 1));
+        q[2 * step] = make_double2(pib(0, 2), pib(1, 2));
       } else {
         q[0] = make_double2(pib(0, 0), pib(1, 1));
-        q[n] = make_double2(0.0, pib(0, 1));
-        q[2 * n] = make_double2(0.0, 0.0);
+        q[step] = make_double2(0.0, pib(0, 1));
+        q[2 * step] = make_double2(0.0, 0.0);
       }
     }
   }
@@ -1841,17 +1847,35 @@ __device__ __forceinline__ void noise_vector(const DevParams& P, int64_t step, u
   }
 }
 
-// One FP64 force record, gathered from its four planes.
+// One FP64 force record, gathered from its four planes (Verlet lists) or from its
+// 64 bytes.
 struct RecF64 {
   double2 a, b, c, d;  // (x, y), (z, p/n^2), (vx, vy), (vz, 1/n^2)
-  uint32_t pid;        // with thermal noise
+  uint32_t pid;        // with thermal noise, from the planes
   double2 q0, q1, q2;  // Oldroyd-B: Pi / n^2 as (xx, yy), (zz, xy), (xz, yz)
 };
-template <bool TENSOR>
+template <bool TENSOR, bool PLANES>
 __device__ __forceinline__ RecF64 load_rec(const DevParams& P, const DeviceState& S, uint32_t j) {
   const double2* __restrict__ pl = reinterpret_cast<const double2*>(S.rec64);
   const int64_t n = P.n;
   RecF64 r;
+  if (!PLANES) {
+    const double2* __restrict__ one = pl + 4 * (int64_t)j;
+    r.a = one[0];
+    r.b = one[1];
+    r.d = one[3];
+    r.c = one[2];
+    // (before anything else: 128^3 1.85 ms without)
+    __builtin_amdgcn_sched_barrier(0);
+    r.pid = 0u;
+    if (TENSOR) {
+      const double2* __restrict__ pt = reinterpret_cast<const double2*>(S.pt64) + 3 * (int64_t)j;
+      r.q0 = pt[0];
+      r.q1 = pt[1];
+      r.q2 = pt[2];
+    }
+    return r;
+  }
   r.a = load_at(pl, j);
   r.b = load_at(pl + n, j);
   r.c = load_at(pl + 2 * n, j);
@@ -1925,7 +1949,7 @@ struct ForceF64 {
       // colloid CYCLE, colloid-colloid pair forces off)
       if (sidi != 0 && (ent & kBoundaryBit) != 0u) return;
     }
-    const RecF64 r = load_rec<(FT >= 5)>(P, S, j);
+    const RecF64 r = load_rec<(FT >= 5), DECIDE>(P, S, j);
     const Images o = decode_images(ent);
     double d0, d1, d2;
     const double r2 = pair_d2<DIM>(P, h, o, r.a.x, r.a.y, r.b.x, d0, d1, d2);
@@ -1948,7 +1972,7 @@ struct ForceF64 {
   }
   using Rec = RecF64;
   __device__ __forceinline__ Rec gather(uint32_t ent) const {
-    return load_rec<(FT >= 5)>(P, S, ent & kIndexMask);
+    return load_rec<(FT >= 5), true>(P, S, ent & kIndexMask);
   }
   // The terms of NB candidates, whose records are gathered already.
   template <int NB>
@@ -2025,7 +2049,14 @@ struct ForceF64 {
                                        double d2, double r2, double jump,
                                        double (&t)[kTerms]) const {
     const int j = (int)(ent & kIndexMask);
-    const uint32_t pidj = rj.pid;
+    // j's pid, where the noise needs it.  Lists rebuilt every step gather it there,
+    // not with the record: a wave that asked for both at once, and so went on
+    // sooner, had its lines taken from the L1 by others' (128^3 2.04 and 1.72 ms).
+    auto pid_j = [&]() {
+      if constexpr (DECIDE) return rj.pid;
+      __builtin_amdgcn_sched_barrier(0);
+      return (uint32_t)S.pid[j];
+    };
     const bool jb = COLL && (ent & kBoundaryBit) != 0u;
     const double ir = rsqrt_nr(r2);
     const double r = r2 * ir;
@@ -2077,7 +2108,7 @@ struct ForceF64 {
       a0 = fd1 * u0 + se * d0;
       a1 = fd1 * u1 + se * d1;
       a2 = fd1 * u2 + se * d2;
-      if (P.noise) espanol_noise(pidj, d0, d1, d2, ir, gnn, a0, a1, a2);
+      if (P.noise) espanol_noise(pid_j(), d0, d1, d2, ir, gnn, a0, a1, a2);
     } else if (FT == 4) {
       // rhs_force_ff_Newtonian_HuAdams_angular.F90:166-229: everything
       // along e = d / r
@@ -2085,6 +2116,7 @@ struct ForceF64 {
       const double aij = (bi + bj) * gw;
       double sc = P.eta_coef * P.eta * aij * du * (ir * ir) - aij * pij;
       if (P.noise) {
+        const uint32_t pidj = pid_j();
         float g[4];
         pair_normals(P.seed, pidi < pidj ? pidi : pidj, pidi < pidj ? pidj : pidi, step, g);
         sc = sc + (double)g[0] * P.sqrt_2kt_eta * sqrt_nr(-P.eta_coef * aij * ir) * P.inv_sqrt_dt;
@@ -2148,11 +2180,12 @@ struct ForceF64 {
         }
       }
       if (FT == 6 && P.noise) {
-        espanol_noise(pidj, d0, d1, d2, ir,
+        espanol_noise(pid_j(), d0, d1, d2, ir,
                       gw * ir * inv_ni / S.rho[j], a0, a1, a2);
       } else if (FT != 7 && P.noise) {
         // f_r W e with W e = s ca (g + cb / ca (g.e) e), e = d / r, s = +1 when
         // pid_i < pid_j (noise_vector), written on d to save operations
+        const uint32_t pidj = pid_j();
         float g[4];
         pair_normals(P.seed, pidi < pidj ? pidi : pidj, pidi < pidj ? pidj : pidi, step, g);
         // sqrt(-4 kT f_d / dt) / sqrt(2) as one root, in units of cg < 0 (the
@@ -2624,9 +2657,13 @@ __device__ __forceinline__ void conformation_rate(const DevParams& P, const Devi
 
 // The FP64 walk of per-step lists (without colloids) takes 8 KB of LDS per
 // workgroup, its entry buffer plus a reserve.  That holds it to five waves
-// per SIMD.  Its registers alone would allow six, but on the 128^3 box six
-// waves' gathers ran 6 % slower (1.99 against 1.88 ms per pass).
-constexpr int kForceLdsWordsF64 = 2048;
+// per SIMD: each lane's gather touches a line of its own, and more waves take
+// each other's lines from the L1.  (The 128^3 box: 1.99 ms per pass with six
+// waves, 1.88 with five, before the noise's present form; 1.70 with five now,
+// 1.75 with four.)  Oldroyd-B's records are 112 bytes: held below three waves,
+// 100^3 1.56 ms instead of 1.60, 64^3 354 us instead of 367.
+template <int FT>
+constexpr int kForceLdsWordsF64 = FT >= 5 ? 4096 : 2048;
 
 // What the pair bodies need of the home particle ii.
 template <int DIM, int FT, bool DECIDE, bool LEAVE>
@@ -2808,7 +2845,7 @@ __global__ __launch_bounds__(kWave) void k_forces(DevParams P, DeviceState S) {
   const int le_box = P.le_g;
   if (!LE) P.le_g = -1;
   __shared__ float4 tile[SCAN ? kTile + 1 : 1];
-  __shared__ uint32_t buf[(!MIXED && !COLL && !SCAN) ? kForceLdsWordsF64 : kBuf * kWave];
+  __shared__ uint32_t buf[(!MIXED && !COLL && !SCAN) ? kForceLdsWordsF64<FT> : kBuf * kWave];
   if (SCAN && VERLET) {
     const int slots = chunk_slots(P);
     for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
