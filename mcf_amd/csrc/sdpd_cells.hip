@@ -153,7 +153,8 @@ __global__ void k_scatter(int n, const int32_t* __restrict__ key, const int32_t*
 //   back     the state copied back, with x_ref and the walks' positions
 //                                               ITEM particles (Verlet lists)
 // The counts are zero between sorts.
-constexpr int kSortThreads = 256;
+constexpr int kSortThreads = 256;    // of a launch per phase, and particles per item
+constexpr int kChainThreads = 1024;  // of the one launch, likewise
 enum SortPhase { kKeys = 0, kSums, kStarts, kScatter, kPlace, kBack, kSortPhases };
 
 struct SortPlan {
@@ -438,12 +439,14 @@ __device__ __forceinline__ void sort_item(const DevParams& P, const DeviceState&
 }
 
 // One launch per phase: for callers that may overlap on the same buffers
-// (k_sort_chain's counters would not survive that).
-template <int ITEM>
+// (k_sort_chain's counters would not survive that), and for lists rebuilt every
+// step.  ADVANCE: also one marching step.
+template <bool ADVANCE>
 __global__ __launch_bounds__(kSortThreads) void k_sort_phase(DevParams P, DeviceState S,
                                                              SortPlan plan, int phase) {
-  __shared__ int32_t wsum[4];
-  sort_item<kSortThreads, ITEM>(P, S, plan, phase, blockIdx.x, wsum);
+  __shared__ int32_t wsum[kSortThreads / 64];
+  if (ADVANCE && blockIdx.x == 0 && threadIdx.x == 0) advance_step(S.step_dev, S.time_dev, P.dt);
+  sort_item<kSortThreads, kSortThreads>(P, S, plan, phase, blockIdx.x, wsum);
 }
 
 // Whether the lists are rebuilt this step: a particle moved more than skin / 2
@@ -493,32 +496,47 @@ __device__ __forceinline__ void set_gate(const DeviceState& S, bool moved) {
 // unfinished item never waits on one that has not started: the waits end
 // whatever the number of workgroups on the GPU.
 //
+// A workgroup counts its items of a phase in one go, before it waits for the
+// next phase or ends: the count needs its XCD's L2 written back, and with a
+// write-back per item, and workgroups of 256, a rebuild's sort took 893 us at
+// 128^3, 490 at 100^3, 140 at 45^3 and 48 at 30^3 (349, 188, 50 and 37 now).  For
+// the same reason the workgroups are large and few: 128 of 1024 threads, 256
+// beyond 2^20 particles (64^3 80 us with 128, 91 with 256; 128^3 384 and 349).
+//
 // ctl: [0] tickets, [1 + phase] items done, [7] workgroups that left; zero
 // between launches (the last workgroup to leave clears them).
-// mode 0: per-step lists.  1 (Verlet lists): sorts when the lists are
-// outdated.  2 (Verlet lists): sorts in any case.  advance: also one marching
-// step (nothing else here reads the step).
-template <int ITEM>
-__global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, DeviceState S,
+// Verlet lists only.  mode 1: sorts when the lists are outdated, 2: in any case.
+// advance: also one marching step (nothing else here reads the step).
+__global__ __launch_bounds__(kChainThreads) void k_sort_chain(DevParams P, DeviceState S,
                                                              SortPlan plan, int mode,
                                                              int advance) {
-  __shared__ int32_t wsum[4];
+  constexpr int T = kChainThreads;
+  __shared__ int32_t wsum[T / 64];
   __shared__ int32_t drawn;
   bool moved = mode == 2;
   if (advance && blockIdx.x == 0 && threadIdx.x == 0) advance_step(S.step_dev, S.time_dev, P.dt);
   if (mode == 1 && !lists_outdated(P, S, moved)) return;
   int32_t* ctl = S.sort_ctl;
-  int total = 0;
-  for (int p = 0; p < kSortPhases; ++p) total += plan.items[p];
   int ready = -1;  // phases up to this one are known to be done
+  int held = 0, of = 0;  // items of phase `of` done here and not yet counted
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) drawn = atomicAdd(&ctl[0], 1);
     __syncthreads();
-    int item = drawn;
-    if (item >= total) break;
-    int phase = 0;
-    while (item >= plan.items[phase]) item -= plan.items[phase++];
+    int item = drawn, phase = 0;
+    while (phase < kSortPhases && item >= plan.items[phase]) item -= plan.items[phase++];
+    if (held > 0 && phase != of) {
+      // every wave's stores have reached the L2 before thread 0 writes it back
+      // (a workgroup barrier alone does not wait for them)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_fetch_add(&ctl[1 + of], held, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      held = 0;
+    }
+    if (phase == kSortPhases) break;
     if (phase - 1 > ready) {
       // (a phase without items is done; the phases before the last one with
       // items were done when that one began)
@@ -535,21 +553,17 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, Device
       }
       ready = phase - 1;
     }
-    sort_item<kSortThreads, ITEM>(P, S, plan, phase, item, wsum);
-    // every wave's stores have reached the L2 before thread 0 writes it back
-    // (a workgroup barrier alone does not wait for them)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      __hip_atomic_fetch_add(&ctl[1 + phase], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    sort_item<T, T>(P, S, plan, phase, item, wsum);
+    held += 1;
+    of = phase;
   }
   if (threadIdx.x != 0) return;
+  // (this workgroup's counts are in before it is counted out)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (atomicAdd(&ctl[7], 1) != (int)gridDim.x - 1) return;
   // the last workgroup: every other one has read what is written here
   for (int q = 0; q < 8; ++q) ctl[q] = 0;
-  if (mode != 0) set_gate(S, moved);
+  set_gate(S, moved);
 }
 
 // The sort of a small box: every workgroup counts all the cells for itself in
@@ -557,8 +571,9 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_chain(DevParams P, Device
 // particles; the last one to finish copies the state back.  Nothing waits, and
 // ctl[0] alone is shared.  64 x 64 particles: 20 us, 51 with k_sort_chain,
 // 39 with the whole sort in one workgroup (one CU's issue rate).
-// mode: k_sort_chain's, and without the gate 3 as 2, 4 as 0; keys_done: the
-// step boundary has counted the cells in S.count, which are cleared.
+// mode: k_sort_chain's, without the gate 3 as 2, and 0 and 4 for lists rebuilt
+// every step; keys_done: the step boundary has counted the cells in S.count, which
+// are cleared.
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallPer = 4;
 constexpr int kSmallParticles = kSmallThreads * kSmallPer;
@@ -720,17 +735,25 @@ static inline dim3 small_grid(const DevParams& P) {
   return dim3((P.n + kSmallOwn - 1) / kSmallOwn);
 }
 
-// Particles per item: 256 as long as that leaves the tickets few (32^3: 28
-// us for the six phases, 47 with 1024), 1024 beyond.
-constexpr int kSmallItem = 256, kLargeItem = 1024;
-constexpr int kSmallItems = 1 << 17;
-
-// Workgroups of the chain: up to four per CU, no more than its longest phase
-// has items.
-static inline dim3 sort_grid(const SortPlan& plan) {
+// Workgroups of the chain, no more than its longest phase has items.
+static inline dim3 sort_grid(const DevParams& P, const SortPlan& plan) {
   int most = 1;
   for (int p = 0; p < kSortPhases; ++p) most = std::max(most, plan.items[p]);
-  return dim3(std::min(most, 1024));
+  return dim3(std::min(most, P.n > (1 << 20) ? 256 : 128));
+}
+
+// (Lists rebuilt every step always sort: nothing to gain from a launch that may
+// return at once.  us with the chain and with a launch per phase: 30^3 25 and 24,
+// 45^3 31 and 26, 64^3 47 and 35, 100^3 103 and 81, 128^3 180 and 139.)
+static void launch_phases(hipStream_t s, const DevParams& P, const DeviceState& S, bool keys,
+                          bool copy_back, bool advance) {
+  const SortPlan plan = sort_plan(P, kSortThreads, keys, copy_back);
+  for (int p = 0; p < kSortPhases; ++p)
+    if (plan.items[p] > 0) {
+      const auto kernel = advance ? k_sort_phase<true> : k_sort_phase<false>;
+      hipLaunchKernelGGL(kernel, dim3(plan.items[p]), dim3(kSortThreads), 0, s, P, S, plan, p);
+      advance = false;
+    }
 }
 
 void launch_sort(hipStream_t s, const DevParams& P, const DeviceState& S, SortKind kind,
@@ -741,14 +764,12 @@ void launch_sort(hipStream_t s, const DevParams& P, const DeviceState& S, SortKi
   if (sort_small(P)) {
     hipLaunchKernelGGL(k_sort_small, small_grid(P), dim3(kSmallThreads), 0, s, P, S, mode,
                        keys ? 0 : 1, advance ? 1 : 0);
-  } else if (P.n <= kSmallItems) {
-    const SortPlan plan = sort_plan(P, kSmallItem, keys, verlet);
-    hipLaunchKernelGGL(k_sort_chain<kSmallItem>, sort_grid(plan), dim3(kSortThreads), 0, s, P, S,
-                       plan, mode, advance ? 1 : 0);
+  } else if (!verlet) {
+    launch_phases(s, P, S, keys, false, advance);
   } else {
-    const SortPlan plan = sort_plan(P, kLargeItem, keys, verlet);
-    hipLaunchKernelGGL(k_sort_chain<kLargeItem>, sort_grid(plan), dim3(kSortThreads), 0, s, P, S,
-                       plan, mode, advance ? 1 : 0);
+    const SortPlan plan = sort_plan(P, kChainThreads, true, true);
+    hipLaunchKernelGGL(k_sort_chain, sort_grid(P, plan), dim3(kChainThreads), 0, s, P, S, plan, mode,
+                       advance ? 1 : 0);
   }
 }
 
@@ -758,11 +779,7 @@ void launch_sort_phases(hipStream_t s, const DevParams& P, const DeviceState& S,
                        copy_back ? 3 : 4, 0, 0);
     return;
   }
-  const SortPlan plan = sort_plan(P, kSmallItem, true, copy_back);
-  for (int p = 0; p < kSortPhases; ++p)
-    if (plan.items[p] > 0)
-      hipLaunchKernelGGL(k_sort_phase<kSmallItem>, dim3(plan.items[p]), dim3(kSortThreads), 0, s,
-                         P, S, plan, p);
+  launch_phases(s, P, S, true, copy_back, false);
 }
 
 void launch_reference_cells(hipStream_t s, const DevParams& P, const DeviceState& S) {

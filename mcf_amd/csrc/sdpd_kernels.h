@@ -94,9 +94,9 @@ struct DeviceState {
 void launch_fill_i32(hipStream_t s, int32_t* a, int32_t v, int64_t n);
 void launch_fill_f64(hipStream_t s, double* a, double v, int64_t n);
 // The cell sort of the step grid (cell counts and sort_ctl are zero before and
-// after).  Lists rebuilt every step: the sorted state is in the *_alt buffers
-// and the caller swaps the ping-pong pointers (kStepKeysDone: the step
-// boundary has counted the cells already).  Verlet lists: the sorted state is
+// after).  Lists rebuilt every step: a launch per phase (small boxes: one); the
+// sorted state is in the *_alt buffers and the caller swaps the ping-pong pointers
+// (kStepKeysDone: the step boundary has counted the cells already).  Verlet lists: the sorted state is
 // copied back into the primary buffers (and into x_ref), so the buffers never
 // change and a captured graph can hold the sort; kVerletGated runs only if the
 // lists are outdated, and either way sets gate[0] when the next density pass

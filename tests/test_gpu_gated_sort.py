@@ -60,13 +60,15 @@ def test_against_oracle(oracle, shape, n, mixed):
     assert vec_err(f, st.f) < (1e-4 if mixed else 1e-10)
 
 
-# items of 256 particles up to 2^17 of them, of 1024 beyond
-@pytest.mark.parametrize("n", [131071, 131072, 131073, 132651])
-def test_items(n):
-    box = fast_box((51, 51, 51), n)
+# items of 1024 particles on one workgroup each, on fewer than that, beyond 2^20
+# particles
+@pytest.mark.parametrize("side,n", [(51, 131071), (51, 131072), (51, 131073), (51, 132651),
+                                    (102, 1048577)])
+def test_items(side, n):
+    box = fast_box((side, side, side), n)
     print(f"gated sort: n={n}", flush=True)
     (x, v, rho, f), (x0, v0, rho0, f0) = run(box, SKIN), run(box, 0.0)
     assert rel_err(rho, rho0) < 1e-12
-    assert np.abs(x - x0).max() < 1e-10 * 51
+    assert np.abs(x - x0).max() < 1e-10 * side
     assert vec_err(v, v0) < 1e-10
     assert vec_err(f, f0) < 1e-10
