@@ -35,6 +35,7 @@
 #include <type_traits>
 
 #include "sdpd_kernels.h"
+#include "sdpd_window.h"
 
 namespace sdpd {
 
@@ -409,7 +410,7 @@ __device__ __forceinline__ Home load_home(const DevParams& P, const DeviceState&
       // from the build cell unwrapped: the window centre is taken in that
       // frame, so a lane that crossed an x face since stays with its wave
       const double xw = P.verlet ? (double)h.cx * cs + (double)h.a.x : h.x0;
-      const int wc = (int)floor((xw - sp) / cs);
+      const int wc = window_cell(xw, h.cx, cs, sp);
       const float dxf = (float)((double)(h.cx - wc) * cs - sp);
       int mn = h.active ? wc : INT_MAX, mx = h.active ? wc : INT_MIN;
 #pragma unroll

@@ -124,3 +124,27 @@ def test_position(mixed):
     assert np.abs(f1[:-1] - f0[:-1]).max() < 1e-5 * np.abs(f0).max()
     # the lists are rebuilt once, without it
     assert builds == (2 if mixed else 1)
+
+
+@pytest.mark.parametrize("lists", ["verlet", "every step", "mixed"])
+@pytest.mark.parametrize("speed", [np.nan, np.inf, 1e9, 1e300])
+def test_lost_between_sheared_faces(lists, speed):
+    # A particle that leaves the box, or whose position is not a number, has no
+    # window in the sheared frame: its cell's is taken, and the particles beyond
+    # its neighbours' neighbours go on.
+    box = W.tait_box_3d(20, kt=1e-3)
+    prm = box.prm.replace(le_dim=2, le_v_lower=[-0.3, 0, 0], le_v_upper=[0.3, 0, 0])
+    i = int(np.argmin(np.abs(box.x - 10.0).sum(1)))
+    far = distances(box.x, i, prm) > 3.2 * prm.cut_off
+    assert far.sum() > 1000
+    box.v[i] = speed
+    print(f"lost between sheared faces: {lists} speed={speed}", flush=True)
+    with SDPD(prm.replace(precision=1) if lists == "mixed" else prm) as g:
+        if lists == "every step":
+            g.set_skin(0.0)
+        g.upload(box.x, box.v, box.m, box.pid)
+        g.integrate_VV(2)
+        x, v = g.download()
+        rho = g.download_density()[0]
+    assert np.isfinite(x[far]).all() and np.isfinite(v[far]).all()
+    assert (np.abs(rho[far] - 1.0) < 0.2).all()
