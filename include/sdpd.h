@@ -151,7 +151,11 @@ int sdpd_stats(sdpd_ctx *ctx, double *mom /*[3]*/, double *ekin);
 int sdpd_stats_replicas(sdpd_ctx *ctx, double *mom, double *ekin);
 
 /* Copies state back in upload order.  Any pointer may be NULL.
- * x, v, f: (num_dim, n); rho, p: n; ct, vgt: (num_dim*num_dim, n). */
+ * x, v, f: (num_dim, n); rho, p: n; ct, vgt: (num_dim*num_dim, n).
+ * The first download allocates pinned host memory for the transfers, what the
+ * context's largest one takes and at most 8 MiB, kept until sdpd_destroy, and
+ * each copies out with up to eight threads.  SDPD_ERR_STATE if the device's
+ * permutation is corrupt. */
 int sdpd_download(sdpd_ctx *ctx, double *x, double *v, double *rho,
                   double *p, double *f);
 int sdpd_download_tensors(sdpd_ctx *ctx, double *ct, double *vgt);

@@ -1373,8 +1373,8 @@ int sdpd_set_lees_edwards(sdpd_ctx* c, int32_t le_dim, const double* v_lower,
     return fail(c, SDPD_ERR_ARG, "sdpd_set_lees_edwards: le_dim must be 2 (y) or 3 (z)");
   if (c->P.nrep != 1 || !c->rep_lo.empty())
     return fail(c, SDPD_ERR_STATE, "sdpd_set_lees_edwards: one box only (batched context)");
-  // the colloid force pass sizes its band of sheared rows at upload, and
-  // Verlet lists (chosen at upload) serve boxes without sheared faces only
+  // the colloid force pass sizes its band of sheared rows at upload, and mixed
+  // precision's Verlet lists (chosen at upload) serve no sheared faces
   if ((c->P.ncoll > 0 || c->P.verlet) && c->n > 0)
     return fail(c, SDPD_ERR_STATE,
                 "sdpd_set_lees_edwards: with colloids or Verlet lists, set the faces before "

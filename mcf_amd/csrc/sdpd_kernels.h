@@ -82,8 +82,8 @@ struct DeviceState {
   // the rescan passes have work; gate[3]: workgroups of k_stats done, 0 between
   // launches; gate[4] = 1: the step's force walk came to sums that are not
   // finite, so the rescan of the forces has work; gate[5] = 1: a download met a
-  // corrupt permutation), the bits of the largest squared displacement since the build
-  // seen this step, and the in-cut-off neighbours of each particle in the
+  // corrupt permutation), the bits of the largest squared displacement since the build,
+  // and the in-cut-off neighbours of each particle in the
   // last density pass (every mode)
   double* x_ref;
   int32_t* gate;
